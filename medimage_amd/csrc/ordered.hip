@@ -3,9 +3,9 @@
 // reference program adds it, so results equal the reference's bit for bit:
 //   * A: one lane per ray sums its products in the order proj.c emits them;
 //   * AStar: one lane per pixel, likewise;
-//   * energies, norms, inner products: one wave per sum, terms computed by
-//     the 64 lanes in parallel and folded into one running double in
-//     row-major order (v_readlane, no reassociation).
+//   * energies, norms, inner products: one workgroup per sum, whose result
+//     is the running double's after adding the terms one by one in
+//     row-major order (k_chains).
 #include "ordered.hpp"
 #include "gc_stencil.hpp"
 
@@ -112,15 +112,9 @@ struct ChainArgs {
     int nchains;
     int nx, ny;
     double alpha, beta, eps;
-    int edge_c;            // epilogue: chains are nNablaD, nD, sum n d^2 ->
-    Scalars *sc;           //   sc->e_c (main.c:329); skipped once edge_done
+    int edge_c;            // chains are nNablaD, nD, sum n d^2 of the edge step; then
+    Scalars *sc;           //   sc->e_c (main.c:329); all skipped once edge_done
 };
-
-__device__ __forceinline__ double lane_value(double x, int k) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(x), k);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(x), k);
-    return __hiloint2double(hi, lo);
-}
 
 template <int TERM>
 __device__ __forceinline__ void chain_term(const ChainSeg &s, const ChainArgs &a, int64_t e, double &t0, double &t1) {
@@ -134,16 +128,18 @@ __device__ __forceinline__ void chain_term(const ChainSeg &s, const ChainArgs &a
     } else if constexpr (TERM == CT_DOT) {
         t0 = A[e] * B[e];
     } else if constexpr (TERM == CT_REG_INT) {
-        const int64_t q = (1 + e / (ny - 2)) * (int64_t)ny + 1 + e % (ny - 2);
+        // pixel counts fit 32 bits (a 64-bit division is some 100 instructions)
+        const unsigned w2 = (unsigned)(ny - 2), i = (unsigned)e / w2;
+        const int64_t q = (int64_t)(1 + i) * ny + 1 + ((unsigned)e - i * w2);
         const double z = A[q], zu = A[q - ny], zl = A[q - 1], w = B[q];
         t0 = a.alpha * (w * w + 0.01 * (a.eps * a.eps)) * ((z - zu) * (z - zu) + (z - zl) * (z - zl));
     } else if constexpr (TERM == CT_NV) {
-        const int i = (int)(e / ny), j = (int)(e % ny);
+        const int i = (int)((unsigned)e / (unsigned)ny), j = (int)e - i * ny;
         const double z = A[e], zu = gc_ld(A, i - 1, j, nx, ny, 0.0), zl = gc_ld(A, i, j - 1, nx, ny, 0.0);
         const double w = B[e];
         t0 = (w * w + 0.01 * (a.eps * a.eps)) * ((z - zu) * (z - zu) + (z - zl) * (z - zl));
     } else if constexpr (TERM == CT_NABLA2) {
-        const int i = (int)(e / ny), j = (int)(e % ny);
+        const int i = (int)((unsigned)e / (unsigned)ny), j = (int)e - i * ny;
         const double x = 0.5 * (gc_ld(A, i + 1, j, nx, ny, 0.0) - gc_ld(A, i - 1, j, nx, ny, 0.0));
         const double y = 0.5 * (gc_ld(A, i, j + 1, nx, ny, 0.0) - gc_ld(A, i, j - 1, nx, ny, 0.0));
         t0 = x * x;
@@ -153,77 +149,189 @@ __device__ __forceinline__ void chain_term(const ChainSeg &s, const ChainArgs &a
     }
 }
 
-// Folds the segment's terms into acc in index order.  The next 64 terms
-// are loaded before the current ones are folded.
-template <int TERM>
-__device__ double chain_segment(const ChainSeg &s, const ChainArgs &a, double acc) {
-    constexpr bool two = TERM == CT_NABLA2;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t n = s.n;
-    double c0 = 0.0, c1 = 0.0;
-    if (lane < n) chain_term<TERM>(s, a, lane, c0, c1);
-    for (int64_t b0 = 0; b0 < n; b0 += kWave) {
-        double n0 = 0.0, n1 = 0.0;
-        if (b0 + kWave + lane < n) chain_term<TERM>(s, a, b0 + kWave + lane, n0, n1);
-        if (n - b0 >= kWave) {
+// One sequential sum per workgroup, 4096 terms a step.
+//
+// The terms are computed by all lanes, and folding them in index order
+// (rounding after every add, as the reference's loop does) need not be a
+// serial chain.  While the running sum acc stays inside one binade, adding a
+// term t moves it by t rounded to acc's own unit in the last place, whatever
+// acc's bits are, unless t lies exactly halfway between two multiples of it
+// (then ties-to-even looks at acc).  So per 256 terms (one wave) the rounded
+// terms are integers that may be added in any order, and the 16 waves' sums
+// are applied in order as long as (a) no term is a tie, infinite, NaN or
+// 2^50 units or more, and (b) acc plus the wave's positive terms stays below
+// the binade's upper end and acc plus its negative ones (each up to half a
+// unit more than its rounded value) above the lower end.
+// A wave that fails this is folded term by term from LDS, after which the
+// waves behind it are rounded again for acc's new binade.  acc's binade
+// changes about log2(n) times, so a sum of 4e5 terms folds some 20 waves of
+// 1600 serially.
+//
+// Measured over the sums of one GoldenC alternation (2.6e5 to 5.2e5 terms):
+// 696 us a launch, against 5189 us (13 ns a term) with one wave per sum that
+// took each term from its lane and added it.
+constexpr int kChainThreads = 1024, kChainPer = 4, kChainStep = kChainThreads * kChainPer;
+constexpr int kChainWaves = kChainThreads / kWave, kChainSub = kWave * kChainPer;
+
+struct ChainLds {
+    double term[kChainStep];
+    long long sum[kChainWaves], pos[kChainWaves], low[kChainWaves];   // low: bound of the negative terms, 0 without any
+    int bad[kChainWaves], zero[kChainWaves];
+    double acc;
+};
+
+__device__ __forceinline__ long long wave_sum_i64(long long x) {
 #pragma unroll
-            for (int k = 0; k < kWave; ++k) {
-                acc = acc + lane_value(c0, k);
-                if (two) acc = acc + lane_value(c1, k);
-            }
-        } else {
-            const int m = (int)(n - b0);
-            for (int k = 0; k < m; ++k) {
-                acc = acc + lane_value(c0, k);
-                if (two) acc = acc + lane_value(c1, k);
-            }
+    for (int o = kWave / 2; o > 0; o >>= 1) x += __shfl_xor(x, o, kWave);
+    return x;
+}
+
+// The terms of lane slots first .. first + 3 of the segment (zeros past its
+// end; adding +0 leaves every running sum but -0 as it is, and the sums start
+// at +0).
+template <int TERM>
+__device__ __forceinline__ void chain_load(const ChainSeg &s, const ChainArgs &a, int64_t first, double (&t)[kChainPer]) {
+    if constexpr (TERM == CT_NABLA2) {
+#pragma unroll
+        for (int k = 0; k < kChainPer; k += 2) {
+            const int64_t e = (first + k) >> 1;
+            t[k] = t[k + 1] = 0.0;
+            if (e < s.n) chain_term<TERM>(s, a, e, t[k], t[k + 1]);
         }
-        c0 = n0;
-        c1 = n1;
+    } else {
+#pragma unroll
+        for (int k = 0; k < kChainPer; ++k) {
+            double none = 0.0;
+            t[k] = 0.0;
+            if (first + k < s.n) chain_term<TERM>(s, a, first + k, t[k], none);
+        }
+    }
+}
+
+template <int TERM>
+__device__ double chain_segment(const ChainSeg &s, const ChainArgs &a, double acc, ChainLds &L) {
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+    const int64_t n = TERM == CT_NABLA2 ? 2 * s.n : s.n;
+    double t[kChainPer], nx[kChainPer];
+    chain_load<TERM>(s, a, (int64_t)tid * kChainPer, t);
+    for (int64_t b0 = 0; b0 < n; b0 += kChainStep) {
+        // the next step's terms load while this one is folded
+        chain_load<TERM>(s, a, b0 + kChainStep + (int64_t)tid * kChainPer, nx);
+#pragma unroll
+        for (int k = 0; k < kChainPer; ++k) L.term[tid * kChainPer + k] = t[k];
+        const int waves = (int)min((int64_t)kChainWaves, (n - b0 + kChainSub - 1) / kChainSub);
+        for (int from = 0; from < waves;) {
+            // acc = +-A 2^(e - 52), 2^52 <= A < 2^53, where e is its exponent
+            const long long bits = __double_as_longlong(acc);
+            const int be = (int)((bits >> 52) & 0x7ff);
+            const bool normal = be >= 53 && be <= 2000;   // the scale 2^(52 - e) is a normal number too
+            const double scale = __longlong_as_double(((long long)(2098 - be) << 52) | (bits & ((long long)1 << 63)));
+            if (wv >= from && wv < waves) {
+                long long p = 0, q = 0;
+                bool bad = false, zero = true, below = false;
+                constexpr double M = 6755399441055744.0;   // 1.5 2^52: adding it rounds to an integer
+#pragma unroll
+                for (int k = 0; k < kChainPer; ++k) {
+                    const double x = t[k] * scale, r = x + M;
+                    const long long i = __double_as_longlong(r) - __double_as_longlong(M);
+                    bad |= !(fabs(x) < 1125899906842624.0) | (fabs(x - (r - M)) == 0.5);
+                    zero &= t[k] == 0.0;
+                    below |= x < 0.0;
+                    p += i > 0 ? i : 0;
+                    q += i < 0 ? i : 0;
+                }
+                bad |= !normal;
+                bad = __any(bad);
+                zero = __all(zero);
+                below = __any(below);
+                if (!bad) {
+                    p = wave_sum_i64(p);
+                    if (below) q = wave_sum_i64(q);
+                }
+                if (lane == 0) {
+                    L.sum[wv] = p + q;
+                    L.pos[wv] = p;
+                    L.low[wv] = below ? q - kChainSub : 0;
+                    L.bad[wv] = bad;
+                    L.zero[wv] = zero;
+                }
+            }
+            __syncthreads();
+            // every thread applies the waves' sums in order
+            constexpr long long kLo = (long long)1 << 52;
+            long long A = (bits & (kLo - 1)) | kLo;
+            int k = from;
+            for (; k < waves; ++k) {
+                if (L.zero[k]) continue;   // +-0 terms leave acc as it is
+                if (L.bad[k] || A + L.pos[k] >= 2 * kLo || (L.low[k] < 0 && A + L.low[k] <= kLo)) break;
+                A += L.sum[k];
+            }
+            if (normal) acc = __longlong_as_double((bits & ~(kLo - 1)) | (A & (kLo - 1)));
+            if (k < waves) {
+                // wave k term by term, by one wave (all lanes alike)
+                if (wv == 0) {
+                    const int m = (int)min((int64_t)kChainSub, n - b0 - (int64_t)k * kChainSub);
+                    const double *q = L.term + k * kChainSub;
+                    int i = 0;
+                    for (; i + 16 <= m; i += 16) {
+                        double x[16];
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) x[j] = q[i + j];
+#pragma unroll
+                        for (int j = 0; j < 16; ++j) acc = acc + x[j];
+                    }
+                    for (; i < m; ++i) acc = acc + q[i];
+                    if (lane == 0) L.acc = acc;
+                }
+                ++k;
+                __syncthreads();
+                acc = L.acc;
+            }
+            from = k;
+            __syncthreads();   // the tables (and, at the end, the terms) are written again
+        }
+#pragma unroll
+        for (int k = 0; k < kChainPer; ++k) t[k] = nx[k];
     }
     return acc;
 }
 
-__global__ void k_chains(ChainArgs a) {
-    __shared__ double res[4];
+// One workgroup per sum.
+__global__ __launch_bounds__(kChainThreads) void k_chains(ChainArgs a) {
+    __shared__ ChainLds L;
     if (a.edge_c && (a.sc->edge_done || a.sc->converged)) return;
-    const int w = threadIdx.x / kWave;
-    if (w < a.nchains) {
-        const ChainDesc &c = a.c[w];
-        double acc = 0.0;
-        for (int k = 0; k < c.nseg; ++k) {
-            const ChainSeg &s = c.seg[k];
-            switch (s.term) {
-                case CT_SQDIFF: acc = chain_segment<CT_SQDIFF>(s, a, acc); break;
-                case CT_SQ: acc = chain_segment<CT_SQ>(s, a, acc); break;
-                case CT_DOT: acc = chain_segment<CT_DOT>(s, a, acc); break;
-                case CT_REG_INT: acc = chain_segment<CT_REG_INT>(s, a, acc); break;
-                case CT_NV: acc = chain_segment<CT_NV>(s, a, acc); break;
-                case CT_NABLA2: acc = chain_segment<CT_NABLA2>(s, a, acc); break;
-                default: acc = chain_segment<CT_NDSQ>(s, a, acc); break;
-            }
-        }
-        if ((threadIdx.x & (kWave - 1)) == 0) {
-            res[w] = acc;
-            if (c.out) *c.out = acc;
+    const ChainDesc &c = a.c[blockIdx.x];
+    double acc = 0.0;
+    for (int k = 0; k < c.nseg; ++k) {
+        const ChainSeg &s = c.seg[k];
+        switch (s.term) {
+            case CT_SQDIFF: acc = chain_segment<CT_SQDIFF>(s, a, acc, L); break;
+            case CT_SQ: acc = chain_segment<CT_SQ>(s, a, acc, L); break;
+            case CT_DOT: acc = chain_segment<CT_DOT>(s, a, acc, L); break;
+            case CT_REG_INT: acc = chain_segment<CT_REG_INT>(s, a, acc, L); break;
+            case CT_NV: acc = chain_segment<CT_NV>(s, a, acc, L); break;
+            case CT_NABLA2: acc = chain_segment<CT_NABLA2>(s, a, acc, L); break;
+            default: acc = chain_segment<CT_NDSQ>(s, a, acc, L); break;
         }
     }
-    if (!a.edge_c) return;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        Scalars *sc = a.sc;
-        const double nnd = res[0], nd = res[1], tmp = res[2];
-        sc->e_nnd = nnd;
-        sc->e_nd = nd;
-        sc->e_nd2 = tmp;
-        sc->e_c = nd / (a.alpha * tmp + a.beta * a.eps * nnd + (a.beta / (4 * a.eps)) * nd);
-    }
+    if (threadIdx.x == 0) *c.out = acc;
+}
+
+// The edge step from its three sums (main.c:329).
+__global__ void k_chain_edge(ChainArgs a) {
+    Scalars *sc = a.sc;
+    if (sc->edge_done || sc->converged) return;
+    sc->e_c = sc->e_nd / (a.alpha * sc->e_nd2 + a.beta * a.eps * sc->e_nnd + (a.beta / (4 * a.eps)) * sc->e_nd);
 }
 
 void launch_chains(hipStream_t st, const ChainArgs &a) {
     MI_REQUIRE(a.nchains >= 1 && a.nchains <= 4, MI_E_ARG, "1 to 4 sums per launch");
-    k_chains<<<1, kWave * a.nchains, 0, st>>>(a);
+    k_chains<<<a.nchains, kChainThreads, 0, st>>>(a);
     MI_HIP(hipGetLastError());
+    if (a.edge_c) {
+        k_chain_edge<<<1, 1, 0, st>>>(a);
+        MI_HIP(hipGetLastError());
+    }
 }
 
 ChainSeg seg(int term, int64_t n, const double *a, const double *b = nullptr) { return ChainSeg{term, n, a, b}; }
@@ -467,9 +575,9 @@ void gc_edge_step_ordered(mi_context *ctx, JobState<double> &js, double alpha, d
     ca.edge_c = 1;
     ca.sc = js.sc.p;
     ca.nchains = 3;
-    ca.c[0] = chain(nullptr, seg(CT_NABLA2, npix, js.d.p));
-    ca.c[1] = chain(nullptr, seg(CT_SQ, npix, js.d.p));
-    ca.c[2] = chain(nullptr, seg(CT_NDSQ, npix, js.w.p, js.d.p));
+    ca.c[0] = chain(&ca.sc->e_nnd, seg(CT_NABLA2, npix, js.d.p));
+    ca.c[1] = chain(&ca.sc->e_nd, seg(CT_SQ, npix, js.d.p));
+    ca.c[2] = chain(&ca.sc->e_nd2, seg(CT_NDSQ, npix, js.w.p, js.d.p));
     launch_pass_begin(st, js.sc.p);
     for (int k = 0; k < iter_edge; ++k) {
         launch_edge_grad_n<double>(st, nx, ny, js.u.p, js.v.p, js.d.p, js.w.p, alpha, beta, eps, js.sc.p);

@@ -6,8 +6,8 @@
 // and norm in row-major loop order.  Its CG with median filters and a revert
 // test amplifies rounding differences by about 20x per alternation, so the
 // drop-in keeps those orders exactly: one lane per ray (or pixel) sums its
-// products in the reference's order, and each reduction is one wave's
-// sequential chain.  The results are then the reference's bit for bit.
+// products in the reference's order, and each reduction equals the running
+// sum of its terms in order.  The results are then the reference's bit for bit.
 #pragma once
 
 #include "solver.hpp"
