@@ -16,9 +16,17 @@ int pow2ceil(int n) {
     return k;
 }
 
+// FP32 units of a geometry with lines project along them.
+template <typename T>
+bool use_lines(const Matrix &m) {
+    return sizeof(T) == 4 && m.has_lines;
+}
+
 template <typename T>
 int64_t unit_state_bytes(const Matrix &m, int K) {
-    return (int64_t)K * (2 * m.nrows + 4 * m.npix_t) * (int64_t)sizeof(T);
+    int64_t e = 2 * m.nrows + 4 * m.npix_t;
+    if (use_lines<T>(m)) e += line_elems(m.g.nx, m.g.ny) + line_elems(m.g.ny, m.g.nx);
+    return (int64_t)K * e * (int64_t)sizeof(T);
 }
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -29,7 +37,14 @@ int64_t max_slices(const Sell &q) {
     for (size_t s = 0; s + 1 < q.slice0.size(); ++s) r = std::max(r, q.slice0[s + 1] - q.slice0[s]);
     return r;
 }
+int64_t line_blocks(const Matrix &m) {
+    int64_t r = 0;
+    for (int s = 0; s < m.S; ++s) r = std::max(r, m.lines.slice0[s + 1] - m.lines.slice0[s]);
+    return r / 4;
+}
+template <typename T>
 int64_t fp_blocks(const Matrix &m) {
+    if (use_lines<T>(m)) return line_blocks(m);
     if (m.has_otf) {
         int64_t r = 0;
         for (int s = 0; s < m.S; ++s) r = std::max(r, m.otf.slice0[s + 1] - m.otf.slice0[s]);
@@ -41,8 +56,9 @@ int64_t bp_blocks(const Matrix &m) { return cdiv(max_slices(m.bs), kBlock / kWav
 int64_t px_blocks(const Matrix &m) { return cdiv(m.npix_t, kPixBlock); }
 
 // Partials per job per slot of a unit over `m`.
+template <typename T>
 int64_t part_cap(const Matrix &m) {
-    return std::max({fp_blocks(m), bp_blocks(m), px_blocks(m), (int64_t)1});
+    return std::max({fp_blocks<T>(m), bp_blocks(m), px_blocks(m), (int64_t)1});
 }
 
 int64_t free_device_bytes() {
@@ -52,6 +68,26 @@ int64_t free_device_bytes() {
 }
 
 }  // namespace
+
+template <typename T>
+void Unit<T>::alloc(hipStream_t st) {
+    g.n = r.n = (size_t)m->nrows * K;
+    for (Part *b : {&u, &v, &d, &w}) b->n = (size_t)m->npix_t * K;
+    if (use_lines<T>(*m)) {
+        px.n = (size_t)line_elems(m->g.nx, m->g.ny) * K;
+        py.n = (size_t)line_elems(m->g.ny, m->g.nx) * K;
+    }
+    constexpr size_t kAlign = 256 / sizeof(T);   // each part starts on a 256-byte line, as an allocation of its own does
+    size_t at = 0;
+    for (Part *b : {&g, &r, &u, &v, &d, &w, &px, &py}) at += (b->n + kAlign - 1) / kAlign * kAlign;
+    state.alloc(at);
+    at = 0;
+    for (Part *b : {&g, &r, &u, &v, &d, &w, &px, &py}) {
+        if (b->n) b->p = state.p + at;
+        at += (b->n + kAlign - 1) / kAlign * kAlign;
+    }
+    MI_HIP(hipMemsetAsync(state.p, 0, state.bytes(), st));
+}
 
 template <typename T>
 Batch<T>::Batch(mi_context *c, int n_subsets) : ctx(c), S(n_subsets) {
@@ -180,13 +216,7 @@ Unit<T> *Batch<T>::place(BatchJob<T> &j, int group) {
     U->K = K;
     for (auto &x : U->jobs) x = -1;
     const hipStream_t st = ctx->stream;
-    U->g.alloc((size_t)m.nrows * K);
-    U->r.alloc((size_t)m.nrows * K);
-    U->u.alloc((size_t)m.npix_t * K);
-    U->v.alloc((size_t)m.npix_t * K);
-    U->d.alloc((size_t)m.npix_t * K);
-    U->w.alloc((size_t)m.npix_t * K);
-    for (auto *b : {&U->g, &U->r, &U->u, &U->v, &U->d, &U->w}) MI_HIP(hipMemsetAsync(b->p, 0, b->bytes(), st));
+    U->alloc(st);
     U->jobs[0] = j.id;
     j.uid = uid;
     j.slot = 0;
@@ -214,6 +244,7 @@ void Batch<T>::load_job(BatchJob<T> &j) {
     } else {
         eng_put_img<T>(st, U.u.p, U.K, j.slot, nx, ny, m.tny, nullptr, T(0));
     }
+    if (U.px.p) eng_spread<T>(st, U.u.p, U.px.p, U.py.p, U.K, nx, ny, m.tny);
     if (!j.v0.empty()) {
         MI_HIP(hipMemcpyAsync(stage.p, j.v0.data(), m.npix * sizeof(T), hipMemcpyHostToDevice, st));
         eng_put_img<T>(st, U.v.p, U.K, j.slot, nx, ny, m.tny, stage.p, T(1));
@@ -363,13 +394,7 @@ void Batch<T>::compact() {
             U->uid = uid;
             U->K = K;
             for (auto &x : U->jobs) x = -1;
-            U->g.alloc((size_t)mp->nrows * K);
-            U->r.alloc((size_t)mp->nrows * K);
-            U->u.alloc((size_t)mp->npix_t * K);
-            U->v.alloc((size_t)mp->npix_t * K);
-            U->d.alloc((size_t)mp->npix_t * K);
-            U->w.alloc((size_t)mp->npix_t * K);
-            for (auto *b : {&U->g, &U->r, &U->u, &U->v, &U->d, &U->w}) MI_HIP(hipMemsetAsync(b->p, 0, b->bytes(), st));
+            U->alloc(st);
             for (int k = 0; k < K && next < ids.size(); ++k, ++next) {
                 BatchJob<T> &j = job(ids[next]);
                 Unit<T> *src = nullptr;
@@ -385,6 +410,7 @@ void Batch<T>::compact() {
                 j.uid = uid;
                 j.slot = k;
             }
+            if (U->px.p) eng_spread<T>(st, U->u.p, U->px.p, U->py.p, K, mp->g.nx, mp->g.ny, mp->tny);
             units[uid] = std::move(U);
             live.push_back(uid);
         }
@@ -422,7 +448,7 @@ void Batch<T>::rebuild() {
     any_median = false;
     pix.nunits = (int)live.size();
     pix.start[0] = 0;
-    for (Launch *L : {&rows[0], &rows[1], &bpl[0][0], &bpl[0][1], &bpl[1][0], &bpl[1][1], &bpg[0], &bpg[1]}) {
+    for (Launch *L : {&rows[0], &rows[1], &ln[0], &ln[1], &bpl[0][0], &bpl[0][1], &bpl[1][0], &bpl[1][1], &bpg[0], &bpg[1]}) {
         *L = Launch{};
         L->map.nunits = (int)live.size();
         L->map.start[0] = 0;
@@ -433,6 +459,18 @@ void Batch<T>::rebuild() {
         const Matrix &m = *U.m;
         UnitDesc<T> &D = desc[i];
         std::memset(&D, 0, sizeof(D));
+        const bool lines = use_lines<T>(m);
+        if (lines) {
+            D.ln_slice0 = m.lines.d_slice0.p;
+            D.ln_mb = m.lines.mb.p;
+            D.ln_len = m.lines.len.p;
+            D.ln_inv = m.lines.inv.p;
+            D.ln_dlen = m.lines.dlen.p;
+            D.ln_drop = m.lines.drop.p;
+            D.ln_rng = m.lines.rng.p;
+            D.px = U.px.p;
+            D.py = U.py.p;
+        }
         D.fs_slice0 = m.has_otf ? m.otf.d_slice0.p : m.fs.d_slice0.p;
         if (m.has_otf) {
             D.ot_lam = m.otf.lam.p;
@@ -470,7 +508,8 @@ void Batch<T>::rebuild() {
         Launch &B = in_lds ? bpl[bc][lc] : bpg[bc];
         B.kmax = std::max(B.kmax, U.K);
         if (in_lds) B.lds = std::max(B.lds, need);
-        rows[rc].kmax = std::max(rows[rc].kmax, U.K);
+        Launch &F = lines ? ln[rc] : rows[rc];
+        F.kmax = std::max(F.kmax, U.K);
         D.sub_row0 = m.d_sub_row0.p;
         D.g = U.g.p;
         D.r = U.r.p;
@@ -480,7 +519,7 @@ void Batch<T>::rebuild() {
         D.w = U.w.p;
         D.npix_t = m.npix_t;
         D.nrows = m.nrows;
-        D.cap = part_cap(m);
+        D.cap = part_cap<T>(m);
         D.part_off = off;
         off += (int64_t)SL_COUNT * U.K * D.cap;
         D.nx = m.g.nx;
@@ -492,7 +531,9 @@ void Batch<T>::rebuild() {
         D.job0 = U.uid * kMaxK;
         MI_REQUIRE(m.has_sell && (!f64 || m.has64), MI_E_STATE, "matrix lacks the engine's sliced layout");
         for (int c = 0; c < 2; ++c) {
-            rows[c].map.start[i + 1] = rows[c].map.start[i] + (c == rc ? (int)fp_blocks(m) : 0);
+            const int fb = c == rc ? (int)fp_blocks<T>(m) : 0;
+            rows[c].map.start[i + 1] = rows[c].map.start[i] + (lines ? 0 : fb);
+            ln[c].map.start[i + 1] = ln[c].map.start[i] + (lines ? fb : 0);
             for (int l = 0; l < 2; ++l)
                 bpl[c][l].map.start[i + 1] =
                     bpl[c][l].map.start[i] + (in_lds && c == bc && l == lc ? (int)bp_blocks(m) : 0);
@@ -500,7 +541,7 @@ void Batch<T>::rebuild() {
         }
         pix.start[i + 1] = pix.start[i] + (int)px_blocks(m);
         kmax = std::max(kmax, U.K);
-        all_walk = all_walk && m.has_otf;
+        all_walk = all_walk && (lines || m.has_otf);
         for (int k = 0; k < U.K; ++k) {
             if (U.jobs[k] < 0) continue;
             const JobParams &P = h_jp[D.job0 + k];
@@ -551,6 +592,12 @@ void Batch<T>::record_pass(bool timed) {
             if (has1) launch1(st);
         }
     };
+    // the units with lines (FP32) of class c
+    auto line_fp = [&](hipStream_t q, int c, int s, bool resid) {
+        if constexpr (sizeof(T) == 4) {
+            if (ln[c].any()) eng_line_fp(q, args, ln[c].map, s, ln[c].kmax, resid);
+        }
+    };
     eng_finalize<T>(st, args, EF_BEGIN, 0);
     for (int s = 0; s < S; ++s) {
         auto nnz_s = [&](const Unit<T> &U) { return (double)U.m->sub_nnz[s]; };
@@ -560,9 +607,12 @@ void Batch<T>::record_pass(bool timed) {
                 return nnz_s(U) * (4 + sz) + U.m->npix * sz * U.K + 2 * nr_s(U) * sz * U.K;
             }), true);
             auto one = [&](int c) {
-                return [&, c](hipStream_t q) { eng_fp_resid<T>(q, args, rows[c].map, s, rows[c].kmax, all_walk); };
+                return [&, c](hipStream_t q) {
+                    if (rows[c].any()) eng_fp_resid<T>(q, args, rows[c].map, s, rows[c].kmax, all_walk);
+                    line_fp(q, c, s, true);
+                };
             };
-            branches(one(0), one(1), rows[0].any(), rows[1].any());
+            branches(one(0), one(1), rows[0].any() || ln[0].any(), rows[1].any() || ln[1].any());
         }
         {
             LaunchTimer lt(ctx, MI_K_BP, sum([&](const Unit<T> &U) {
@@ -583,9 +633,12 @@ void Batch<T>::record_pass(bool timed) {
                 return nnz_s(U) * (4 + sz) + U.m->npix * sz * U.K;
             }), true);
             auto one = [&](int c) {
-                return [&, c](hipStream_t q) { eng_fp_sq<T>(q, args, rows[c].map, s, rows[c].kmax, all_walk); };
+                return [&, c](hipStream_t q) {
+                    if (rows[c].any()) eng_fp_sq<T>(q, args, rows[c].map, s, rows[c].kmax, all_walk);
+                    line_fp(q, c, s, false);
+                };
             };
-            branches(one(0), one(1), rows[0].any(), rows[1].any());
+            branches(one(0), one(1), rows[0].any() || ln[0].any(), rows[1].any() || ln[1].any());
         }
         {
             LaunchTimer lt(ctx, MI_K_STEP, sum([&](const Unit<T> &U) { return 5.0 * U.m->npix * sz * U.K; }));

@@ -31,7 +31,16 @@ struct Unit {
     int uid = -1;                  // stable: job slots uid * kMaxK + j
     int K = 1;
     int64_t jobs[kMaxK];           // job id per slot, -1 when free
-    DevBuf<T> g, r, u, v, d, w;
+    // The state of K jobs over m: parts of one zeroed allocation (a call of
+    // its own for each part is most of a small unit's admission).
+    struct Part {
+        T *p = nullptr;
+        size_t n = 0;
+    };
+    DevBuf<T> state;
+    Part g, r, u, v, d, w;
+    Part px, py;                   // projection images (units with lines)
+    void alloc(hipStream_t st);
     int used() const {
         int n = 0;
         for (int j = 0; j < K; ++j) n += jobs[j] >= 0;
@@ -120,7 +129,8 @@ struct Batch {
         size_t lds = 0;
         bool any() const { return map.start[map.nunits] > 0; }
     };
-    Launch rows[2], bpl[2][2], bpg[2];   // bpl[K class][LDS class]
+    // Units with lines have their forward rows in ln instead of rows.
+    Launch rows[2], ln[2], bpl[2][2], bpg[2];   // bpl[K class][LDS class]
     hipStream_t side = nullptr;   // the second class of a phase
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     EngArgs<T> args{};

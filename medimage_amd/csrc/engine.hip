@@ -53,8 +53,12 @@ struct UG {
     const GL int64_t *bs_vtab0;
     const GL double *ot_lam, *ot_ax, *ot_ay, *ot_stx, *ot_sty;
     const GL int32_t *ot_cx, *ot_cy, *ot_sg, *ot_cnt;
+    const GL int64_t *ln_slice0;
+    const GL double *ln_mb, *ln_len;
+    const GL float *ln_inv, *ln_dlen;
+    const GL int32_t *ln_drop, *ln_rng;
     const GL int64_t *sub_row0;
-    GL T *g, *r, *u, *v, *d, *w;
+    GL T *g, *r, *u, *v, *d, *w, *px, *py;
     int64_t npix_t, nrows, part_off, cap;
     int nx, ny, tny, K, fs_P, bs_P, job0, nbins;
     __device__ __forceinline__ explicit UG(const UnitDesc<T> &D)
@@ -71,8 +75,11 @@ struct UG {
           ot_stx((const GL double *)D.ot_stx), ot_sty((const GL double *)D.ot_sty),
           ot_cx((const GL int32_t *)D.ot_cx), ot_cy((const GL int32_t *)D.ot_cy),
           ot_sg((const GL int32_t *)D.ot_sg), ot_cnt((const GL int32_t *)D.ot_cnt),
+          ln_slice0((const GL int64_t *)D.ln_slice0), ln_mb((const GL double *)D.ln_mb),
+          ln_len((const GL double *)D.ln_len), ln_inv((const GL float *)D.ln_inv), ln_dlen((const GL float *)D.ln_dlen),
+          ln_drop((const GL int32_t *)D.ln_drop), ln_rng((const GL int32_t *)D.ln_rng),
           sub_row0((const GL int64_t *)D.sub_row0), g((GL T *)D.g), r((GL T *)D.r), u((GL T *)D.u),
-          v((GL T *)D.v), d((GL T *)D.d), w((GL T *)D.w), npix_t(D.npix_t), nrows(D.nrows),
+          v((GL T *)D.v), d((GL T *)D.d), w((GL T *)D.w), px((GL T *)D.px), py((GL T *)D.py), npix_t(D.npix_t), nrows(D.nrows),
           part_off(D.part_off), cap(D.cap), nx(D.nx), ny(D.ny), tny(D.tny), K(D.K), fs_P(D.fs_P), bs_P(D.bs_P),
           job0(D.job0), nbins(D.nbins) {}
     // Tiled index of pixel (i, j), or -1 outside the image.
@@ -180,6 +187,14 @@ __device__ __forceinline__ void storek(GL T *__restrict__ p, const T (&o)[K]) {
     } else {
         p[0] = o[0];
     }
+}
+
+// Pixel (i, j) of the unit's projection images, where it has them.
+template <typename T, int K>
+__device__ __forceinline__ void put_proj(const UG<T> &U, int i, int j, const T (&o)[K]) {
+    if (!U.px) return;
+    storek<T, K>(U.px + ((int64_t)i * line_stride(U.ny) + j + kLinePad) * K, o);
+    storek<T, K>(U.py + ((int64_t)j * line_stride(U.nx) + i + kLinePad) * K, o);
 }
 
 template <typename T, int K>
@@ -595,6 +610,159 @@ __device__ __forceinline__ void fp_unit(const EngArgs<T> &a, const UG<T> &U, int
     block_store<T, K, false>(a, U, RESID ? SL_DF : SL_AD, lb, m, lds);
 }
 
+// Forward projection along the lines (Lines, runtime.hpp), FP32.
+//
+// One workgroup is one group of kLineRays neighbouring rays; its kLineWaves
+// waves cut the lines the group crosses into as many runs, one lane per ray.
+// At line a of the dominant axis a ray covers at most two neighbouring pixels
+// of that line, so a step is one 2K-value load from the projection image that
+// holds the line contiguously and the interpolation
+//   w u[j] + (1 - w) u[j - 1],   w = min(1, frac(hi) / |m|),
+// with hi the upper end of the covered interval, j = floor(hi).  hi advances
+// by m, one double add, and is biased by 2^20 + 2^19 so that its low word is
+// frac(hi) 2^32 and its high word j plus a constant (rounded to 2^-33 pixel a
+// step, under 2^-24 over a run of 512 lines).  Positions outside the image
+// read the zero padding.  The run's sum is double; a ray's runs are added in
+// order, times the ray's length per line, less the piece the tracer drops.
+//
+// What bounds it: the load, 17 accesses of the CU's L1 a line (four lanes an
+// access), beside 10 VALU instructions; a line brings the two pixels' entries
+// (1.4 entries of the matrix on average), where the checkpointed walk spends 26
+// VALU instructions and such a load on each entry.  512 x 512 pixels, 60 views
+// of 736 bins: 17.5 us (residual) and 17.0 us, against 32.4 and 32.1 us of the
+// walk; 4 waves a group 18.1 / 17.5 us, 16 waves 21.5 / 20.9, four lines in
+// flight instead of eight 18.0 / 17.4.  The run length is a multiple of 8
+// whatever K is, so a ray's sum does not depend on K.
+constexpr int kLineWaves = 8, kLineBlock = kLineWaves * kWave;
+constexpr double kLineBias = 1572864.0;                    // 2^20 + 2^19
+constexpr int kLineHi0 = (0x413 << 20) + (1 << 19);        // high word of kLineBias
+
+template <int K>
+__device__ __forceinline__ void load_pair(__amdgpu_buffer_rsrc_t rs, uint32_t off, int line, float (&o)[2 * K]) {
+    if constexpr (K == 1) {
+        const u32x2 a = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)off, line, 0);
+        __builtin_memcpy(o, &a, 8);
+    } else {
+#pragma unroll
+        for (int c = 0; c < K / 2; ++c) {
+            const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(off + 16 * c), line, 0);
+            __builtin_memcpy(&o[4 * c], &a, 16);
+        }
+    }
+}
+
+// Adds this lane's ray over lines c0 .. c0 + n - 1 (n a multiple of 8) to acc.
+template <int K>
+__device__ __forceinline__ void line_run(const GL float *img, int na, int nb, int c0, int n, double m, double b0,
+                                         float inv, double (&acc)[K]) {
+    constexpr int OS = K <= 2 ? 8 : (K == 4 ? 4 : 2);
+    const uint32_t lineb = (uint32_t)line_stride(nb) * K * 4;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc((const void *)img, (uint32_t)line_elems(na, nb) * K * 4);
+    double hi = b0 + 0.5 * fabs(m) + m * c0 + kLineBias;
+    const float sc = inv * 2.3283064365386963e-10f;   // 2^-32
+    uint32_t at = (uint32_t)c0 * lineb;
+    auto stage = [&](float (&w)[OS], float (&x)[OS][2 * K]) {
+        uint32_t off[OS];
+#pragma unroll
+        for (int k = 0; k < OS; ++k) {
+            const int h = __double2hiint(hi);
+            w[k] = __builtin_amdgcn_fmed3f((float)(uint32_t)__double2loint(hi) * sc, 0.0f, 1.0f);
+            const int j = max(kLineHi0 - 1, min(h, kLineHi0 + nb + 1));   // zeros beyond
+            off[k] = (uint32_t)(j - (kLineHi0 - 1)) * (4 * K);            // pixel j - 1, behind two of padding
+            hi += m;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < OS; ++k) load_pair<K>(rs, off[k], (int)(at + k * lineb), x[k]);
+        at += OS * lineb;
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto consume = [&](const float (&w)[OS], const float (&x)[OS][2 * K]) {
+#pragma unroll
+        for (int k = 0; k < OS; ++k)
+#pragma unroll
+            for (int j = 0; j < K; ++j) acc[j] += (double)__builtin_fmaf(w[k], x[k][K + j] - x[k][j], x[k][j]);
+    };
+    float wa[OS], wb[OS], xa[OS][2 * K], xb[OS][2 * K];
+    const int ng = n / OS;
+    stage(wa, xa);
+    int g = 1;
+    for (; g + 1 < ng; g += 2) {
+        stage(wb, xb);
+        consume(wa, xa);
+        stage(wa, xa);
+        consume(wb, xb);
+    }
+    if (g < ng) {
+        stage(wb, xb);
+        consume(wa, xa);
+        consume(wb, xb);
+    } else {
+        consume(wa, xa);
+    }
+}
+
+// RESID: r = g - A u (stored), partial sum r^2; else partial sum (A d)^2.
+template <int K, bool RESID>
+__device__ __forceinline__ void line_fp_unit(const EngArgs<float> &a, const UG<float> &U, int s, int lb, double *lds) {
+    const int lane = threadIdx.x & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int64_t g0 = U.ln_slice0[s] / 4;
+    if (lb >= U.ln_slice0[s + 1] / 4 - g0) return;
+    const int per = (U.nbins + kLineRays - 1) / kLineRays;
+    const int view = lb / per, bin = (lb - view * per) * kLineRays + lane;
+    const int64_t row = U.sub_row0[s] + (int64_t)view * U.nbins + bin;
+    const GL int32_t *rng = U.ln_rng + 4 * (g0 + lb);
+    double m = 0.0, b0 = 0.0;
+    float inv = 0.0f;
+    const bool valid = bin < U.nbins;
+    if (valid) {
+        m = U.ln_mb[2 * row];
+        b0 = U.ln_mb[2 * row + 1];
+        inv = U.ln_inv[row];
+    }
+    double acc[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) acc[j] = 0.0;
+#pragma unroll
+    for (int ax = 0; ax < 2; ++ax) {
+        const int r0 = rng[2 * ax], r1 = rng[2 * ax + 1];
+        if (r0 >= r1) continue;
+        // runs of a multiple of 8 lines; one reaching past r1 reads zeros
+        // there (its rays have left the image)
+        const int run = ((r1 - r0 + kLineWaves - 1) / kLineWaves + 7) & ~7, c0 = r0 + wv * run;
+        if (c0 >= r1) continue;
+        const bool mine = valid && (inv < 0.0f) == (ax == 1);
+        line_run<K>(ax ? U.py : U.px, ax ? U.ny : U.nx, ax ? U.nx : U.ny, c0, min(run, (r1 - c0 + 7) & ~7),
+                    mine ? m : 0.0, mine ? b0 : -64.0, mine ? fabsf(inv) : 0.0f, acc);
+    }
+    // thread (job k, ray): the ray's runs in order
+#pragma unroll
+    for (int j = 0; j < K; ++j) lds[(wv * K + j) * kLineRays + lane] = acc[j];
+    __syncthreads();
+    if (wv >= K) return;
+    double tot = 0.0;
+#pragma unroll
+    for (int w = 0; w < kLineWaves; ++w) tot += lds[(w * K + wv) * kLineRays + lane];
+    double mm = 0.0;
+    if (valid) {
+        tot *= U.ln_len[row];
+        const int dp = U.ln_drop[row];
+        if (dp >= 0) {
+            const int i = dp / U.ny, j = dp - i * U.ny;
+            tot -= (double)U.ln_dlen[row] * (double)U.px[((int64_t)i * line_stride(U.ny) + j + kLinePad) * K + wv];
+        }
+        if (RESID) {
+            const float o = (float)((double)U.g[row * K + wv] - tot);
+            U.r[row * K + wv] = o;
+            mm = (double)o * (double)o;
+        } else {
+            mm = tot * tot;
+        }
+    }
+    mm = group_sum<kWave>(mm);
+    if (lane == 0) part_at(a, U, RESID ? SL_DF : SL_AD, wv)[lb] = mm;
+}
+
 // K interleaved values at pixel (i, j), or `pad` outside the image.
 template <typename T, int K>
 __device__ __forceinline__ void ldn(const UG<T> &U, const GL T *arr, int i, int j, T (&o)[K], T pad) {
@@ -799,6 +967,7 @@ __device__ __forceinline__ void bp_unit(const EngArgs<T> &a, const UG<T> &U, int
                     dv[k] = (T)d;
                     m[k] = (double)dv[k] * (double)dv[k];
                 }
+                put_proj<T, K>(U, i, j, dv);
             } else {
                 zerok<T, K>(dv);
             }
@@ -906,9 +1075,8 @@ __device__ __forceinline__ void nv_unit(const EngArgs<T> &a, const UG<T> &U, int
     block_store<T, K, false>(a, U, SL_NV, lb, m, lds);
 }
 
-__device__ __forceinline__ bool real_pixel(int64_t q, int64_t npix_t, int tny, int nx, int ny) {
+__device__ __forceinline__ bool real_pixel(int64_t q, int64_t npix_t, int tny, int nx, int ny, int &i, int &j) {
     if (q >= npix_t) return false;
-    int i, j;
     tile_coords(q, tny, i, j);
     return i < nx && j < ny;
 }
@@ -917,21 +1085,23 @@ __device__ __forceinline__ bool real_pixel(int64_t q, int64_t npix_t, int tny, i
 template <typename T, int K>
 __device__ __forceinline__ void axpy_unit(const EngArgs<T> &a, const UG<T> &U, int lb) {
     const int64_t q = (int64_t)lb * kPixBlock + threadIdx.x;
-    if (!real_pixel(q, U.npix_t, U.tny, U.nx, U.ny)) return;
+    int i, j;
+    if (!real_pixel(q, U.npix_t, U.tny, U.nx, U.ny, i, j)) return;
     T uu[K], dd[K];
     loadk<T, K>(U.u + q * K, uu);
     loadk<T, K>(U.d + q * K, dd);
 #pragma unroll
-    for (int j = 0; j < K; ++j) {
-        const int js = U.job0 + j;
+    for (int k = 0; k < K; ++k) {
+        const int js = U.job0 + k;
         if (!job_live(a, js)) continue;
         const GL JobParams &P = jpar(a, js);
-        double yn = (double)uu[j] + jsc(a, js).c * (double)dd[j];
+        double yn = (double)uu[k] + jsc(a, js).c * (double)dd[k];
         if (yn < P.lower) yn = P.lower;
         if (yn > P.upper) yn = P.upper;
-        uu[j] = (T)yn;
+        uu[k] = (T)yn;
     }
     storek<T, K>(U.u + q * K, uu);
+    put_proj<T, K>(U, i, j, uu);
 }
 
 template <typename T>
@@ -987,10 +1157,12 @@ __device__ __forceinline__ void median_unit(const EngArgs<T> &a, const UG<T> &U,
 template <typename T, int K>
 __device__ __forceinline__ void copy_wu_unit(const UG<T> &U, int lb) {
     const int64_t q = (int64_t)lb * kPixBlock + threadIdx.x;
-    if (!real_pixel(q, U.npix_t, U.tny, U.nx, U.ny)) return;
+    int i, j;
+    if (!real_pixel(q, U.npix_t, U.tny, U.nx, U.ny, i, j)) return;
     T t[K];
     loadk<T, K>(U.w + q * K, t);
     storek<T, K>(U.u + q * K, t);
+    put_proj<T, K>(U, i, j, t);
 }
 
 template <typename T>
@@ -1082,7 +1254,8 @@ __device__ __forceinline__ void edge_update_unit(const EngArgs<T> &a, const UG<T
     double m[K];
 #pragma unroll
     for (int j = 0; j < K; ++j) m[j] = 0.0;
-    if (real_pixel(q, U.npix_t, U.tny, U.nx, U.ny)) {
+    int pi, pj;
+    if (real_pixel(q, U.npix_t, U.tny, U.nx, U.ny, pi, pj)) {
         T vv[K], ww[K];
         loadk<T, K>(U.v + q * K, vv);
         loadk<T, K>(U.w + q * K, ww);
@@ -1135,6 +1308,18 @@ __global__ __launch_bounds__(kBlock) void k_eng_fp(EngArgs<T> a, BlockMap m, int
     if (unit_idle(a, U)) return;
     const int lb = b - m.start[ui];
     MI_KSWITCH(KMAX, (fp_unit<T, K, RESID, FM>(a, U, s, lb, lds, ldr)))
+}
+
+template <int KMAX, bool RESID>
+__global__ __launch_bounds__(kLineBlock) void k_line_fp(EngArgs<float> a, BlockMap m, int s) {
+    __shared__ double lds[kLineWaves * KMAX * kLineRays];
+    const int b = (int)xcd_block();
+    if (b >= m.start[m.nunits]) return;
+    const int ui = find_unit(m, b);
+    const UG<float> U(a.units[ui]);
+    if (unit_idle(a, U)) return;
+    const int lb = b - m.start[ui];
+    MI_KSWITCH(KMAX, (line_fp_unit<K, RESID>(a, U, s, lb, lds)))
 }
 
 template <typename T, int KMAX, bool LDS, bool SQ>
@@ -1225,7 +1410,8 @@ __device__ __forceinline__ void fin_step(const EngArgs<T> &a, const UG<T> &U, in
     if (!job_live(a, js)) return;
     GL Scalars *sc = &jsc(a, js);
     const GL JobParams &P = jpar(a, js);
-    const int64_t nr = cdiv(U.fs_slice0[s + 1] - U.fs_slice0[s], kBlock / kWave);
+    const GL int64_t *fs0 = U.ln_slice0 ? U.ln_slice0 : U.fs_slice0;
+    const int64_t nr = cdiv(fs0[s + 1] - fs0[s], kBlock / kWave);
     const int64_t nb = cdiv(U.bs_slice0[s + 1] - U.bs_slice0[s], kBlock / kWave);
     const int64_t npx = cdiv(U.npix_t, kPixBlock);
     const GL double *const p[4] = {part_at(a, U, SL_DD, j), part_at(a, U, SL_AD, j), part_at(a, U, SL_NV, j),
@@ -1362,6 +1548,20 @@ __global__ void k_move(T *dst, int Kd, int sd, const T *src, int Ks, int ss, int
     if (i < n) dst[i * Kd + sd] = src[i * Ks + ss];
 }
 
+// u into the projection images: one thread per pixel and job, row by row
+// (px) or column by column (py).
+template <typename T>
+__global__ void k_spread(const T *u, T *px, T *py, int K, int nx, int ny, int tny) {
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= (int64_t)nx * ny * K) return;
+    const int64_t p = e / K;
+    const int k = (int)(e - p * K);
+    const int i = (int)(p / ny), j = (int)(p % ny);
+    const int jt = (int)(p / nx), it = (int)(p % nx);
+    px[((int64_t)i * line_stride(ny) + j + kLinePad) * K + k] = u[tile_index(i, j, tny) * K + k];
+    py[((int64_t)jt * line_stride(nx) + it + kLinePad) * K + k] = u[tile_index(it, jt, tny) * K + k];
+}
+
 // Plain streaming copy, 16 bytes per thread per step (the reference kernel
 // against which memory counters are read).
 __global__ __launch_bounds__(kBlock) void k_copy16(const u32x4 *__restrict__ src, u32x4 *__restrict__ dst,
@@ -1464,6 +1664,26 @@ void eng_fp_sq(hipStream_t st, const EngArgs<T> &a, const BlockMap &rows, int s,
     MI_HIP(hipGetLastError());
 }
 
+void eng_line_fp(hipStream_t st, const EngArgs<float> &a, const BlockMap &m, int s, int kmax, bool resid) {
+    const dim3 grid(grid8(m.start[m.nunits])), block(kLineBlock);
+    if (resid) {
+        if (kmax == 1) launch(k_line_fp<1, true>, grid, block, 0u, st, a, m, s);
+        else if (kmax <= 4) launch(k_line_fp<4, true>, grid, block, 0u, st, a, m, s);
+        else launch(k_line_fp<kMaxK, true>, grid, block, 0u, st, a, m, s);
+    } else {
+        if (kmax == 1) launch(k_line_fp<1, false>, grid, block, 0u, st, a, m, s);
+        else if (kmax <= 4) launch(k_line_fp<4, false>, grid, block, 0u, st, a, m, s);
+        else launch(k_line_fp<kMaxK, false>, grid, block, 0u, st, a, m, s);
+    }
+    MI_HIP(hipGetLastError());
+}
+
+template <typename T>
+void eng_spread(hipStream_t st, const T *u, T *px, T *py, int K, int nx, int ny, int tny) {
+    k_spread<T><<<grid_of((int64_t)nx * ny * K), kBlock, 0, st>>>(u, px, py, K, nx, ny, tny);
+    MI_HIP(hipGetLastError());
+}
+
 template <typename T, int OP>
 static void launch_pix(hipStream_t st, const EngArgs<T> &a, const BlockMap &m, int it, int kmax) {
     const unsigned grid = grid8(m.start[m.nunits]);
@@ -1544,6 +1764,7 @@ void eng_copy(hipStream_t st, void *dst, const void *src, int64_t bytes) {
     template void eng_fp_resid<T>(hipStream_t, const EngArgs<T> &, const BlockMap &, int, int, bool);       \
     template void eng_bp_grad<T>(hipStream_t, const EngArgs<T> &, const BlockMap &, int, int, size_t, int); \
     template void eng_fp_sq<T>(hipStream_t, const EngArgs<T> &, const BlockMap &, int, int, bool);         \
+    template void eng_spread<T>(hipStream_t, const T *, T *, T *, int, int, int, int);                     \
     template void eng_nv<T>(hipStream_t, const EngArgs<T> &, const BlockMap &, int);                        \
     template void eng_axpy<T>(hipStream_t, const EngArgs<T> &, const BlockMap &, int);                      \
     template void eng_median<T>(hipStream_t, const EngArgs<T> &, const BlockMap &, int);                    \

@@ -76,9 +76,20 @@ struct UnitDesc {
     // forward block of kOtfRays rays x kOtfSeg segments (runtime.hpp)
     const double *ot_lam, *ot_ax, *ot_ay, *ot_stx, *ot_sty;
     const int32_t *ot_cx, *ot_cy, *ot_sg, *ot_cnt;
+    // rays as lines (FP32 fan beams; null otherwise), see Lines
+    const int64_t *ln_slice0;
+    const double2 *ln_mb;
+    const double *ln_len;
+    const float *ln_inv, *ln_dlen;
+    const int32_t *ln_drop;
+    const int4 *ln_rng;
     const int64_t *sub_row0;               // S + 1 row offsets
     T *g, *r;                              // rows * K
     T *u, *v, *d, *w;                      // npix_t * K
+    // projection images of a unit with lines: the image to be projected next
+    // (u, or d between the back projection and the update), row by row and
+    // column by column, zero-padded (line_stride / line_elems), K interleaved
+    T *px, *py;
     int64_t npix_t, nrows;
     int64_t part_off, cap;                 // partials: part + part_off + (slot * K + j) * cap
     int nx, ny, tny, K, fs_P, bs_P;
@@ -120,6 +131,12 @@ void eng_bp_grad(hipStream_t st, const EngArgs<T> &a, const BlockMap &m, int s, 
 // residual) and nV(d) (pixel map), as two launches.
 template <typename T>
 void eng_fp_sq(hipStream_t st, const EngArgs<T> &a, const BlockMap &rows, int s, int kmax, bool all_walk);
+// The two forward projections of units with lines (FP32): r = g - A_s u and
+// ||A_s d||^2, from the unit's projection images.
+void eng_line_fp(hipStream_t st, const EngArgs<float> &a, const BlockMap &m, int s, int kmax, bool resid);
+// Writes u into the unit's projection images.
+template <typename T>
+void eng_spread(hipStream_t st, const T *u, T *px, T *py, int K, int nx, int ny, int tny);
 template <typename T>
 void eng_nv(hipStream_t st, const EngArgs<T> &a, const BlockMap &pix, int kmax);
 template <typename T>

@@ -151,6 +151,41 @@ struct Otf {
     }
 };
 
+// Fan-beam rays as lines (FP32 engine).  A ray crosses the image along its
+// dominant axis A (rows x when |rx| >= |ry|, else columns y); in pixel units
+// its cross coordinate at the middle of line a of that axis is b0 + m a,
+// |m| <= 1, so inside line a it covers [b0 + m a - |m| / 2, b0 + m a + |m| / 2]
+// and meets at most two pixels.  The length in pixel (a, j) is
+//   len * min(1, max(0, ((1 + |m|) / 2 - |b0 + m a - j - 1/2|) / |m|)),
+// the tracer's own length up to its rounding, except that the tracer leaves
+// out a piece that begins within 0.05 mm of the exit: that pixel and length
+// are kept per ray (drop / dlen; at most one for pixels above 0.05 mm).
+// build_lines walks every ray with the tracer and checks each piece against
+// this form; a geometry where one differs keeps the stored matrix.
+//
+// Rows are the matrix's (subset order); a group is kLineRays consecutive bins
+// of one view, ceil(n_bins / kLineRays) groups per view.
+constexpr int kLineRays = kWave;
+constexpr int kLinePad = 2;      // zero pixels on each side of a projection image's line
+constexpr int kLineRows = 8;     // zero lines behind its last one
+__host__ __device__ __forceinline__ int64_t line_stride(int n) { return n + 2 * kLinePad; }
+__host__ __device__ __forceinline__ int64_t line_elems(int na, int nb) {
+    return (int64_t)(na + kLineRows) * line_stride(nb);
+}
+struct Lines {
+    std::vector<int64_t> slice0;     // S + 1: 4 x the first group of each subset (a group is one workgroup)
+    DevBuf<int64_t> d_slice0;
+    DevBuf<double2> mb;              // per row: m, b0
+    DevBuf<double> len;              // per row: mm per line of the dominant axis (0: misses the image)
+    DevBuf<float> inv;               // per row: 1 / |m| (1e30 for a ray along the axis), negative when the axis is y
+    DevBuf<int32_t> drop;            // per row: pixel (x ny + y) whose piece is left out, -1: none
+    DevBuf<float> dlen;              // per row: its length
+    DevBuf<int4> rng;                // per group: lines its x-dominant rays cross [x, y), its y-dominant ones [z, w)
+    size_t bytes() const {
+        return d_slice0.bytes() + mb.bytes() + len.bytes() + inv.bytes() + drop.bytes() + dlen.bytes() + rng.bytes();
+    }
+};
+
 constexpr int kGroup = 4;
 __host__ __device__ __forceinline__ int64_t sell_pos(int64_t base, int t, int lane) {
     return base + (int64_t)(t >> 2) * (kGroup * 64) + lane * kGroup + (t & 3);
@@ -212,6 +247,8 @@ struct Matrix {
     Sell fs, bs;
     Otf otf;
     bool has_otf = false;
+    Lines lines;
+    bool has_lines = false;          // every ray of the geometry has the line form
     int tny = 0;
     int64_t npix_t = 0;
     bool has_sell = false;

@@ -350,7 +350,7 @@ void build_sell(Matrix &m, hipStream_t st, bool drop_csr) {
     m.npix_t = (int64_t)((g.nx + kTileH - 1) / kTileH) * kTileH * m.tny * kTileW;
     const bool f64 = m.has64;
     // forward
-    if (!m.has_otf) {   // the checkpointed walk replaces the stored forward slices
+    if (!m.has_otf && !m.has_lines) {   // the lines or the checkpointed walk replace the stored forward slices
         m.fs.P = choose_p(MI_SELL_PF, (double)m.nnz / std::max<int64_t>(m.nrows, 1));
         m.fs.C = kWave / m.fs.P;
         m.fs.slice0.assign(m.S + 1, 0);

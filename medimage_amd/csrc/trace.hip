@@ -384,6 +384,134 @@ void build_otf(Matrix &m, const TraceArgs &a, hipStream_t st) {
     m.has_otf = true;
 }
 
+// One lane per ray, one wave per group: the line form of the ray (Lines), and
+// its check.  The ray is walked with the tracer; every piece must have the
+// length the line form gives its pixel (1e-5 pixel covers the double rounding
+// of both; a piece in another pixel differs by far more), nothing but the one
+// final piece may be missing, and source and detector must lie outside the
+// image.  Rays the tracer treats as parallel to an axis (|r| <= 1e-4 mm across
+// it) stay in their first pixel's line, as its 1e6 sentinel keeps them.
+struct LineOut {
+    double2 *mb;
+    double *len;
+    float *inv, *dlen;
+    int32_t *drop;
+    int4 *rng;
+    unsigned *bad;
+};
+__global__ __launch_bounds__(kLineRays) void k_lines_fill(TraceArgs a, const int64_t *sub_row0, const int64_t *slice0,
+                                                          int S, LineOut o) {
+    const int64_t grp = blockIdx.x;
+    int s = 0;
+    while (s + 1 < S && slice0[s + 1] <= 4 * grp) ++s;
+    const int per = (a.nbins + kLineRays - 1) / kLineRays;
+    const int64_t lg = grp - slice0[s] / 4;
+    const int lane = threadIdx.x, bin = (int)(lg % per) * kLineRays + lane;
+    const int64_t row = sub_row0[s] + lg / per * a.nbins + bin;
+    const FanGeom &g = a.fan;
+    int r0 = INT32_MAX, r1 = 0;   // lines crossed
+    bool yd = false, bad = false;
+    if (bin < a.nbins) {
+        const int view = a.vlist[row / a.nbins];
+        double sx, sy, dx, dy;
+        ray_endpoints(g, a.fcos[view], a.fsin[view], a.dcos, a.dsin, bin, sx, sy, dx, dy);
+        const double rx = dx - sx, ry = dy - sy, L = sqrt(rx * rx + ry * ry);
+        double m = 0.0, b0 = -64.0, len = 0.0, inv = 1e30;
+        int drop = -1;
+        float dlen = 0.0f;
+        SiddonState st;
+        if (siddon_init(sx, sy, dx, dy, g.nx, g.ny, g.vx, g.vy, st)) {
+            yd = fabs(ry) > fabs(rx);
+            const double ra = yd ? ry : rx, rb = yd ? rx : ry, sa = yd ? sy : sx, sb = yd ? sx : sy, v = g.vx;
+            bad = !(st.lam > 0.0) || !(st.hi < L);
+            len = L / fabs(ra) * v;
+            if (fabs(rb) <= 1.e-4) {
+                b0 = (yd ? st.cx : st.cy) + 0.5;
+            } else {
+                m = rb / ra;
+                b0 = sb / v + (0.5 - sa / v) * m;
+                inv = fmin(inv, 1.0 / fabs(m));
+            }
+            const double H = 0.5 + 0.5 * fabs(m);
+            auto length = [&](int cx, int cy) {
+                const double D = b0 + m * (yd ? cy : cx) - (yd ? cx : cy) - 0.5;
+                return len * fmin(1.0, fmax(0.0, (H - fabs(D)) * inv));
+            };
+            const double a0 = (sa + st.lam * ra / L) / v, a1 = (sa + st.hi * ra / L) / v;
+            const int na = yd ? g.ny : g.nx;
+            r0 = max(0, (int)floor(fmin(a0, a1) - 1e-6));
+            r1 = min(na, (int)ceil(fmax(a0, a1) + 1e-6));
+            bool in = true;
+            while (st.lam < st.hi - 5.e-2) {
+                in = st.cx >= 0 && st.cx < g.nx && st.cy >= 0 && st.cy < g.ny;
+                if (!in) break;
+                int cx, cy;
+                double w;
+                siddon_step(st, cx, cy, w);
+                bad |= !(fabs(w - length(cx, cy)) <= 1e-5 * v);
+            }
+            const double rem = st.hi - st.lam;
+            bad |= !in || rem > 5.0000001e-2;
+            if (rem > 1e-9) {
+                if (st.cx >= 0 && st.cx < g.nx && st.cy >= 0 && st.cy < g.ny) {
+                    const double w = length(st.cx, st.cy);
+                    bad |= !(fabs(w - rem) <= 1e-5 * v);
+                    if (w > 0.0) {
+                        drop = st.cx * g.ny + st.cy;
+                        dlen = (float)w;
+                    }
+                } else {
+                    bad |= rem > 1e-5 * v;
+                }
+            }
+        }
+        o.mb[row] = make_double2(m, b0);
+        o.len[row] = len;
+        o.inv[row] = yd ? -(float)inv : (float)inv;
+        o.drop[row] = drop;
+        o.dlen[row] = dlen;
+    }
+    int x0 = yd ? INT32_MAX : r0, x1 = yd ? 0 : r1, y0 = yd ? r0 : INT32_MAX, y1 = yd ? r1 : 0;
+    for (int w = kWave / 2; w > 0; w >>= 1) {
+        x0 = min(x0, __shfl_xor(x0, w, kWave));
+        x1 = max(x1, __shfl_xor(x1, w, kWave));
+        y0 = min(y0, __shfl_xor(y0, w, kWave));
+        y1 = max(y1, __shfl_xor(y1, w, kWave));
+    }
+    if (lane == 0) o.rng[grp] = make_int4(min(x0, x1), x1, min(y0, y1), y1);
+    if (__any(bad) && lane == 0) atomicOr(o.bad, 1u);
+}
+
+// The line form of every ray; false (and nothing kept) when the geometry has
+// a ray without it, or an image beyond the 32-bit offsets of the kernels.
+bool build_lines(Matrix &m, const TraceArgs &a, hipStream_t st) {
+    const mi_geometry &g = m.g;
+    if (!(g.pixel_mm > 0.0501) || (int64_t)(g.nx + 64) * (g.ny + 64) >= (int64_t)1 << 26) return false;
+    Lines &q = m.lines;
+    const int64_t per = (g.n_bins + kLineRays - 1) / kLineRays;
+    q.slice0.assign(m.S + 1, 0);
+    for (int s = 0; s < m.S; ++s) q.slice0[s + 1] = q.slice0[s] + 4 * per * ((m.sub_row0[s + 1] - m.sub_row0[s]) / g.n_bins);
+    const int64_t groups = q.slice0.back() / 4;
+    upload(q.d_slice0, q.slice0, st);
+    q.mb.alloc(m.nrows);
+    q.len.alloc(m.nrows);
+    q.inv.alloc(m.nrows);
+    q.drop.alloc(m.nrows);
+    q.dlen.alloc(m.nrows);
+    q.rng.alloc(groups);
+    DevBuf<unsigned> bad(1);
+    MI_HIP(hipMemsetAsync(bad.p, 0, sizeof(unsigned), st));
+    const LineOut o{q.mb.p, q.len.p, q.inv.p, q.dlen.p, q.drop.p, q.rng.p, bad.p};
+    k_lines_fill<<<(unsigned)groups, kLineRays, 0, st>>>(a, m.d_sub_row0.p, q.d_slice0.p, m.S, o);
+    MI_HIP(hipGetLastError());
+    unsigned h = 0;
+    MI_HIP(hipMemcpyAsync(&h, bad.p, sizeof(h), hipMemcpyDeviceToHost, st));
+    MI_HIP(hipStreamSynchronize(st));
+    m.has_lines = h == 0;
+    if (!m.has_lines) m.lines = Lines{};
+    return m.has_lines;
+}
+
 // Entries of each subset's rows, from the device row pointer.
 void subset_counts(Matrix &m, hipStream_t st) {
     std::vector<int64_t> at(m.S + 1);
@@ -410,7 +538,7 @@ std::vector<int> subset_order(int S) {
 }
 
 size_t Matrix::bytes() const {
-    return otf.bytes() + d_vlist.bytes() + d_sub_row0.bytes() + rowptr.bytes() + idx.bytes() + len32.bytes() + len64.bytes() + colptr.bytes() +
+    return lines.bytes() + otf.bytes() + d_vlist.bytes() + d_sub_row0.bytes() + rowptr.bytes() + idx.bytes() + len32.bytes() + len64.bytes() + colptr.bytes() +
            crow.bytes() + clen32.bytes() + clen64.bytes() + perm.bytes() + fs.bytes() + bs.bytes() +
            seq_bytes(seq.get());
 }
@@ -551,7 +679,11 @@ std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, h
     MI_HIP(hipGetLastError());
     build_csc(*m, m->rowptr.p, m->idx.p, m->len32.p, want64 ? m->len64.p : nullptr, st);
     subset_counts(*m, st);
-    if (otf && (g.beam == MI_BEAM_FAN_FLAT || g.beam == MI_BEAM_FAN_ARC)) build_otf(*m, a, st);
+    if (otf && (g.beam == MI_BEAM_FAN_FLAT || g.beam == MI_BEAM_FAN_ARC)) {
+        // FP32 runs project along the lines; FP64 runs, and geometries with a
+        // ray that has no line form, re-run the tracer from checkpoints
+        if (!build_lines(*m, a, st) || want64) build_otf(*m, a, st);
+    }
     return m;
 }
 
