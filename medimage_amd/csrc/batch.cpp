@@ -598,7 +598,6 @@ void Batch<T>::record_pass(bool timed) {
             if (ln[c].any()) eng_line_fp(q, args, ln[c].map, s, ln[c].kmax, resid);
         }
     };
-    eng_finalize<T>(st, args, EF_BEGIN, 0);
     for (int s = 0; s < S; ++s) {
         auto nnz_s = [&](const Unit<T> &U) { return (double)U.m->sub_nnz[s]; };
         auto nr_s = [&](const Unit<T> &U) { return (double)(U.m->sub_row0[s + 1] - U.m->sub_row0[s]); };
@@ -650,9 +649,10 @@ void Batch<T>::record_pass(bool timed) {
     if (any_median) eng_median<T>(st, args, pix, kmax);
     if (edge_iters > 0) {
         LaunchTimer lt(ctx, MI_K_EDGE, sum([&](const Unit<T> &U) { return 7.0 * U.m->npix * sz * U.K * edge_iters; }));
-        for (int it = 0; it < edge_iters; ++it) eng_edge_iter<T>(st, args, pix, it, kmax);
+        for (int it = 0; it < edge_iters; ++it) eng_edge_iter<T>(st, args, pix, it, kmax, it + 1 == edge_iters);
+    } else {
+        eng_finalize<T>(st, args, EF_END, 0);
     }
-    eng_finalize<T>(st, args, EF_END, 0);
 }
 
 template <typename T>

@@ -1439,12 +1439,6 @@ __device__ __forceinline__ void fin_job(const EngArgs<T> &a, const UG<T> &U, int
     const GL JobParams &P = jpar(a, js);
     const int64_t npx = cdiv(U.npix_t, kPixBlock);
     switch (op) {
-        case EF_BEGIN:
-            if (threadIdx.x == 0) {
-                sc->df_pass = 0.0;
-                sc->edge_done = 0;
-            }
-            break;
         case EF_EDGE_C: {
             if (sc->edge_done || s >= P.iter_edge) return;
             const GL double *const p[3] = {part_at(a, U, SL_E0, j), part_at(a, U, SL_E1, j),
@@ -1462,15 +1456,17 @@ __device__ __forceinline__ void fin_job(const EngArgs<T> &a, const UG<T> &U, int
             }
             break;
         }
-        case EF_EDGE_DONE: {
-            if (sc->edge_done || s >= P.iter_edge) return;
-            const double mx = fin_reduce(part_at(a, U, SL_E3, j), npx, true, lds);
-            if (threadIdx.x == 0) {
-                sc->e_maxcd = mx;
-                if (mx < 1e-5) sc->edge_done = 1;   // main.c:351
+        case EF_EDGE_DONE:
+        case EF_EDGE_END:
+            if (!sc->edge_done && s < P.iter_edge) {
+                const double mx = fin_reduce(part_at(a, U, SL_E3, j), npx, true, lds);
+                if (threadIdx.x == 0) {
+                    sc->e_maxcd = mx;
+                    if (mx < 1e-5) sc->edge_done = 1;   // main.c:351
+                }
             }
-            break;
-        }
+            if (op == EF_EDGE_DONE) break;
+            [[fallthrough]];
         default: {  // EF_END
             if (threadIdx.x != 0) return;
             const double df = sc->df_pass;
@@ -1480,6 +1476,8 @@ __device__ __forceinline__ void fin_job(const EngArgs<T> &a, const UG<T> &U, int
                 if (diff < P.rel_tol * sc->df_prev) sc->converged = 1;
             }
             sc->df_prev = df;
+            sc->df_pass = 0.0;
+            sc->edge_done = 0;
             sc->iters += 1;
             if (sc->converged || (P.max_iters > 0 && sc->iters >= P.max_iters)) sc->done = 1;
             break;
@@ -1710,12 +1708,12 @@ void eng_median(hipStream_t st, const EngArgs<T> &a, const BlockMap &pix, int km
 }
 
 template <typename T>
-void eng_edge_iter(hipStream_t st, const EngArgs<T> &a, const BlockMap &pix, int it, int kmax) {
+void eng_edge_iter(hipStream_t st, const EngArgs<T> &a, const BlockMap &pix, int it, int kmax, bool last) {
     launch_pix<T, PX_EDGE_GRAD>(st, a, pix, it, kmax);
     launch_pix<T, PX_EDGE_NABLA>(st, a, pix, it, kmax);
     eng_finalize<T>(st, a, EF_EDGE_C, it);
     launch_pix<T, PX_EDGE_UPDATE>(st, a, pix, it, kmax);
-    eng_finalize<T>(st, a, EF_EDGE_DONE, it);
+    eng_finalize<T>(st, a, last ? EF_EDGE_END : EF_EDGE_DONE, it);
 }
 
 template <typename T>
@@ -1768,7 +1766,7 @@ void eng_copy(hipStream_t st, void *dst, const void *src, int64_t bytes) {
     template void eng_nv<T>(hipStream_t, const EngArgs<T> &, const BlockMap &, int);                        \
     template void eng_axpy<T>(hipStream_t, const EngArgs<T> &, const BlockMap &, int);                      \
     template void eng_median<T>(hipStream_t, const EngArgs<T> &, const BlockMap &, int);                    \
-    template void eng_edge_iter<T>(hipStream_t, const EngArgs<T> &, const BlockMap &, int, int);            \
+    template void eng_edge_iter<T>(hipStream_t, const EngArgs<T> &, const BlockMap &, int, int, bool);      \
     template void eng_finalize<T>(hipStream_t, const EngArgs<T> &, int, int);                               \
     template void eng_put_rows<T>(hipStream_t, T *, int, int, int64_t, const int64_t *, const T *);         \
     template void eng_put_img<T>(hipStream_t, T *, int, int, int, int, int, const T *, T);                  \

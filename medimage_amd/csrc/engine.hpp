@@ -143,10 +143,14 @@ template <typename T>
 void eng_axpy(hipStream_t st, const EngArgs<T> &a, const BlockMap &pix, int kmax);
 template <typename T>
 void eng_median(hipStream_t st, const EngArgs<T> &a, const BlockMap &pix, int kmax);
+// last: the pass's last iteration, which also ends the pass.
 template <typename T>
-void eng_edge_iter(hipStream_t st, const EngArgs<T> &a, const BlockMap &pix, int it, int kmax);
+void eng_edge_iter(hipStream_t st, const EngArgs<T> &a, const BlockMap &pix, int it, int kmax, bool last);
 
-enum EngFin { EF_BEGIN = 0, EF_STEP, EF_EDGE_C, EF_EDGE_DONE, EF_END };
+// EF_EDGE_END: EF_EDGE_DONE of a pass's last edge iteration and EF_END in one
+// launch.  EF_END leaves the job's sums cleared for its next pass (a new job's
+// scalars start at zero), so no launch opens a pass.
+enum EngFin { EF_STEP = 0, EF_EDGE_C, EF_EDGE_DONE, EF_EDGE_END, EF_END };
 template <typename T>
 void eng_finalize(hipStream_t st, const EngArgs<T> &a, int op, int s);
 
