@@ -24,7 +24,7 @@ bool use_lines(const Matrix &m) {
 
 template <typename T>
 int64_t unit_state_bytes(const Matrix &m, int K) {
-    int64_t e = 2 * m.nrows + 4 * m.npix_t;
+    int64_t e = 2 * m.nrows + kLineEmpty + 4 * m.npix_t;
     if (use_lines<T>(m)) e += line_elems(m.g.nx, m.g.ny) + line_elems(m.g.ny, m.g.nx);
     return (int64_t)K * e * (int64_t)sizeof(T);
 }
@@ -71,7 +71,8 @@ int64_t free_device_bytes() {
 
 template <typename T>
 void Unit<T>::alloc(hipStream_t st) {
-    g.n = r.n = (size_t)m->nrows * K;
+    g.n = (size_t)m->nrows * K;
+    r.n = (size_t)(m->nrows + kLineEmpty) * K;   // the back projection reads past a view's last bin
     for (Part *b : {&u, &v, &d, &w}) b->n = (size_t)m->npix_t * K;
     if (use_lines<T>(*m)) {
         px.n = (size_t)line_elems(m->g.nx, m->g.ny) * K;
@@ -453,6 +454,11 @@ void Batch<T>::rebuild() {
         L->map.nunits = (int)live.size();
         L->map.start[0] = 0;
     }
+    for (auto &k : lnb)
+        for (Launch &L : k) {
+            L = Launch{};
+            L.map.nunits = (int)live.size();
+        }
     const bool f64 = sizeof(T) == 8;
     for (size_t i = 0; i < live.size(); ++i) {
         Unit<T> &U = *units[live[i]];
@@ -468,6 +474,17 @@ void Batch<T>::rebuild() {
             D.ln_dlen = m.lines.dlen.p;
             D.ln_drop = m.lines.drop.p;
             D.ln_rng = m.lines.rng.p;
+            D.ln_mx = m.lines.mx.p;
+            D.ln_my = m.lines.my.p;
+            D.ln_ix = m.lines.ix.p;
+            D.ln_iy = m.lines.iy.p;
+            D.ln_win0 = m.lines.d_win0.p;
+            D.ln_views = m.lines.views.p;
+            D.ln_sod = m.lines.sod;
+            D.ln_k = m.lines.k;
+            D.ln_bin0 = m.lines.bin0;
+            D.ln_pix = (float)m.g.pixel_mm;
+            D.ln_arc = m.lines.arc;
             D.px = U.px.p;
             D.py = U.py.p;
         }
@@ -504,8 +521,9 @@ void Batch<T>::rebuild() {
         const size_t need = m.bs.slot16.p ? (size_t)m.bs.max_slots * U.K * sizeof(T) : kBpLdsHw + 1;
         const bool in_lds = bp_in_lds(m, need);
         const int rc = U.K > 1 ? 1 : 0, bc = U.K > 4 ? 1 : 0;   // the unit's classes
+        const int ng = line_groups(bp_blocks(m)) / 2;   // 0, 1, 2
         const int lc = need > kBpLdsSplit ? 1 : 0;
-        Launch &B = in_lds ? bpl[bc][lc] : bpg[bc];
+        Launch &B = lines ? lnb[bc][ng] : in_lds ? bpl[bc][lc] : bpg[bc];
         B.kmax = std::max(B.kmax, U.K);
         if (in_lds) B.lds = std::max(B.lds, need);
         Launch &F = lines ? ln[rc] : rows[rc];
@@ -536,9 +554,13 @@ void Batch<T>::rebuild() {
             ln[c].map.start[i + 1] = ln[c].map.start[i] + (lines ? fb : 0);
             for (int l = 0; l < 2; ++l)
                 bpl[c][l].map.start[i + 1] =
-                    bpl[c][l].map.start[i] + (in_lds && c == bc && l == lc ? (int)bp_blocks(m) : 0);
-            bpg[c].map.start[i + 1] = bpg[c].map.start[i] + (!in_lds && c == bc ? (int)bp_blocks(m) : 0);
+                    bpl[c][l].map.start[i] + (!lines && in_lds && c == bc && l == lc ? (int)bp_blocks(m) : 0);
+            bpg[c].map.start[i + 1] = bpg[c].map.start[i] + (!lines && !in_lds && c == bc ? (int)bp_blocks(m) : 0);
         }
+        for (int c = 0; c < 2; ++c)
+            for (int l = 0; l < 3; ++l)
+                lnb[c][l].map.start[i + 1] =
+                    lnb[c][l].map.start[i] + (lines && c == bc && l == ng ? (int)bp_blocks(m) : 0);
         pix.start[i + 1] = pix.start[i] + (int)px_blocks(m);
         kmax = std::max(kmax, U.K);
         all_walk = all_walk && (lines || m.has_otf);
@@ -598,6 +620,22 @@ void Batch<T>::record_pass(bool timed) {
             if (ln[c].any()) eng_line_fp(q, args, ln[c].map, s, ln[c].kmax, resid);
         }
     };
+    // ... and their back projection: the K <= 4 units in one group a block on
+    // one stream (branch 0), all others, smaller images and K = 8, beside it
+    auto any_lnb = [&](int c) {
+        bool y = false;
+        for (int k = 0; k < 2; ++k)
+            for (int l = 0; l < 3; ++l) y = y || ((c == 0) == (k == 0 && l == 0) && lnb[k][l].any());
+        return y;
+    };
+    auto line_bp = [&](hipStream_t q, int c, int s) {
+        if constexpr (sizeof(T) == 4) {
+            for (int k = 0; k < 2; ++k)
+                for (int l = 0; l < 3; ++l)
+                    if ((c == 0) == (k == 0 && l == 0) && lnb[k][l].any())
+                        eng_line_bp(q, args, lnb[k][l].map, s, lnb[k][l].kmax, 1 << l);
+        }
+    };
     for (int s = 0; s < S; ++s) {
         auto nnz_s = [&](const Unit<T> &U) { return (double)U.m->sub_nnz[s]; };
         auto nr_s = [&](const Unit<T> &U) { return (double)(U.m->sub_row0[s + 1] - U.m->sub_row0[s]); };
@@ -622,10 +660,11 @@ void Batch<T>::record_pass(bool timed) {
                     for (const Launch &L : bpl[c])
                         if (L.any()) eng_bp_grad<T>(q, args, L.map, s, L.kmax, L.lds, bp_sq);
                     if (bpg[c].any()) eng_bp_grad<T>(q, args, bpg[c].map, s, bpg[c].kmax, 0);
+                    line_bp(q, c, s);
                 };
             };
-            branches(one(0), one(1), bpl[0][0].any() || bpl[0][1].any() || bpg[0].any(),
-                     bpl[1][0].any() || bpl[1][1].any() || bpg[1].any());
+            branches(one(0), one(1), bpl[0][0].any() || bpl[0][1].any() || bpg[0].any() || any_lnb(0),
+                     bpl[1][0].any() || bpl[1][1].any() || bpg[1].any() || any_lnb(1));
         }
         {
             LaunchTimer lt(ctx, MI_K_FPSQ, sum([&](const Unit<T> &U) {

@@ -129,8 +129,11 @@ struct Batch {
         size_t lds = 0;
         bool any() const { return map.start[map.nunits] > 0; }
     };
-    // Units with lines have their forward rows in ln instead of rows.
-    Launch rows[2], ln[2], bpl[2][2], bpg[2];   // bpl[K class][LDS class]
+    // Units with lines have their forward rows in ln instead of rows, and
+    // their back projection in lnb (by K <= 4 / K = 8 and by line_groups 1, 2,
+    // 4; K = 1 units share the launch of larger ones, they would only run one
+    // after the other).
+    Launch rows[2], ln[2], lnb[2][3], bpl[2][2], bpg[2];   // bpl[K class][LDS class]
     hipStream_t side = nullptr;   // the second class of a phase
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     EngArgs<T> args{};

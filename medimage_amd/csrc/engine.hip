@@ -57,10 +57,15 @@ struct UG {
     const GL double *ln_mb, *ln_len;
     const GL float *ln_inv, *ln_dlen;
     const GL int32_t *ln_drop, *ln_rng;
+    const GL double *ln_mx, *ln_my;
+    const GL float *ln_ix, *ln_iy;
+    const GL int64_t *ln_win0;
+    const GL int32_t *ln_views;
     const GL int64_t *sub_row0;
     GL T *g, *r, *u, *v, *d, *w, *px, *py;
     int64_t npix_t, nrows, part_off, cap;
-    int nx, ny, tny, K, fs_P, bs_P, job0, nbins;
+    int nx, ny, tny, K, fs_P, bs_P, job0, nbins, ln_arc;
+    float ln_sod, ln_k, ln_bin0, ln_pix;
     __device__ __forceinline__ explicit UG(const UnitDesc<T> &D)
         : fs_slice0((const GL int64_t *)D.fs_slice0), fs_base((const GL int64_t *)D.fs_base),
           fs_T((const GL int32_t *)D.fs_T), fs_idx((const GL uint32_t *)D.fs_idx),
@@ -77,11 +82,14 @@ struct UG {
           ot_sg((const GL int32_t *)D.ot_sg), ot_cnt((const GL int32_t *)D.ot_cnt),
           ln_slice0((const GL int64_t *)D.ln_slice0), ln_mb((const GL double *)D.ln_mb),
           ln_len((const GL double *)D.ln_len), ln_inv((const GL float *)D.ln_inv), ln_dlen((const GL float *)D.ln_dlen),
-          ln_drop((const GL int32_t *)D.ln_drop), ln_rng((const GL int32_t *)D.ln_rng),
+          ln_drop((const GL int32_t *)D.ln_drop), ln_rng((const GL int32_t *)D.ln_rng), ln_mx((const GL double *)D.ln_mx),
+          ln_my((const GL double *)D.ln_my), ln_ix((const GL float *)D.ln_ix), ln_iy((const GL float *)D.ln_iy),
+          ln_win0((const GL int64_t *)D.ln_win0), ln_views((const GL int32_t *)D.ln_views),
           sub_row0((const GL int64_t *)D.sub_row0), g((GL T *)D.g), r((GL T *)D.r), u((GL T *)D.u),
           v((GL T *)D.v), d((GL T *)D.d), w((GL T *)D.w), px((GL T *)D.px), py((GL T *)D.py), npix_t(D.npix_t), nrows(D.nrows),
           part_off(D.part_off), cap(D.cap), nx(D.nx), ny(D.ny), tny(D.tny), K(D.K), fs_P(D.fs_P), bs_P(D.bs_P),
-          job0(D.job0), nbins(D.nbins) {}
+          job0(D.job0), nbins(D.nbins), ln_arc(D.ln_arc), ln_sod(D.ln_sod), ln_k(D.ln_k), ln_bin0(D.ln_bin0),
+          ln_pix(D.ln_pix) {}
     // Tiled index of pixel (i, j), or -1 outside the image.
     __device__ __forceinline__ int64_t at(int i, int j) const {
         return (i < 0 || j < 0 || i >= nx || j >= ny) ? -1 : tile_index(i, j, tny);
@@ -238,17 +246,19 @@ __device__ __forceinline__ GL double *part_at(const EngArgs<T> &a, const UG<T> &
     return (GL double *)a.part + U.part_off + ((int64_t)slot * U.K + j) * U.cap;
 }
 
-// Sum (or max) of one value per thread for each of K jobs; thread j < K
-// stores job j's block total at part_at(slot, j)[lb].  Fixed order.
+// Sum (or max) of one value per thread (of the block's first kBlock) for each
+// of K jobs; thread j < K stores job j's block total at part_at(slot, j)[lb].
+// Fixed order.
 template <typename T, int K, bool MAX>
 __device__ __forceinline__ void block_store(const EngArgs<T> &a, const UG<T> &U, int slot, int lb,
                                             const double (&m)[K], double *lds) {
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    if (wv < kBlock / kWave)
 #pragma unroll
-    for (int j = 0; j < K; ++j) {
-        const double t = MAX ? wave_max(m[j]) : group_sum<kWave>(m[j]);
-        if (lane == 0) lds[wv * K + j] = t;
-    }
+        for (int j = 0; j < K; ++j) {
+            const double t = MAX ? wave_max(m[j]) : group_sum<kWave>(m[j]);
+            if (lane == 0) lds[wv * K + j] = t;
+        }
     __syncthreads();
     if (threadIdx.x < K) {
         double t = 0.0;
@@ -702,7 +712,8 @@ __device__ __forceinline__ void line_run(const GL float *img, int na, int nb, in
     }
 }
 
-// RESID: r = g - A u (stored), partial sum r^2; else partial sum (A d)^2.
+// RESID: r = g - A u, stored times the ray's length per line (what the back
+// projection weighs), partial sum r^2; else partial sum (A d)^2.
 template <int K, bool RESID>
 __device__ __forceinline__ void line_fp_unit(const EngArgs<float> &a, const UG<float> &U, int s, int lb, double *lds) {
     const int lane = threadIdx.x & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -745,15 +756,17 @@ __device__ __forceinline__ void line_fp_unit(const EngArgs<float> &a, const UG<f
     for (int w = 0; w < kLineWaves; ++w) tot += lds[(w * K + wv) * kLineRays + lane];
     double mm = 0.0;
     if (valid) {
-        tot *= U.ln_len[row];
+        const double len = U.ln_len[row];
+        tot *= len;
         const int dp = U.ln_drop[row];
         if (dp >= 0) {
             const int i = dp / U.ny, j = dp - i * U.ny;
             tot -= (double)U.ln_dlen[row] * (double)U.px[((int64_t)i * line_stride(U.ny) + j + kLinePad) * K + wv];
         }
         if (RESID) {
-            const float o = (float)((double)U.g[row * K + wv] - tot);
-            U.r[row * K + wv] = o;
+            const double res = (double)U.g[row * K + wv] - tot;
+            U.r[row * K + wv] = (float)(res * len);
+            const float o = (float)res;
             mm = (double)o * (double)o;
         } else {
             mm = tot * tot;
@@ -785,10 +798,9 @@ __device__ __forceinline__ int sq_at(int r, int c) { return (r + 1) * kSqW + c +
 
 // L[sq_at(r, c) * K + k] = arr at (i0 + r, j0 + c), `pad` outside the image.
 // Thread (w, lane) stages pixel (tile row w, tile column lane / 32, tile
-// position lane % 32) of the square; threads 0 .. 67 the halo.  Every thread
-// calls it; ends with a barrier.
+// position lane % 32) of the square; threads 0 .. 67 the halo.
 template <typename T, int K>
-__device__ __forceinline__ void stage_square(const UG<T> &U, const GL T *arr, int i0, int j0, T pad, LDSP T *L) {
+__device__ __forceinline__ void put_square(const UG<T> &U, const GL T *arr, int i0, int j0, T pad, LDSP T *L) {
     const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave, w = lane & 31;
     const int r = wv * kTileH + ((w >> 2) & 3), c = (lane >> 5) * kTileW + ((w >> 4) << 2) + (w & 3);
     T x[K];
@@ -804,6 +816,11 @@ __device__ __forceinline__ void stage_square(const UG<T> &U, const GL T *arr, in
 #pragma unroll
         for (int k = 0; k < K; ++k) L[sq_at(hr, hc) * K + k] = x[k];
     }
+}
+// The same; every thread calls it; ends with a barrier.
+template <typename T, int K>
+__device__ __forceinline__ void stage_square(const UG<T> &U, const GL T *arr, int i0, int j0, T pad, LDSP T *L) {
+    put_square<T, K>(U, arr, i0, j0, pad, L);
     __syncthreads();
 }
 
@@ -967,7 +984,6 @@ __device__ __forceinline__ void bp_unit(const EngArgs<T> &a, const UG<T> &U, int
                     dv[k] = (T)d;
                     m[k] = (double)dv[k] * (double)dv[k];
                 }
-                put_proj<T, K>(U, i, j, dv);
             } else {
                 zerok<T, K>(dv);
             }
@@ -975,6 +991,320 @@ __device__ __forceinline__ void bp_unit(const EngArgs<T> &a, const UG<T> &U, int
         }
     }
     block_store<T, K, false>(a, U, SL_DD, lb, m, lds);
+}
+
+// Back projection along the lines (Lines, runtime.hpp), FP32: a lane is a
+// pixel, a workgroup its 16 x 16 block as in bp_unit.  No matrix is read.  Per
+// view the pixel's position on the detector (float) gives the few
+// bins whose rays can meet it, a superset; for each the exact length follows
+// from the ray's line in double,
+//   min(1, max(0, ((1 + |m|) / 2 - |b0 + m a - j - 1/2|) / |m|)),
+// times the residual, which holds the ray's length per line.
+//
+// A block's views come in windows of 64, sorted by axis and by candidates
+// (LineView, prepared with the geometry).  As many views as half of the
+// launch's LDS slots hold, and their rays, are copied there by direct
+// global-to-LDS loads, which run while the lanes work on the other half's
+// views.
+// Where the image has few blocks, 2 or 4 groups of 256 lanes share a block's
+// views (view by view in turn) and their sums are added in order.  The order
+// of a pixel's sum depends on the geometry only, not on K or on the LDS slots.
+//
+// What bounds it: VALU, some 33 instructions a view and pixel (a quarter of the
+// issue slots go to LDS latency at four waves a SIMD).  512 x 512 pixels, 60
+// views: 37.4 us, against 35.4 of the staged matrix form (bp_unit, 179 MB a
+// launch); four jobs 40 against 58 us; 256 x 256, 360 views, one job: 75 us.
+// It needs no matrix at all: an 874 x 874 slice of 576 views is ready in 2 ms
+// (95 ms with the matrix), in 0.2 GB instead of 4.
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+static_assert(sizeof(LineView) == 2 * sizeof(i32x4), "a view is two 16-byte loads");
+
+// Position on the detector of a pixel in units of bins, less bin0.  Flat:
+// (Xk, Yk) = (X, Y) / k and sodk = sod / k.  Arc: X, Y, sod, and the arc
+// tangent of Abramowitz & Stegun 4.4.47 (within 1.2e-5).
+__device__ __forceinline__ float line_bin_flat(float X, float Y, float Xk, float Yk, float c, float s, float sodk) {
+    const float D = __builtin_fmaf(c, Yk, __builtin_fmaf(-s, Xk, sodk));
+    return __builtin_fmaf(s, Y, c * X) * __builtin_amdgcn_rcpf(D);
+}
+__device__ __forceinline__ float line_bin_arc(float X, float Y, float c, float s, float sod, float k) {
+    const float q = __builtin_fmaf(c, Y, -s * X), e = __builtin_fmaf(-s, Y, __builtin_fmaf(-c, X, sod));
+    const float t = q * __builtin_amdgcn_rcpf(e), y = t * t;
+    const float f = __builtin_fmaf(
+        y, __builtin_fmaf(y, __builtin_fmaf(y, __builtin_fmaf(y, .0208351f, -.0851330f), .1801410f), -.3302995f),
+        .9998660f);
+    return -k * t * f;
+}
+
+// One half of the LDS slots: each array holds `cap` of them.
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+template <int K>
+struct LineHalf {
+    const LDSP f64x2 *mb;    // m, b0
+    const LDSP float *inv;   // 1 / |m|
+    const LDSP float *r;     // K residuals
+    const LDSP int32_t *drop;
+};
+constexpr int line_slot_bytes(int K) { return 16 + 4 + 4 * K + 4; }
+
+// What a lane's pixel brings.
+struct LinePix {
+    float X, Y, Xk, Yk, sodk, sod, k;
+    int id;                  // x ny + y
+};
+
+// C candidates of one view (0: `cand` of them, two at a time) added to tot;
+// slot: the first one's, in the half.
+template <int K, bool EDGE, int C>
+__device__ __forceinline__ void line_bp_view(const LineHalf<K> &h, uint32_t slot, int cand, int id, double a, double b,
+                                             double (&tot)[K]) {
+    constexpr int CC = C ? C : 2;
+    for (int q = 0; q < (C ? C : cand); q += CC, slot += CC) {
+        float t[CC];
+#pragma unroll
+        for (int n = 0; n < CC; ++n) {
+            const f64x2 mb = h.mb[slot + n];
+            const double m = mb.x, D = __builtin_fma(m, a, mb.y) - b;
+            const float e = (float)(__builtin_fma(fabs(m), 0.5, 0.5) - fabs(D));
+            t[n] = __builtin_amdgcn_fmed3f(e * h.inv[slot + n], 0.0f, 1.0f);
+            if (EDGE) t[n] = h.drop[slot + n] == id ? 0.0f : t[n];
+        }
+        const LDSP float *r = h.r + slot * K;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            float x = t[0] * r[k];
+#pragma unroll
+            for (int n = 1; n < CC; ++n) x = __builtin_fmaf(t[n], r[n * K + k], x);
+            tot[k] += (double)x;
+        }
+    }
+}
+
+// This group's views k, k + P, ... below k1 of a half, all of one class.  The
+// next view's numbers are read (one address for the wave) while this one's
+// rays are.  off0: the half's first slot in the window.
+template <int K, bool ARC, bool EDGE, int C>
+__device__ __forceinline__ void line_bp_run(const LDSP unsigned char *views, int k, int k1, int P, const LineHalf<K> &h,
+                                            float off0, const LinePix &p, double a, double b, double (&tot)[K]) {
+    auto get = [&](int n, f32x4 &w, float &end, int &meta) {
+        const LDSP unsigned char *v = views + n * (int)sizeof(LineView);
+        w = *(const LDSP f32x4 *)v;   // c, s, lob, first
+        end = *(const LDSP float *)(v + 16);
+        if constexpr (C == 0) meta = *(const LDSP int *)(v + 20);
+    };
+    f32x4 w, nw;
+    float end, nend;
+    int meta = 0, nmeta = 0;
+    get(k, w, end, meta);
+    while (k < k1) {
+        k += P;
+        get(k < k1 ? k : k - P, nw, nend, nmeta);
+        const float u = ARC ? line_bin_arc(p.X, p.Y, w.x, w.y, p.sod, p.k)
+                            : line_bin_flat(p.X, p.Y, p.Xk, p.Yk, w.x, w.y, p.sodk);
+        const uint32_t slot = (uint32_t)(__builtin_amdgcn_fmed3f(u + w.z, w.w, end) - off0);
+        line_bp_view<K, EDGE, C>(h, slot, C ? C : __builtin_amdgcn_readfirstlane(line_cand(meta)), p.id, a, b, tot);
+        w = nw;
+        end = nend;
+        meta = nmeta;
+    }
+}
+
+// d = S A_s^T r + alpha R(u, v) for the block's pixels; partial sum d^2.
+// P groups of 256 lanes; cap: slots of one half.
+template <int K, int P>
+__device__ __forceinline__ void line_bp_unit(const EngArgs<float> &a, const UG<float> &U, int s, int lb, int cap,
+                                             double *lds, LDSP unsigned char *raw) {
+    const int lane = threadIdx.x & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int grp = wv / (kBlock / kWave);   // this wave's group
+    const int tnx = (U.nx + kTileH - 1) / kTileH, nbc = (U.tny + kBpBlockTC - 1) / kBpBlockTC;
+    const int i0 = (lb / nbc) * (kBpBlockTR * kTileH), j0 = (lb % nbc) * (kBpBlockTC * kTileW);
+    const int64_t q = bp_item(lb, wv % (kBlock / kWave), lane, tnx, U.tny);
+    int i = U.nx, j = U.ny;
+    if (q >= 0) tile_coords(q, U.tny, i, j);
+    const bool real = i < U.nx && j < U.ny;
+    // LDS: two halves (each views, mb, inv, r, drop), used again behind the views
+    constexpr int VB = kLineViews * (int)sizeof(LineView);
+    const int half = VB + cap * line_slot_bytes(K);
+    double tot[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) tot[k] = 0.0;
+    if (j0 < U.ny) {   // else: only padding of the tile rows
+        const int64_t row0 = U.sub_row0[s];
+        const int nv = (int)((U.sub_row0[s + 1] - row0) / U.nbins);
+        const int64_t nblk = bp_blocks_of(tnx, U.tny);
+        const int nwin = (nv + kLineViews - 1) / kLineViews;
+        const bool edge = i0 == 0 || j0 == 0 || i0 + 16 >= U.nx || j0 + 16 >= U.ny;
+        LinePix p;
+        p.X = (i + 0.5f - 0.5f * U.nx) * U.ln_pix;
+        p.Y = (j + 0.5f - 0.5f * U.ny) * U.ln_pix;
+        p.k = U.ln_k;
+        p.sod = U.ln_sod;
+        p.Xk = p.X / p.k;
+        p.Yk = p.Y / p.k;
+        p.sodk = p.sod / p.k;
+        p.id = i * U.ny + j;
+        const double id = i, jd = j;
+
+        // A window: lane l holds view l (its second half: end, meta, src, row;
+        // and first), and the views up to the end of each class.
+        struct Window {
+            const GL char *tab;   // its views
+            i32x4 b;
+            float first;
+            int n;
+        };
+        auto load = [&](int w) {
+            Window W;
+            W.tab = (const GL char *)U.ln_views + ((U.ln_win0[s] + w) * nblk + lb) * VB;
+            W.n = min(kLineViews, nv - w * kLineViews);
+            W.b = i32x4{0, 0, 0, 0};
+            W.first = 0.0f;
+            if (lane < W.n) {
+                W.b = *(const GL i32x4 *)(W.tab + lane * sizeof(LineView) + 16);
+                W.first = *(const GL float *)(W.tab + lane * sizeof(LineView) + 12);
+            }
+            return W;
+        };
+        auto fit = [&](const Window &W, int off) {   // as many views as a half holds (the slots' ends only grow)
+            return (int)__popcll(__ballot(lane < W.n && line_stop(W.b.y) - off <= cap));
+        };
+        // copies views k0 .. k1 - 1 of a window and their rays to a half
+        auto copy = [&](const Window &W, int k0, int k1, int off0, LDSP unsigned char *to) {
+            if (wv == 0)
+                for (int e = lane; e < (k1 - k0) * 2; e += kWave)
+                    __builtin_amdgcn_global_load_lds((const GL void *)(W.tab + k0 * sizeof(LineView) + e * 16u),
+                                                     (LDSP void *)(to + (e - lane) * 16), 16, 0, 0);
+            to += VB;
+            for (int k = k0 + wv; k < k1; k += P * (kBlock / kWave)) {
+                const int first = (int)__uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(W.first), k));
+                const int meta = __builtin_amdgcn_readlane(W.b.y, k);
+                const int n = line_stop(meta) - first, at = first - off0;
+                const int64_t src = __builtin_amdgcn_readlane(W.b.z, k) + first;
+                const int64_t row = row0 + __builtin_amdgcn_readlane(W.b.w, k) + first;
+                const bool yd = line_axis(meta);
+                const GL char *mb = (const GL char *)(yd ? U.ln_my : U.ln_mx) + src * 16;
+                const GL char *iv = (const GL char *)(yd ? U.ln_iy : U.ln_ix) + src * 4;
+                const GL char *rr = (const GL char *)U.r + row * (4 * K), *dr = (const GL char *)U.ln_drop + row * 4;
+                LDSP unsigned char *o = to + at * 16;
+                for (int e = lane; e < n; e += kWave)
+                    __builtin_amdgcn_global_load_lds((const GL void *)(mb + e * 16u), (LDSP void *)(o + (e - lane) * 16), 16,
+                                                     0, 0);
+                o = to + cap * 16 + at * 4;
+                for (int e = lane; e < n; e += kWave)
+                    __builtin_amdgcn_global_load_lds((const GL void *)(iv + e * 4u), (LDSP void *)(o + (e - lane) * 4), 4, 0,
+                                                     0);
+                o = to + cap * 20 + at * (4 * K);
+                for (int e = lane; e < n * K; e += kWave)
+                    __builtin_amdgcn_global_load_lds((const GL void *)(rr + e * 4u), (LDSP void *)(o + (e - lane) * 4), 4, 0,
+                                                     0);
+                if (edge) {
+                    o = to + cap * (20 + 4 * K) + at * 4;
+                    for (int e = lane; e < n; e += kWave)
+                        __builtin_amdgcn_global_load_lds((const GL void *)(dr + e * 4u), (LDSP void *)(o + (e - lane) * 4),
+                                                         4, 0, 0);
+                }
+            }
+        };
+        // The round at hand: views k0 .. k1 - 1 of window w, slots from off0;
+        // W: the window of the round behind it, N: the window behind W.
+        int w = 0, k0 = 0, off0 = 0, par = 0;
+        Window W = load(0), N = load(nwin > 1 ? 1 : 0);
+        int k1 = fit(W, 0);
+        copy(W, k0, k1, off0, raw);
+        while (w < nwin) {
+            // the classes of this round's views: along x with 2, 3, more candidates, along y likewise
+            int upto[6];
+            const int cls = line_class(W.b.y);
+#pragma unroll
+            for (int c = 0; c < 6; ++c)
+                upto[c] = min(k1, (int)__popcll(__ballot(lane < W.n && cls <= c)));
+            int nw = w, nk0 = k1, noff = line_stop(__builtin_amdgcn_readlane(W.b.y, k1 - 1)), nk1 = 0;
+            if (nk0 >= W.n) {
+                ++nw;
+                nk0 = noff = 0;
+                W = N;
+                if (nw + 1 < nwin) N = load(nw + 1);
+            }
+            if (nw < nwin) nk1 = fit(W, noff);
+            __builtin_amdgcn_s_waitcnt(0);   // this round's copies have landed
+            __syncthreads();                 // ... everybody's, and the other half is free
+            if (nw < nwin) copy(W, nk0, nk1, noff, raw + (par ^ 1) * half);
+            const LDSP unsigned char *vt = raw + par * half, *b = vt + VB;
+            vt -= k0 * (int)sizeof(LineView);
+            const LineHalf<K> h{(const LDSP f64x2 *)b, (const LDSP float *)(b + cap * 16), (const LDSP float *)(b + cap * 20),
+                                (const LDSP int32_t *)(b + cap * (20 + 4 * K))};
+            auto run = [&](auto arc, auto ed) {
+                auto one = [&](auto c, int e) {
+                    constexpr int C = decltype(c)::value;
+                    const int c0 = max(k0, e ? upto[e - 1] : 0);
+                    const int k = c0 + (grp - c0 % P + P) % P;   // the window's views go to the groups in turn
+                    if (k < upto[e])
+                        line_bp_run<K, decltype(arc)::value, decltype(ed)::value, C>(
+                            vt, k, upto[e], P, h, (float)off0, p, e < 3 ? id : jd, (e < 3 ? jd : id) + 0.5, tot);
+                };
+                using std::integral_constant;
+#pragma unroll
+                for (int e = 0; e < 6; e += 3) {
+                    one(integral_constant<int, 2>{}, e);
+                    one(integral_constant<int, 3>{}, e + 1);
+                    one(integral_constant<int, 0>{}, e + 2);
+                }
+            };
+            if (U.ln_arc) {
+                if (edge) run(std::true_type{}, std::true_type{});
+                else run(std::true_type{}, std::false_type{});
+            } else {
+                if (edge) run(std::false_type{}, std::true_type{});
+                else run(std::false_type{}, std::false_type{});
+            }
+            w = nw;
+            k0 = nk0;
+            k1 = nk1;
+            off0 = noff;
+            par ^= 1;
+        }
+        __syncthreads();   // the slots' LDS is used again
+    }
+    if constexpr (P > 1) {   // the groups' sums, in order
+        LDSP double *part = (LDSP double *)raw;
+        if (grp > 0)
+#pragma unroll
+            for (int k = 0; k < K; ++k) part[((grp - 1) * K + k) * kBlock + threadIdx.x % kBlock] = tot[k];
+        __syncthreads();
+        if (grp == 0)
+#pragma unroll
+            for (int g = 1; g < P; ++g)
+#pragma unroll
+                for (int k = 0; k < K; ++k) tot[k] += part[((g - 1) * K + k) * kBlock + threadIdx.x];
+        __syncthreads();
+    }
+    LDSP float *Lu = (LDSP float *)raw, *Lv = Lu + kSqN * K;
+    if (grp == 0) {
+        put_square<float, K>(U, U.u, i0, j0, 0.0f, Lu);
+        put_square<float, K>(U, U.v, i0, j0, 1.0f, Lv);
+    }
+    __syncthreads();
+    double m[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) m[k] = 0.0;
+    if (grp == 0 && q >= 0) {
+        float dv[K];
+        zerok<float, K>(dv);
+        if (real) {
+            double eps[K], reg[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) eps[k] = jpar(a, U.job0 + k).eps;
+            gc_reg<float, K>(Lu, Lv, i - i0, j - j0, eps, reg);
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                dv[k] = (float)((double)a.S * tot[k] + jpar(a, U.job0 + k).alpha * reg[k]);
+                m[k] = (double)dv[k] * (double)dv[k];
+            }
+            put_proj<float, K>(U, i, j, dv);
+        }
+        storek<float, K>(U.d + q * K, dv);
+    }
+    block_store<float, K, false>(a, U, SL_DD, lb, m, lds);
 }
 
 // Stencil kernels: one thread per tiled position q (256 per block); the
@@ -1320,6 +1650,19 @@ __global__ __launch_bounds__(kLineBlock) void k_line_fp(EngArgs<float> a, BlockM
     if (unit_idle(a, U)) return;
     const int lb = b - m.start[ui];
     MI_KSWITCH(KMAX, (line_fp_unit<K, RESID>(a, U, s, lb, lds)))
+}
+
+template <int KMAX, int P>
+__global__ __launch_bounds__(P * kBlock) void k_line_bp(EngArgs<float> a, BlockMap m, int s, int cap) {
+    __shared__ double lds[kBlock / kWave * kMaxK];
+    extern __shared__ __align__(16) unsigned char ldr_raw[];
+    const int b = (int)xcd_block();
+    if (b >= m.start[m.nunits]) return;
+    const int ui = find_unit(m, b);
+    const UG<float> U(a.units[ui]);
+    if (unit_idle(a, U)) return;
+    const int lb = b - m.start[ui];
+    MI_KSWITCH(KMAX, (line_bp_unit<K, P>(a, U, s, lb, cap, lds, (LDSP unsigned char *)ldr_raw)))
 }
 
 template <typename T, int KMAX, bool LDS, bool SQ>
@@ -1673,6 +2016,37 @@ void eng_line_fp(hipStream_t st, const EngArgs<float> &a, const BlockMap &m, int
         else if (kmax <= 4) launch(k_line_fp<4, false>, grid, block, 0u, st, a, m, s);
         else launch(k_line_fp<kMaxK, false>, grid, block, 0u, st, a, m, s);
     }
+    MI_HIP(hipGetLastError());
+}
+
+// LDS slots of a half: fewer rounds with more of them, so the workgroups that
+// a CU gets share its LDS, up to six of them (874 x 874, 72 views: 97.9 us; four
+// 109.4, eight 99.6).
+constexpr int kLineResident = 6;
+template <int KM, int P>
+static void line_bp_launch(hipStream_t st, const EngArgs<float> &a, const BlockMap &m, int s) {
+    const int blocks = m.start[m.nunits];
+    constexpr int per = 2 * line_slot_bytes(KM), fix = 2 * kLineViews * (int)sizeof(LineView);
+    const int res = std::min(kLineResident, (blocks + 255) / 256);
+    const int lim = (int)std::min<size_t>(kBpLdsLaunch, ((size_t)160 << 10) / res - 1024);
+    const int cap = std::max(kLineSlots, std::min(1024, (lim - fix) / per & ~3));
+    const size_t lds = std::max({(size_t)cap * per + fix, (size_t)2 * kSqN * KM * sizeof(float),
+                                 (size_t)(P - 1) * KM * kBlock * sizeof(double)});
+    launch(k_line_bp<KM, P>, dim3(grid8(blocks)), dim3(P * kBlock), (uint32_t)lds, st, a, m, s, cap);
+}
+static_assert(kLineSlots * 2 * line_slot_bytes(kMaxK) + 2 * kLineViews * sizeof(LineView) <= kBpLdsLaunch,
+              "the slots of eight jobs fit a launch");
+
+void eng_line_bp(hipStream_t st, const EngArgs<float> &a, const BlockMap &m, int s, int kmax, int groups) {
+    auto go = [&](auto km) {
+        constexpr int KM = decltype(km)::value;
+        if (groups == 4) line_bp_launch<KM, 4>(st, a, m, s);
+        else if (groups == 2) line_bp_launch<KM, 2>(st, a, m, s);
+        else line_bp_launch<KM, 1>(st, a, m, s);
+    };
+    if (kmax == 1) go(std::integral_constant<int, 1>{});
+    else if (kmax <= 4) go(std::integral_constant<int, 4>{});
+    else go(std::integral_constant<int, kMaxK>{});
     MI_HIP(hipGetLastError());
 }
 

@@ -166,11 +166,34 @@ struct Otf {
 // Rows are the matrix's (subset order); a group is kLineRays consecutive bins
 // of one view, ceil(n_bins / kLineRays) groups per view.
 constexpr int kLineRays = kWave;
+constexpr int kLineSlots = 320;  // rays of one view that may meet a 16 x 16 pixel block (half of a launch's LDS slots)
 constexpr int kLinePad = 2;      // zero pixels on each side of a projection image's line
 constexpr int kLineRows = 8;     // zero lines behind its last one
 __host__ __device__ __forceinline__ int64_t line_stride(int n) { return n + 2 * kLinePad; }
 __host__ __device__ __forceinline__ int64_t line_elems(int na, int nb) {
     return (int64_t)(na + kLineRows) * line_stride(nb);
+}
+constexpr int kLineEmpty = 8;    // empty entries behind a view's bins: the most candidates a pixel may have
+constexpr int kLineViews = kWave;   // views of a back-projection window
+// One view of a 16 x 16 pixel block.  Its slots are the window's from `first`:
+// the rays that can meet the block, from `end` on as many more as a pixel has
+// candidates (they meet none of its pixels).
+struct LineView {
+    float c, s;          // the view's cos and sin
+    float lob;           // slot of position 0 on the detector, less the half width of a pixel's shadow, plus 1
+    float first, end;
+    int32_t meta;        // slot behind its last, candidates of a pixel (2, 3 or even), axis its lines are taken along (1: y)
+    int32_t src, row;    // entry of slot 0 in mx .. iy; residual row of slot 0 (of the subset)
+};
+__host__ __device__ __forceinline__ int line_meta(int stop, int cand, int axis) { return stop | cand << 20 | axis << 24; }
+__host__ __device__ __forceinline__ int line_stop(int meta) { return meta & 0xfffff; }
+__host__ __device__ __forceinline__ int line_cand(int meta) { return meta >> 20 & 15; }
+__host__ __device__ __forceinline__ int line_axis(int meta) { return meta >> 24 & 1; }
+// A window's views are sorted by class: along x with 2, 3 and more candidates,
+// along y likewise.
+__host__ __device__ __forceinline__ int line_class(int meta) {
+    const int c = line_cand(meta);
+    return 3 * line_axis(meta) + (c < 4 ? c - 2 : 2);
 }
 struct Lines {
     std::vector<int64_t> slice0;     // S + 1: 4 x the first group of each subset (a group is one workgroup)
@@ -181,8 +204,25 @@ struct Lines {
     DevBuf<int32_t> drop;            // per row: pixel (x ny + y) whose piece is left out, -1: none
     DevBuf<float> dlen;              // per row: its length
     DevBuf<int4> rng;                // per group: lines its x-dominant rays cross [x, y), its y-dominant ones [z, w)
+    // Back projection.  The lines along x and along y of every ray (a ray far
+    // from that axis, or past the view's last bin: weight 0 everywhere), views
+    // kLineEmpty entries longer than their bins; 1 / min(1, |m|).
+    DevBuf<double2> mx, my;
+    DevBuf<float> ix, iy;
+    // Where a pixel's rays lie: with (X, Y) the pixel's centre from the image
+    // centre (mm) and (c, s) the view's cos and sin,
+    //   flat: bin k (c X + s Y) / (sod - s X + c Y) + bin0, k = sdd / bin_mm
+    //   arc:  bin -k atan((c Y - s X) / (sod - c X - s Y)) + bin0, k = 1 / (radians per bin)
+    // and, per block and window of kLineViews views, the views by line_class:
+    // window w of subset s and block b at ((win0[s] + w) nblk + b) kLineViews.
+    std::vector<int64_t> win0;
+    DevBuf<int64_t> d_win0;
+    DevBuf<LineView> views;
+    int arc = 0;
+    float sod = 0.f, k = 0.f, bin0 = 0.f;
     size_t bytes() const {
-        return d_slice0.bytes() + mb.bytes() + len.bytes() + inv.bytes() + drop.bytes() + dlen.bytes() + rng.bytes();
+        return d_slice0.bytes() + mb.bytes() + len.bytes() + inv.bytes() + drop.bytes() + dlen.bytes() + rng.bytes() +
+               mx.bytes() + my.bytes() + ix.bytes() + iy.bytes() + d_win0.bytes() + views.bytes();
     }
 };
 
@@ -197,6 +237,8 @@ __host__ __device__ __forceinline__ int64_t sell_pos(int64_t base, int t, int la
 // (j & 3)), so each 64-byte half line is a square.
 constexpr int kTileH = 4, kTileW = 8;
 constexpr int kStripTiles = 8;   // tiles of a stencil strip; each tile row holds a multiple of it
+// Tiles of a tile row of images ny wide.
+inline int tiled_ny(int ny) { return (ny + kStripTiles * kTileW - 1) / (kStripTiles * kTileW) * kStripTiles; }
 __host__ __device__ __forceinline__ int64_t tile_index(int i, int j, int tny) {
     return ((int64_t)(i >> 2) * tny + (j >> 3)) * (kTileH * kTileW) + (((j >> 2) & 1) << 4) + ((i & 3) << 2) +
            (j & 3);

@@ -346,11 +346,11 @@ void build_sell(Matrix &m, hipStream_t st, bool drop_csr) {
     const mi_geometry &g = m.g;
     // tile rows padded to a multiple of 8 tiles: a stencil block (8 tiles) is
     // then a 4 x 64 pixel strip of one tile row
-    m.tny = (g.ny + kStripTiles * kTileW - 1) / (kStripTiles * kTileW) * kStripTiles;
+    m.tny = tiled_ny(g.ny);
     m.npix_t = (int64_t)((g.nx + kTileH - 1) / kTileH) * kTileH * m.tny * kTileW;
     const bool f64 = m.has64;
     // forward
-    if (!m.has_otf && !m.has_lines) {   // the lines or the checkpointed walk replace the stored forward slices
+    if (m.has_csr && !m.has_otf) {   // the checkpointed walk replaces the stored forward slices
         m.fs.P = choose_p(MI_SELL_PF, (double)m.nnz / std::max<int64_t>(m.nrows, 1));
         m.fs.C = kWave / m.fs.P;
         m.fs.slice0.assign(m.S + 1, 0);
@@ -373,6 +373,14 @@ void build_sell(Matrix &m, hipStream_t st, bool drop_csr) {
     const int64_t nblk = bp_blocks_of(tnx, m.tny), per = nblk * 4;
     m.bs.slice0.assign(m.S + 1, 0);
     for (int s = 0; s < m.S; ++s) m.bs.slice0[s + 1] = m.bs.slice0[s] + per;
+    if (!m.has_csr) {   // lines only: the blocks without a matrix
+        m.bs.d_slice0.alloc(m.bs.slice0.size());
+        MI_HIP(hipMemcpyAsync(m.bs.d_slice0.p, m.bs.slice0.data(), m.bs.slice0.size() * sizeof(int64_t),
+                              hipMemcpyHostToDevice, st));
+        MI_HIP(hipStreamSynchronize(st));
+        m.has_sell = true;
+        return;
+    }
     BItems bi{m.colptr.p, nullptr, m.S, m.bs.P, m.bs.C, g.nx, g.ny, tnx, m.tny, m.npix, m.npix_t};
     fill_sell(m.bs, bi, m.crow.p, m.clen32.p, f64 ? m.clen64.p : nullptr, false, g.ny, m.tny, st);
     bi.slice0 = m.bs.d_slice0.p;

@@ -392,12 +392,14 @@ void build_otf(Matrix &m, const TraceArgs &a, hipStream_t st) {
 // image.  Rays the tracer treats as parallel to an axis (|r| <= 1e-4 mm across
 // it) stay in their first pixel's line, as its 1e6 sentinel keeps them.
 struct LineOut {
-    double2 *mb;
+    double2 *mb, *mx, *my;
+    float *ix, *iy;
     double *len;
     float *inv, *dlen;
     int32_t *drop;
     int4 *rng;
     unsigned *bad;
+    unsigned long long *nnz;   // per subset: the tracer's entries
 };
 __global__ __launch_bounds__(kLineRays) void k_lines_fill(TraceArgs a, const int64_t *sub_row0, const int64_t *slice0,
                                                           int S, LineOut o) {
@@ -410,6 +412,7 @@ __global__ __launch_bounds__(kLineRays) void k_lines_fill(TraceArgs a, const int
     const int64_t row = sub_row0[s] + lg / per * a.nbins + bin;
     const FanGeom &g = a.fan;
     int r0 = INT32_MAX, r1 = 0;   // lines crossed
+    unsigned pieces = 0;
     bool yd = false, bad = false;
     if (bin < a.nbins) {
         const int view = a.vlist[row / a.nbins];
@@ -448,6 +451,7 @@ __global__ __launch_bounds__(kLineRays) void k_lines_fill(TraceArgs a, const int
                 int cx, cy;
                 double w;
                 siddon_step(st, cx, cy, w);
+                ++pieces;
                 bad |= !(fabs(w - length(cx, cy)) <= 1e-5 * v);
             }
             const double rem = st.hi - st.lam;
@@ -470,6 +474,17 @@ __global__ __launch_bounds__(kLineRays) void k_lines_fill(TraceArgs a, const int
         o.inv[row] = yd ? -(float)inv : (float)inv;
         o.drop[row] = drop;
         o.dlen[row] = dlen;
+        // Both lines.  Turned, m -> 1 / m: the length in a pixel stays len times
+        // min(1, max(0, ((1 + |m|) / 2 - |..|) / min(1, |m|))) with |m| > 1.  Only
+        // rays near the diagonal are looked at along their other axis.
+        const int64_t e = row / a.nbins * (a.nbins + kLineEmpty) + bin;
+        const bool near = fabs(m) > 0.25;
+        const double2 own = make_double2(m, b0), no = make_double2(0.0, -64.0);
+        const double2 other = near ? make_double2(1.0 / m, 0.5 + (0.5 - b0) / m) : no;
+        o.mx[e] = yd ? other : own;
+        o.my[e] = yd ? own : other;
+        o.ix[e] = yd ? (near ? 1.0f : 0.0f) : (float)inv;
+        o.iy[e] = yd ? (float)inv : (near ? 1.0f : 0.0f);
     }
     int x0 = yd ? INT32_MAX : r0, x1 = yd ? 0 : r1, y0 = yd ? r0 : INT32_MAX, y1 = yd ? r1 : 0;
     for (int w = kWave / 2; w > 0; w >>= 1) {
@@ -477,39 +492,189 @@ __global__ __launch_bounds__(kLineRays) void k_lines_fill(TraceArgs a, const int
         x1 = max(x1, __shfl_xor(x1, w, kWave));
         y0 = min(y0, __shfl_xor(y0, w, kWave));
         y1 = max(y1, __shfl_xor(y1, w, kWave));
+        pieces += __shfl_xor(pieces, w, kWave);
     }
+    if (lane == 0) atomicAdd(o.nnz + s, (unsigned long long)pieces);
     if (lane == 0) o.rng[grp] = make_int4(min(x0, x1), x1, min(y0, y1), y1);
     if (__any(bad) && lane == 0) atomicOr(o.bad, 1u);
 }
 
+// A view (cos c, sin s) for the block at pixel (i0, j0): its first bin and bin
+// count there, the half width of a pixel's shadow in bins, the dominant axis
+// at the block's centre.
+struct LineGeo {
+    int nx, ny, nbins, arc;
+    float pix, sod, k, bin0;
+};
+__device__ __forceinline__ void line_view(const LineGeo &g, float c, float s, int i0, int j0, int &b0, int &cnt, float &hw,
+                                          int &axis) {
+    const float p = g.pix, sod = g.sod, k = g.k;
+    const float X0 = (i0 - 0.5f * g.nx) * p, Y0 = (j0 - 0.5f * g.ny) * p;
+    // the block's corners: extremes of the position (a monotonic function of
+    // a ratio of linear ones) and of the two parts of a pixel's half shadow
+    float lo = 1e30f, hi = -1e30f, ax = 0.f, ay = 0.f, rn = 0.f;
+    for (int q = 0; q < 4; ++q) {
+        const float X = X0 + (q & 1) * 16 * p, Y = Y0 + (q >> 1) * 16 * p;
+        if (g.arc) {
+            const float y = c * Y - s * X, e = sod - c * X - s * Y, u = -k * atanf(y / e);
+            lo = fminf(lo, u);
+            hi = fmaxf(hi, u);
+            ax = fmaxf(ax, fabsf(y * c - e * s) * k);
+            ay = fmaxf(ay, fabsf(y * s + e * c) * k);
+            rn = fmaxf(rn, 1.0f / (y * y + e * e));
+        } else {
+            const float rD = 1.0f / (sod - s * X + c * Y), u = (c * X + s * Y) * k * rD;
+            lo = fminf(lo, u);
+            hi = fmaxf(hi, u);
+            ax = fmaxf(ax, fabsf(c * k + s * u));
+            ay = fmaxf(ay, fabsf(s * k - c * u));
+            rn = fmaxf(rn, rD);
+        }
+    }
+    // first order in the pixel; the arc's least distance may lie between the
+    // corners; the float rounding, and the arc tangent's error on the arc
+    const float step = g.arc ? sqrtf(rn) * p : rn * p;
+    const float near = g.arc ? 1.0f + 256.0f * step * step : 1.0f;
+    hw = 0.5f * p * (ax + ay) * rn * near * (1.0f + 2.0f * step) + 0.01f + (g.arc ? 1.2e-5f * k : 0.0f);
+    b0 = max(0, (int)ceilf(lo + g.bin0 - hw - 0.01f));
+    cnt = max(0, min(g.nbins - 1, (int)floorf(hi + g.bin0 + hw + 1.01f)) - b0 + 1);
+    b0 = min(b0, g.nbins);
+    const float Xc = X0 + 8 * p, Yc = Y0 + 8 * p;
+    axis = g.arc ? fabsf(Yc - sod * s) > fabsf(Xc - sod * c) : fabsf(Yc + sod * c) > fabsf(Xc - sod * s);
+}
+
+// One wave per (window of views, block), lane = view.  *most: the largest slot
+// count of a view; candidates above kLineEmpty count as a view that does not
+// fit.
+__global__ __launch_bounds__(kLineViews) void k_line_windows(LineGeo g, int tnx, int tny, int64_t nblk, const double *fcos,
+                                                             const double *fsin, const int *vlist,
+                                                             const int64_t *sub_row0, const int64_t *win0, int S,
+                                                             LineView *views, int *most) {
+    const int64_t at = blockIdx.x;   // window * nblk + block
+    const int64_t win = at / nblk;
+    const int lb = (int)(at % nblk), lane = threadIdx.x;
+    int s = 0;
+    while (s + 1 < S && win0[s + 1] <= win) ++s;
+    const int64_t row0 = sub_row0[s];
+    const int nv = (int)((sub_row0[s + 1] - row0) / g.nbins), vs = (int)(row0 / g.nbins);
+    const int v = (int)(win - win0[s]) * kLineViews + lane;   // view of the subset
+    const int nbc = (tny + kBpBlockTC - 1) / kBpBlockTC;
+    const int i0 = (lb / nbc) * (kBpBlockTR * kTileH), j0 = (lb % nbc) * (kBpBlockTC * kTileW);
+    const bool in = v < nv;
+    int b0 = 0, cnt = 0, axis = 0;
+    float hw = 0.0f, c = 1.0f, sn = 0.0f;
+    if (in) {
+        c = (float)fcos[vlist[vs + v]];
+        sn = (float)fsin[vlist[vs + v]];
+        line_view(g, c, sn, i0, j0, b0, cnt, hw, axis);
+    }
+    // an interval of 2 hw holds at most floor(2 hw) + 1 bins
+    int cand = min(15, max(2, (int)floorf(2.0f * hw) + 1));
+    if (cand > 3) cand = (cand + 1) & ~1;
+    // sorted by class; slots in that order: sizes pushed to their place,
+    // summed, pulled back
+    const int cls = in ? line_class(line_meta(0, cand, axis)) : 6;
+    int pos = lane, before = 0;
+    for (int k = 0; k < 7; ++k) {
+        const uint64_t mk = __ballot(cls == k);
+        if (cls == k) pos = before + __popcll(mk & (((uint64_t)1 << lane) - 1));
+        before += __popcll(mk);
+    }
+    const int size = in ? cnt + cand : 0;
+    int upto = __builtin_amdgcn_ds_permute(4 * pos, size);
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int x = __shfl_up(upto, o, kWave);
+        if (lane >= o) upto += x;
+    }
+    const int off = __shfl(upto, pos, kWave) - size;
+    if (in) {
+        LineView w;
+        w.c = c;
+        w.s = sn;
+        w.lob = g.bin0 - hw + 1.0f + (float)(off - b0);   // + 1: the conversion to a slot rounds down
+        w.first = (float)off;
+        w.end = (float)(off + cnt);
+        w.meta = line_meta(off + size, cand, axis);
+        w.src = (vs + v) * (g.nbins + kLineEmpty) + b0 - off;
+        w.row = v * g.nbins + b0 - off;
+        views[at * kLineViews + pos] = w;
+        if (i0 < g.nx && j0 < g.ny) atomicMax(most, cand > kLineEmpty ? INT32_MAX : size);
+    }
+}
+
 // The line form of every ray; false (and nothing kept) when the geometry has
-// a ray without it, or an image beyond the 32-bit offsets of the kernels.
-bool build_lines(Matrix &m, const TraceArgs &a, hipStream_t st) {
+// a ray without it, an image or sinogram beyond the kernels' 32-bit offsets, a
+// source too near (for the arc: the 45 degrees of its arc tangent), or bins so
+// fine that the rays of one view through a 16 x 16 pixel block do not fit the
+// back projection's LDS slots.
+bool try_lines(Matrix &m, const TraceArgs &a, hipStream_t st) {
     const mi_geometry &g = m.g;
     if (!(g.pixel_mm > 0.0501) || (int64_t)(g.nx + 64) * (g.ny + 64) >= (int64_t)1 << 26) return false;
     Lines &q = m.lines;
+    q.arc = g.beam == MI_BEAM_FAN_ARC;
+    q.sod = (float)g.sod_mm;
+    q.k = (float)(q.arc ? 180.0 / (M_PI * g.bin_mm) : g.sdd_mm / g.bin_mm);
+    q.bin0 = (float)(q.arc ? g.n_bins / 2 - g.det_offset : g.n_bins / 2 - 0.5 - g.det_offset);
+    // every corner of a block, also one that reaches past the image, lies in
+    // front of the source
+    const double rad = 0.5 * g.pixel_mm * std::hypot((double)g.nx, (double)g.ny), blk = 16 * M_SQRT2 * g.pixel_mm;
+    if (!(g.sod_mm - rad - blk > 0.02 * g.sod_mm)) return false;
+    if (m.nrows + (int64_t)g.n_views * kLineEmpty >= (int64_t)1 << 30) return false;
+    if (q.arc && !(1.42 * (rad + g.pixel_mm) < g.sod_mm)) return false;
     const int64_t per = (g.n_bins + kLineRays - 1) / kLineRays;
     q.slice0.assign(m.S + 1, 0);
     for (int s = 0; s < m.S; ++s) q.slice0[s + 1] = q.slice0[s] + 4 * per * ((m.sub_row0[s + 1] - m.sub_row0[s]) / g.n_bins);
     const int64_t groups = q.slice0.back() / 4;
     upload(q.d_slice0, q.slice0, st);
+    const int64_t entries = (int64_t)g.n_views * (g.n_bins + kLineEmpty);
     q.mb.alloc(m.nrows);
     q.len.alloc(m.nrows);
     q.inv.alloc(m.nrows);
-    q.drop.alloc(m.nrows);
+    q.drop.alloc(m.nrows + kLineEmpty);   // read past a view's last bin
     q.dlen.alloc(m.nrows);
     q.rng.alloc(groups);
-    DevBuf<unsigned> bad(1);
-    MI_HIP(hipMemsetAsync(bad.p, 0, sizeof(unsigned), st));
-    const LineOut o{q.mb.p, q.len.p, q.inv.p, q.dlen.p, q.drop.p, q.rng.p, bad.p};
+    for (auto *b : {&q.mx, &q.my}) b->alloc(entries);
+    for (auto *b : {&q.ix, &q.iy}) b->alloc(entries);
+    MI_HIP(hipMemsetAsync(q.drop.p, 0xff, q.drop.bytes(), st));
+    // the empty entries: any finite line with weight 0
+    for (auto *b : {&q.mx, &q.my}) MI_HIP(hipMemsetAsync(b->p, 0, b->bytes(), st));
+    for (auto *b : {&q.ix, &q.iy}) MI_HIP(hipMemsetAsync(b->p, 0, b->bytes(), st));
+    q.win0.assign(m.S + 1, 0);
+    for (int s = 0; s < m.S; ++s)
+        q.win0[s + 1] = q.win0[s] + ((m.sub_row0[s + 1] - m.sub_row0[s]) / g.n_bins + kLineViews - 1) / kLineViews;
+    upload(q.d_win0, q.win0, st);
+    const int tnx = (g.nx + kTileH - 1) / kTileH, tny = tiled_ny(g.ny);
+    const int64_t nblk = bp_blocks_of(tnx, tny), wins = q.win0.back() * nblk;
+    if (wins >= INT32_MAX / 8) return false;
+    q.views.alloc(wins * kLineViews);
+    DevBuf<int> flags(2);   // a ray without the form; the largest slot count
+    MI_HIP(hipMemsetAsync(flags.p, 0, flags.bytes(), st));
+    MI_HIP(hipMemsetAsync(q.views.p, 0, q.views.bytes(), st));
+    DevBuf<unsigned long long> nnz(m.S);
+    MI_HIP(hipMemsetAsync(nnz.p, 0, nnz.bytes(), st));
+    const LineOut o{q.mb.p, q.mx.p, q.my.p, q.ix.p, q.iy.p, q.len.p, q.inv.p, q.dlen.p, q.drop.p, q.rng.p,
+                    (unsigned *)flags.p, nnz.p};
     k_lines_fill<<<(unsigned)groups, kLineRays, 0, st>>>(a, m.d_sub_row0.p, q.d_slice0.p, m.S, o);
     MI_HIP(hipGetLastError());
-    unsigned h = 0;
-    MI_HIP(hipMemcpyAsync(&h, bad.p, sizeof(h), hipMemcpyDeviceToHost, st));
+    const LineGeo lg{g.nx, g.ny, g.n_bins, q.arc, (float)g.pixel_mm, q.sod, q.k, q.bin0};
+    k_line_windows<<<(unsigned)wins, kLineViews, 0, st>>>(lg, tnx, tny, nblk, a.fcos, a.fsin, a.vlist, m.d_sub_row0.p,
+                                                         q.d_win0.p, m.S, q.views.p, flags.p + 1);
+    MI_HIP(hipGetLastError());
+    int h[2] = {0, 0};
+    std::vector<unsigned long long> n(m.S);
+    MI_HIP(hipMemcpyAsync(h, flags.p, sizeof(h), hipMemcpyDeviceToHost, st));
+    MI_HIP(hipMemcpyAsync(n.data(), nnz.p, nnz.bytes(), hipMemcpyDeviceToHost, st));
     MI_HIP(hipStreamSynchronize(st));
-    m.has_lines = h == 0;
-    if (!m.has_lines) m.lines = Lines{};
-    return m.has_lines;
+    if (h[0] != 0 || h[1] > kLineSlots) return false;
+    m.sub_nnz.assign(n.begin(), n.end());
+    m.nnz = std::accumulate(m.sub_nnz.begin(), m.sub_nnz.end(), (int64_t)0);
+    return m.has_lines = true;
+}
+
+bool build_lines(Matrix &m, const TraceArgs &a, hipStream_t st) {
+    if (try_lines(m, a, st)) return true;
+    m.lines = Lines{};
+    return false;
 }
 
 // Entries of each subset's rows, from the device row pointer.
@@ -665,6 +830,14 @@ std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, h
         a.psin = psin.p;
     }
 
+    // FP32 engine runs of a fan beam project along the lines and need no
+    // matrix; FP64 runs, and geometries with a ray that has no line form, re-run
+    // the tracer from checkpoints and read the matrix.
+    const bool fan = g.beam == MI_BEAM_FAN_FLAT || g.beam == MI_BEAM_FAN_ARC;
+    if (otf && fan && build_lines(*m, a, st) && !want64) {
+        m->has_csr = false;
+        return m;
+    }
     m->rowptr.alloc(m->nrows + 1);
     MI_HIP(hipMemsetAsync(m->rowptr.p, 0, sizeof(int64_t), st));
     k_trace_count<<<grid_of(m->nrows, 64), 64, 0, st>>>(a, m->nrows, m->rowptr.p);
@@ -679,11 +852,7 @@ std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, h
     MI_HIP(hipGetLastError());
     build_csc(*m, m->rowptr.p, m->idx.p, m->len32.p, want64 ? m->len64.p : nullptr, st);
     subset_counts(*m, st);
-    if (otf && (g.beam == MI_BEAM_FAN_FLAT || g.beam == MI_BEAM_FAN_ARC)) {
-        // FP32 runs project along the lines; FP64 runs, and geometries with a
-        // ray that has no line form, re-run the tracer from checkpoints
-        if (!build_lines(*m, a, st) || want64) build_otf(*m, a, st);
-    }
+    if (otf && fan) build_otf(*m, a, st);
     return m;
 }
 

@@ -32,6 +32,8 @@ GEOMS = {
     "half_turn": _fan(90, 90, 2.5, 31, 111, 3.3, span=180.0),
     "source_in_corner": _fan(64, 64, 4.0, 40, 96, 6.0, sod=150.0, sdd=500.0),
     "fine_pixels": _fan(48, 48, 0.04, 24, 80, 0.05, sod=20.0, sdd=40.0),   # pixels below the tracer's exit margin
+    "two_groups": _fan(336, 336, 1.0, 70, 96, 4.0),    # 441 blocks: two groups share a block's views
+    "one_group": _fan(432, 420, 0.8, 270, 64, 6.0),    # 729 blocks; 67 or 68 views a subset: two windows
     "arc": mi.arc_geometry(96, 3.0, 48, 98, 0.45, 595.0, 1085.6, 1.75),
     "arc_wide": mi.arc_geometry(61, 4.0, 40, 64, 1.6, 250.0, 600.0, -0.25),
 }
