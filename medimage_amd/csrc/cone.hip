@@ -23,7 +23,10 @@
 // Steps are taken in groups of 8: the group's voxel offsets and lengths are
 // computed first, its 8 loads issued together, then accumulated in order.
 //
-// Back projection (gather form, no atomics).  One lane per voxel column
+// Back projection (gather form, no atomics).  The usual cone beam goes by
+// panel patches (k_cone_bp_patch, where it is described); the parallel beam
+// and a source so near that a voxel's chord spans several rows go ray by ray
+// (k_cone_bp): one lane per voxel column
 // (x, y) and a chunk of kZc slices along z.  For each view the four corners
 // of the column are projected onto the panel: the columns whose rays can
 // cross it, and per slice the rows.  For each candidate ray the exact length
@@ -43,8 +46,10 @@
 
 #include <mutex>
 
+#include <climits>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 namespace mi {
@@ -56,7 +61,7 @@ constexpr int kConeGroup = 8;   // forward: walk steps per load group
 // Back projection: slices per lane.  A lane's per-view work on its column
 // (footprint, panel columns, x / y clip) is shared by its kZc slices, whose
 // double sums live in LDS (kZc x 2 KiB per workgroup, beside the rows' 1 / w):
-// C4 (512^3, 720 views) back projection 644 ms with 6 (18 KiB, 8 workgroups
+// 512^3, 720 views of 1024 x 768 (without k_cone_bp_patch): 644 ms with 6 (18 KiB, 8 workgroups
 // per CU), 663 with 7, 674 with 5, 680 with 8 (22 KiB, 7 per CU), 689 with 4.
 #ifndef MI_CONE_ZC
 #define MI_CONE_ZC 6
@@ -428,31 +433,15 @@ __device__ __forceinline__ void cone_slab_inv(double s, double ir, double a, dou
 // RLDS: the rows' 1 / w (nrows doubles) are copied to LDS (dynamic shared
 // memory) first.
 template <bool PAR, bool RLDS>
-__global__ __launch_bounds__(kBlock) void k_cone_bp(ConeDev g, const float *cs, const double *rowtab,
-                                                    const double2 *__restrict__ vinv, const float *__restrict__ vl2,
-                                                    const float4 *__restrict__ vsrc, const float2 *__restrict__ vpos,
-                                                    const int *views, int nv, const float *__restrict__ sino,
-                                                    double *carry, int first, int last, float *__restrict__ vol) {
-    // Workgroup: 16 x 16 voxel columns, wave 8 x 8 of them; kZc slices.
-    const int tx = (g.nx + 15) / 16, ty = (g.ny + 15) / 16;
-    const unsigned b = xcd_block();
-    const int per_z = tx * ty;
-    const int zc = (int)(b / per_z), tile = (int)(b % per_z);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int x = (tile / ty) * 16 + (wv >> 1) * 8 + (lane >> 3);
-    const int y = (tile % ty) * 16 + (wv & 1) * 8 + (lane & 7);
-    const int z0 = zc * kZc;
-    extern __shared__ double riw[];
-    if (RLDS) {
-        for (int r = threadIdx.x; r < g.nrows; r += kBlock) riw[r] = rowtab[2 * r + 1];
-        __syncthreads();
-    }
-    if (x >= g.nx || y >= g.ny || z0 >= g.nz) return;
-
+__device__ __forceinline__ void cone_bp_voxels(const ConeDev &g, const float *cs, const double *rowtab,
+                                               const double2 *__restrict__ vinv, const float *__restrict__ vl2,
+                                               const float4 *__restrict__ vsrc, const float2 *__restrict__ vpos,
+                                               const int *views, int nv, const float *__restrict__ sino, double *carry,
+                                               int first, int last, float *__restrict__ vol, int x, int y, int z0, int nk,
+                                               const double *riw, double (*acc)[kBlock]) {
     // Per-lane sums of the kZc voxels in LDS (each lane owns its own slots,
     // so no barrier is needed); a register sums one (column, slice) first.
-    __shared__ double acc[kZc][kBlock];
-    const int nk = min(kZc, g.nz - z0);
+    // nk <= kZc: the slices from z0.
     // carry: the double sums of the earlier view chunks of a back projection
     // split into several launches (nullptr for a single launch).
 #pragma unroll
@@ -563,6 +552,377 @@ __global__ __launch_bounds__(kBlock) void k_cone_bp(ConeDev g, const float *cs, 
     }
 }
 
+template <bool PAR, bool RLDS>
+__global__ __launch_bounds__(kBlock) void k_cone_bp(ConeDev g, const float *cs, const double *rowtab,
+                                                    const double2 *__restrict__ vinv, const float *__restrict__ vl2,
+                                                    const float4 *__restrict__ vsrc, const float2 *__restrict__ vpos,
+                                                    const int *views, int nv, const float *__restrict__ sino,
+                                                    double *carry, int first, int last, float *__restrict__ vol) {
+    // Workgroup: 16 x 16 voxel columns, wave 8 x 8 of them; kZc slices.
+    const int tx = (g.nx + 15) / 16, ty = (g.ny + 15) / 16;
+    const unsigned b = xcd_block();
+    const int per_z = tx * ty;
+    const int zc = (int)(b / per_z), tile = (int)(b % per_z);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int x = (tile / ty) * 16 + (wv >> 1) * 8 + (lane >> 3);
+    const int y = (tile % ty) * 16 + (wv & 1) * 8 + (lane & 7);
+    const int z0 = zc * kZc;
+    extern __shared__ double riw[];
+    __shared__ double acc[kZc][kBlock];
+    if (RLDS) {
+        for (int r = threadIdx.x; r < g.nrows; r += kBlock) riw[r] = rowtab[2 * r + 1];
+        __syncthreads();
+    }
+    if (x >= g.nx || y >= g.ny || z0 >= g.nz) return;
+    cone_bp_voxels<PAR, RLDS>(g, cs, rowtab, vinv, vl2, vsrc, vpos, views, nv, sino, carry, first, last, vol, x, y, z0,
+                              min(kZc, g.nz - z0), riw, acc);
+}
+
+// ---------------------------------------------------------------------------
+// Back projection of the cone beam from panel patches.
+//
+// For a panel column and a voxel column (x, y) the in-plane chord [lo, hi] is
+// the same for every row.  At chord parameter t row r is at height w_r t over
+// the source (w falls with r), so of a plane dZ over the source the rows
+// before some r1 are above it over the whole chord and those behind it are
+// below; where (rows / 2) x (chord / source distance) is less than one row, as
+// in every usual scanner, at most one row crosses it.  The sum of (row value x
+// chord length above the plane) is then
+//   B(dZ) = span PS[r1] + cut q_r1,
+// with q = sinogram x ray length, PS its running sum over the rows and cut
+// the part of the chord on which row r1 is above; a voxel between two planes
+// gets B(lower) - B(upper).  A lane so keeps one double per plane of its kNk
+// slices and spends some 14 instructions on a plane, where the form that
+// clips every candidate ray (k_cone_bp) spends about 40 on a slice (3.3
+// candidate rows, each with two double FMAs, a reciprocal, and a load).
+//
+// A workgroup is 16 x 16 voxel columns by kNk slices.  Per view it takes the
+// panel patch its voxels can see (up to some 60 x 70 pixels), one lane per
+// column and run of rows: each value is multiplied by its ray's length
+// (the hardware's square root, one ulp) and the running sums go to LDS; the
+// next view's values are loaded into registers meanwhile.  Summing order and
+// everything else is fixed by the geometry.
+//
+// Bounded by LDS reads (24 bytes per lane, plane and column, 12 clocks of a
+// CU per wave) and vector issue in about equal parts; two or three workgroups
+// per CU, which the patches' LDS allows.  512^3, 720 views of 1024 x 768: 508
+// ms ray by ray, 152 so; 256^3 x 360: 35.5 and 10.1; 128^3 x 180: 3.83 and
+// 0.94; 64^3 x 100: 0.91 and 0.30.  Against 64-bit sums of the exact lengths
+// both are off by 4.9e-7 of the largest voxel at 128^3.
+constexpr int kConeRun = 24, kConeStep = 4;   // rows of a patch column per lane: at most, a multiple of
+constexpr int kConeBatch = 5;                 // planes whose LDS reads are issued together (9: 4% slower at C4)
+struct ConeView {
+    int col0, ncol, r0, nr;       // the patch: panel columns, rows
+    int run, cand;                // rows per lane; candidate columns of a voxel column
+    float hw, icol;               // half width of a voxel column's shadow, 1 / ncol
+};
+
+// A value that all lanes hold, in scalar registers.
+__device__ __forceinline__ double uniform(double x) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u), hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// View (cos c, sin s) of the block of columns (x0, y0) .. and slices z0 .. z0 + nk.
+__device__ __forceinline__ ConeView cone_view(const ConeDev &g, float c, float s, int x0, int y0, int z0, int nk) {
+    const float kcol = g.sdd / g.pixel, sodv = g.sod / g.sample, h5 = (float)g.halfdet - 0.5f;
+    const float za = (float)z0 - g.nz / 2.0f, zb = za + (float)nk;
+    float lo = 1e30f, hi = -1e30f, ax = 0.f, ay = 0.f, rn = 0.f, rf = 1e30f;
+    for (int q = 0; q < 4; ++q) {
+        const float X = (float)min(g.nx, x0 + (q & 1) * 16) - g.nx / 2.0f, Y = (float)min(g.ny, y0 + (q >> 1) * 16) - g.ny / 2.0f;
+        const float rD = 1.0f / (-s * X + c * Y + sodv), u = (c * X + s * Y) * kcol * rD;
+        lo = fminf(lo, u);
+        hi = fmaxf(hi, u);
+        ax = fmaxf(ax, fabsf(c * kcol + s * u));
+        ay = fmaxf(ay, fabsf(s * kcol - c * u));
+        rn = fmaxf(rn, rD);
+        rf = fminf(rf, rD);
+    }
+    ConeView w;
+    // first order in the voxel (1 + 2 rn covers the rest), and the float rounding
+    w.hw = 0.5f * (ax + ay) * rn * (1.0f + 2.0f * rn) + 0.01f;
+    w.cand = (int)floorf(2.0f * w.hw) + 1;
+    const float rlo = h5 - kcol * fmaxf(zb * rn, zb * rf), rhi = h5 - kcol * fminf(za * rn, za * rf);
+    w.col0 = max(0, (int)floorf(lo + h5 - w.hw) - 1);
+    w.ncol = max(0, min(g.ncols - 1, (int)ceilf(hi + h5 + w.hw) + 1) - w.col0 + 1);
+    w.r0 = min(g.nrows, max(0, (int)floorf(rlo) - 2));
+    w.nr = max(0, min(g.nrows - 1, (int)ceilf(rhi) + 2) - w.r0 + 1);
+    if (w.ncol == 0 || w.nr == 0) w.ncol = w.nr = 0;
+    const int seg = kBlock / max(w.ncol, 1);
+    w.run = seg > 0 ? ((w.nr + seg - 1) / seg + kConeStep - 1) / kConeStep * kConeStep : INT_MAX;
+    if (seg > 0 && w.nr > 0) w.nr = (w.nr + w.run - 1) / w.run * w.run;   // whole runs: rows behind the panel read as 0
+    w.icol = 1.0f / (float)max(w.ncol, 1);
+    return w;
+}
+
+// The largest patch of any block and view: m[0] columns, m[1] rows, m[2] rows
+// per lane; m[3] the most rows a block sees over all views.
+__global__ __launch_bounds__(kWave) void k_cone_patch(ConeDev g, const float *cs, int nk, int *m) {
+    const int tx = (g.nx + 15) / 16, ty = (g.ny + 15) / 16;
+    const int b = (int)blockIdx.x, zc = b / (tx * ty), tile = b % (tx * ty);
+    int nc = 0, nr = 0, run = 0, r0 = INT_MAX, r1 = 0;
+    for (int v = (int)threadIdx.x; v < g.nviews; v += kWave) {
+        const ConeView w = cone_view(g, cs[2 * v], cs[2 * v + 1], tile / ty * 16, tile % ty * 16, zc * nk, nk);
+        nc = max(nc, w.ncol);
+        nr = max(nr, w.nr);
+        run = max(run, w.run);
+        if (w.nr > 0) {
+            r0 = min(r0, w.r0);
+            r1 = max(r1, w.r0 + w.nr);
+        }
+    }
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        nc = max(nc, __shfl_xor(nc, o));
+        nr = max(nr, __shfl_xor(nr, o));
+        run = max(run, __shfl_xor(run, o));
+        r0 = min(r0, __shfl_xor(r0, o));
+        r1 = max(r1, __shfl_xor(r1, o));
+    }
+    if (threadIdx.x == 0) {
+        atomicMax(m, nc);
+        atomicMax(m + 1, nr);
+        atomicMax(m + 2, run);
+        if (r1 > 0) atomicMax(m + 3, r1 - r0);
+    }
+}
+
+// LDS of a workgroup: the running sums (column major; one entry before the
+// first row and one behind the last), 1 / w and w^2 of the rows its views
+// see, 1 / (d - s) per column, the lanes' totals, the views.
+constexpr int kConeViews = 36;
+__host__ __device__ __forceinline__ int cone_patch_stride(int rows) { return (rows + 3) | 1; }
+__host__ __device__ __forceinline__ size_t cone_patch_lds(int cols, int rows, int span) {
+    const size_t sums = ((size_t)cols * cone_patch_stride(rows) + 1) & ~(size_t)1;
+    const size_t need = 8 * (sums + 2 * (size_t)cols + kBlock + span + 2) + 4 * (size_t)(span + 2) + kConeViews * sizeof(ConeView);
+    return need > kZc * kBlock * 8 ? need : kZc * kBlock * 8;   // (the sums of the ray by ray form)
+}
+
+// CROSS: the source's height lies within the block's slices.
+template <int NK, bool CROSS>
+__device__ __forceinline__ void cone_bp_block(
+    const ConeDev &g, const float *cs, const double *rowtab, const double2 *__restrict__ vinv, const float *__restrict__ vl2,
+    const float4 *__restrict__ vsrc, const int *views, int nv, const float *__restrict__ sino, float *__restrict__ vol,
+    int cols, int rows, int span_rows, int x0, int y0, int z0) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int x = x0 + (wv >> 1) * 8 + (lane >> 3), y = y0 + (wv & 1) * 8 + (lane & 7);
+    extern __shared__ double smem[];
+    const int stride = cone_patch_stride(rows);
+    double *PS = smem;
+    double2 *irs = (double2 *)(PS + ((cols * stride + 1) & ~1));
+    double *tots = (double *)(irs + cols), *iws = tots + kBlock;
+    ConeView *info = (ConeView *)(iws + span_rows + 2);
+    float *w2s = (float *)(info + kConeViews);
+    __shared__ int sh_r0, sh_r1;
+    const float kcol = g.sdd / g.pixel, kz = g.sample / g.pixel, sodv = g.sod / g.sample, h5 = (float)g.halfdet - 0.5f;
+    const float px = (float)x + 0.5f - g.nx / 2.0f, py = (float)y + 0.5f - g.ny / 2.0f;
+    const double sz = (double)vsrc[views[0]].z, xd = x, yd = y;   // the source's height is every view's
+
+    // the planes' heights: all over the source (or at it), all under, or both
+    const float dz0 = (float)z0 - g.nz / 2.0f;
+    const bool over = dz0 >= 0.0f;
+    const int kover = __builtin_amdgcn_readfirstlane((int)floorf(-dz0) + 1);   // the first plane over the source
+    double A[NK + 1], mdZ[NK + 1];
+#pragma unroll
+    for (int k = 0; k <= NK; ++k) {
+        A[k] = 0.0;
+        mdZ[k] = uniform(-fabs((double)(z0 + k) - sz));
+    }
+    float raw[kConeRun], l2 = 0.f;
+    double2 ir = make_double2(0.0, 0.0);
+    const int rowb = g.ncols * 4;
+    // this lane's part of view iv's patch, into registers (rows behind its
+    // run are other lanes', rows behind the panel read as 0)
+    int v0 = 0;
+    bool bad = false;   // a sum of this lane was not finite
+    auto load = [&](int iv) {
+        const ConeView w = info[iv];
+        const int seg = (int)(((float)tid + 0.5f) * w.icol), col = tid - seg * w.ncol;   // tid / ncol
+        const size_t panel = (size_t)g.nrows * g.ncols;
+        const int v = __builtin_amdgcn_readfirstlane(views[v0 + iv]);
+        const auto rs = __builtin_amdgcn_make_buffer_rsrc((void *)(sino + v * panel), 0, (int)(panel * 4), 0x00020000);
+        const int run = __builtin_amdgcn_readfirstlane(w.run);
+        const int at = ((w.r0 + seg * run) * g.ncols + w.col0 + col) * 4;
+        const bool any = w.ncol > 0 && seg * run < w.nr;
+        if (any) {
+            l2 = vl2[(size_t)v * g.ncols + w.col0 + col];
+#pragma unroll
+            for (int i = 0; i < kConeRun; i += kConeStep)
+                if (i < run)
+#pragma unroll
+                    for (int h = i; h < i + kConeStep; ++h)
+                        raw[h] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, at + h * rowb, 0, 0));
+        }
+        if (tid < w.ncol) ir = vinv[(size_t)v * g.ncols + w.col0 + tid];
+    };
+    for (; v0 < nv; v0 += kConeViews) {
+        const int ng = min(kConeViews, nv - v0);
+        if (tid == 0) {
+            sh_r0 = g.nrows;
+            sh_r1 = 0;
+        }
+        __syncthreads();
+        if (tid < ng) {
+            const int v = views[v0 + tid];
+            const ConeView w = cone_view(g, cs[2 * v], cs[2 * v + 1], x0, y0, z0, NK);
+            info[tid] = w;
+            if (w.nr > 0) {
+                atomicMin(&sh_r0, w.r0);
+                atomicMax(&sh_r1, w.r0 + w.nr);
+            }
+        }
+        __syncthreads();
+        const int rbase = sh_r0, rspan = sh_r1 - sh_r0;
+        for (int i = tid; i < rspan + 2; i += kBlock) {   // entry i: row rbase + i - 1
+            const int r = min(max(rbase + i - 1, 0), g.nrows - 1);
+            const float wr = (float)rowtab[2 * r];
+            iws[i] = rowtab[2 * r + 1];
+            w2s[i] = wr * wr;
+        }
+        load(0);
+        __syncthreads();
+        for (int iv = 0; iv < ng; ++iv) {
+            ConeView w = info[iv];
+            w.ncol = __builtin_amdgcn_readfirstlane(w.ncol);   // (0: the view does not see the block)
+            w.cand = __builtin_amdgcn_readfirstlane(w.cand);
+            w.nr = __builtin_amdgcn_readfirstlane(w.nr);
+            w.run = __builtin_amdgcn_readfirstlane(w.run);
+            w.r0 = __builtin_amdgcn_readfirstlane(w.r0);
+            w.col0 = __builtin_amdgcn_readfirstlane(w.col0);
+            const int v = __builtin_amdgcn_readfirstlane(views[v0 + iv]);
+            // q = sinogram x ray length, the runs' totals
+            const int seg = (int)(((float)tid + 0.5f) * w.icol), col = tid - seg * w.ncol;
+            const int r = seg * w.run;
+            const bool any = r < w.nr;
+            double sum = 0.0;
+            if (any) {
+                const float *w2 = w2s + (w.r0 - rbase + r + 1);
+#pragma unroll
+                for (int i = 0; i < kConeRun; i += kConeStep)
+                    if (i < w.run)
+#pragma unroll
+                        for (int h = i; h < i + kConeStep; ++h) {
+                            raw[h] *= __builtin_amdgcn_sqrtf(w2[h] + l2);
+                            sum += (double)raw[h];
+                            asm volatile("" : "+v"(raw[h]));   // (converted again below: not 24 doubles kept)
+                        }
+            }
+            bad |= !(fabs(sum) < INFINITY);
+            tots[tid] = sum;
+            // a ray along an axis: all or nothing on the other, by a huge finite
+            // inverse (0 x infinity has no value)
+            if (tid < w.ncol) irs[tid] = make_double2(fmin(fmax(ir.x, -1e300), 1e300), fmin(fmax(ir.y, -1e300), 1e300));
+            __syncthreads();
+            if (any) {
+                double run = 0.0;
+                for (int i = 0; i < seg; ++i) run += tots[i * w.ncol + col];
+                double *P = PS + col * stride + 2 + r;   // P[i]: the rows up to r + i
+                if (seg == 0) P[-2] = P[-1] = 0.0;
+#pragma unroll
+                for (int i = 0; i < kConeRun; i += kConeStep)
+                    if (i < w.run)
+#pragma unroll
+                        for (int h = i; h < i + kConeStep; ++h) P[h] = run += (double)raw[h];
+                if (r + w.run == w.nr) P[w.run] = run;
+            }
+            __syncthreads();
+            if (iv + 1 < ng) load(iv + 1);
+
+            const float c = cs[2 * v], sn = cs[2 * v + 1];
+            const float4 sp = vsrc[v];
+            const float rD = __builtin_amdgcn_rcpf(-sn * px + c * py + sodv);
+            const int c0 = (int)ceilf((c * px + sn * py) * kcol * rD + h5 - w.hw) - w.col0;
+            const double *iw0 = iws + (w.r0 - rbase);   // entry i: row r0 + i - 1
+            const float h5r = h5 - (float)w.r0;
+            for (int j = 0; j < (w.ncol > 0 ? w.cand : 0); ++j) {
+                const bool in = (unsigned)(c0 + j) < (unsigned)w.ncol;
+                const int lc = in ? c0 + j : 0;
+                const double2 irc = irs[lc];
+                const double ax = (xd - (double)sp.x) * irc.x, ay = (yd - (double)sp.y) * irc.y;
+                const double bx = ax + irc.x, by = ay + irc.y;
+                const double lo = fmax(fmax(fmin(ax, bx), fmin(ay, by)), 0.0), hi = fmin(fmin(fmax(ax, bx), fmax(ay, by)), 1.0);
+                const float span = (in && hi > lo) ? (float)(hi - lo) : 0.0f;
+                if (!__any(span > 0.0f)) continue;
+                const float inv = span > 0.0f ? (__builtin_amdgcn_rcpf((float)lo) + __builtin_amdgcn_rcpf((float)hi)) * (0.5f * kz) : 0.0f;
+                const double spand = (double)span, nlo = -lo, base = over ? hi : nlo;
+                const double *P = PS + lc * stride;
+                const float last = (float)(w.nr + 1);
+                // the row nearest the plane's at the middle of the chord; planes
+                // at the source's height between two rows take the one on their
+                // block's side of it
+                float pos = __builtin_fmaf(-dz0, inv, h5r + (over ? 1.495f : 1.505f));
+#pragma unroll
+                for (int k0 = 0; k0 <= NK; k0 += kConeBatch) {   // the planes' LDS reads, a few together
+                    double a[kConeBatch], b[kConeBatch], iw[kConeBatch];
+#pragma unroll
+                    for (int k = k0; k < k0 + kConeBatch && k <= NK; ++k) {
+                        const int i = (int)__builtin_amdgcn_fmed3f(pos, 0.0f, last);
+                        pos -= inv;
+                        a[k - k0] = P[i];
+                        b[k - k0] = P[i + 1];
+                        iw[k - k0] = iw0[i];
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int k = k0; k < k0 + kConeBatch && k <= NK; ++k) {
+                        double from = base;
+                        if constexpr (CROSS) {
+                            int kz = kover;
+                            asm volatile("" : "+v"(kz));   // (compared here: no mask per plane kept in registers)
+                            from = k >= kz ? hi : nlo;
+                        }
+                        const float cut = __builtin_amdgcn_fmed3f((float)__builtin_fma(mdZ[k], iw[k - k0], from), 0.0f, span);
+                        // (a row entirely above counts like the rows before it, so that
+                        // two planes with no row between them sum alike, to the bit)
+                        const double from0 = cut < span ? a[k - k0] : b[k - k0];
+                        A[k] = __builtin_fma(spand, from0, A[k]);
+                        A[k] = __builtin_fma((double)cut, b[k - k0] - from0, A[k]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            __syncthreads();   // the patch is written again
+        }
+    }
+    if (__syncthreads_or(bad)) {
+        // A value that is not finite would reach every row behind it through
+        // the running sums: the block's voxels ray by ray instead.
+        const int zend = min(z0 + NK, g.nz);
+        for (int z = z0; z < zend; z += kZc) {
+            if (x >= g.nx || y >= g.ny) break;
+            cone_bp_voxels<false, false>(g, cs, rowtab, vinv, vl2, vsrc, nullptr, views, nv, sino, nullptr, 1, 1, vol, x, y,
+                                         z, min(kZc, zend - z), nullptr, (double(*)[kBlock])smem);
+        }
+        return;
+    }
+    if (x >= g.nx || y >= g.ny) return;
+    const int nk = min(NK, g.nz - z0);
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+        if (k < nk) {
+            const size_t i = ((size_t)(z0 + k) * g.nx + x) * g.ny + y;
+            vol[i] = (float)(A[k] - A[k + 1]);
+        }
+}
+
+template <int NK>
+__global__ __launch_bounds__(kBlock) void k_cone_bp_patch(
+    ConeDev g, const float *cs, const double *rowtab, const double2 *__restrict__ vinv, const float *__restrict__ vl2,
+    const float4 *__restrict__ vsrc, const int *views, int nv, const float *__restrict__ sino, float *__restrict__ vol,
+    int cols, int rows, int span_rows) {
+    const int tx = (g.nx + 15) / 16, ty = (g.ny + 15) / 16;
+    const unsigned blk = xcd_block();
+    const int z0 = (int)(blk / (tx * ty)) * NK, tile = (int)(blk % (tx * ty));
+    if (z0 >= g.nz) return;
+    const int x0 = (tile / ty) * 16, y0 = (tile % ty) * 16;
+    if (2 * z0 < g.nz && 2 * (z0 + NK) > g.nz)
+        cone_bp_block<NK, true>(g, cs, rowtab, vinv, vl2, vsrc, views, nv, sino, vol, cols, rows, span_rows,
+                                x0, y0, z0);
+    else
+        cone_bp_block<NK, false>(g, cs, rowtab, vinv, vl2, vsrc, views, nv, sino, vol, cols, rows, span_rows,
+                                 x0, y0, z0);
+}
+
 unsigned grid8(size_t blocks) { return (unsigned)((blocks + 7) / 8 * 8); }
 
 }  // namespace
@@ -636,6 +996,32 @@ ConeTables &cone_tables(mi_context *ctx, const mi_cone_geometry &g) {
     hipLaunchKernelGGL(k_cone_vctab, dim3((unsigned)((nvc + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream, t->d,
                        t->cs.p, t->vinv.p, t->vl2.p, t->vsrc.p, t->vpos.p);
     MI_HIP(hipGetLastError());
+    if (!t->d.parallel) {
+        // At most one row may cross a plane within a voxel column's chord
+        // (sqrt 2 voxels at the least distance from the source).
+        const double near = g.sod_mm / (double)g.sample_mm - 0.5 * std::hypot((double)g.nx, (double)g.ny);
+        const double far = std::max(t->d.halfdet, g.n_rows - t->d.halfdet) + 1.0;
+        if (near > 1.0 && far * std::sqrt(2.0) / near + 0.05 < 1.0) {
+            DevBuf<int> m(8);
+            int h[8];
+            MI_HIP(hipMemsetAsync(m.p, 0, m.bytes(), ctx->stream));
+            for (int i = 0; i < 2; ++i) {
+                const size_t nb = (size_t)((g.nx + 15) / 16) * ((g.ny + 15) / 16) * ((g.nz + kConeNk[i] - 1) / kConeNk[i]);
+                hipLaunchKernelGGL(k_cone_patch, dim3((unsigned)nb), dim3(kWave), 0, ctx->stream, t->d, t->cs.p, kConeNk[i],
+                                   m.p + 4 * i);
+                MI_HIP(hipGetLastError());
+            }
+            MI_HIP(hipMemcpyAsync(h, m.p, sizeof(h), hipMemcpyDeviceToHost, ctx->stream));
+            MI_HIP(hipStreamSynchronize(ctx->stream));
+            for (int i = 0; i < 2; ++i)
+                if (h[4 * i] > 0 && h[4 * i + 2] <= kConeRun && ((size_t)g.n_rows + kConeRun) * g.n_cols < (size_t)1 << 29 &&
+                    cone_patch_lds(h[4 * i], h[4 * i + 1], h[4 * i + 3]) <= ((size_t)63 << 10)) {
+                    t->patch_cols[i] = h[4 * i];
+                    t->patch_rows[i] = h[4 * i + 1];
+                    t->patch_span[i] = h[4 * i + 3];
+                }
+        }
+    }
     MI_HIP(hipStreamSynchronize(ctx->stream));
     ctx->cone = t;
     return *t;
@@ -695,21 +1081,38 @@ int64_t cone_scratch_voxels() { return (int64_t)kScratchCarry; }
 
 void cone_bp_views(hipStream_t st, const ConeTables &t, const int *views, int nv, const float *sino, float *vol,
                    int device_scratch) {
-    const size_t blocks = (size_t)((t.d.nx + 15) / 16) * ((t.d.ny + 15) / 16) * ((t.d.nz + kZc - 1) / kZc);
-    // Views in chunks whose sinogram rows stay cached while every workgroup
-    // sweeps them; double sums carried between chunks (a buffer allocated
-    // here, or the device's fixed scratch array).
     const int chunks = (nv + kBpViewChunk - 1) / kBpViewChunk;
     const size_t nvox = (size_t)t.d.nx * t.d.ny * t.d.nz;
-    DevBuf<double> own(chunks > 1 && device_scratch < 0 ? nvox : 0);
-    double *carry = own.p;
     if (chunks > 1 && device_scratch >= 0) {
         MI_REQUIRE(nvox <= kScratchCarry, MI_E_LIMIT,
                    "volume of " + std::to_string(nvox) + " voxels exceeds the allocation-free back projection's " +
                        std::to_string(kScratchCarry) + "-voxel scratch");
-        carry = g_scratch_ptr[device_scratch];
-        MI_REQUIRE(carry, MI_E_STATE, "device scratch not initialised");
+        MI_REQUIRE(g_scratch_ptr[device_scratch], MI_E_STATE, "device scratch not initialised");
     }
+    auto grid = [&](int nk) { return (size_t)((t.d.nx + 15) / 16) * ((t.d.ny + 15) / 16) * ((t.d.nz + nk - 1) / nk); };
+    // The patch form where the geometry has it, all views in one launch (the
+    // sums stay in registers: 5 launches of 36 views and their carry volume
+    // were 1.31 ms at 128^3 x 180 views, one is 1.14).  16 slices a workgroup,
+    // 8 where that leaves fewer workgroups than two per CU or 16 slices' patch
+    // does not fit: 128^3 x 180 views (512 workgroups of 16) 0.94 ms with 16
+    // and 1.22 with 8, 512^3 x 720 152 and 214, 64^3 x 100 (64 workgroups of
+    // 16) 0.40 and 0.30.
+    int patch = t.patch_cols[0] > 0 ? 0 : -1;
+    if (t.patch_cols[1] > 0 && (patch < 0 || grid(kConeNk[0]) < 512)) patch = 1;
+    if (patch >= 0) {
+        const int pc = t.patch_cols[patch], pr = t.patch_rows[patch], ps = t.patch_span[patch];
+        launch(patch == 0 ? k_cone_bp_patch<kConeNk[0]> : k_cone_bp_patch<kConeNk[1]>, dim3(grid8(grid(kConeNk[patch]))),
+               dim3(kBlock), (uint32_t)cone_patch_lds(pc, pr, ps), st, t.d, t.cs.p, t.rows.p, t.vinv.p, t.vl2.p, t.vsrc.p,
+               views, nv, sino, vol, pc, pr, ps);
+        MI_HIP(hipGetLastError());
+        return;
+    }
+    const size_t blocks = grid(kZc);
+    // Views in chunks whose sinogram rows stay cached while every workgroup
+    // sweeps them; double sums carried between chunks (a buffer allocated
+    // here, or the device's fixed scratch array).
+    DevBuf<double> own(chunks > 1 && device_scratch < 0 ? nvox : 0);
+    double *carry = chunks > 1 && device_scratch >= 0 ? g_scratch_ptr[device_scratch] : own.p;
     for (int c = 0; c < chunks; ++c) {
         const int v0 = c * kBpViewChunk, n = std::min(kBpViewChunk, nv - v0);
         if (t.d.parallel)

@@ -28,8 +28,13 @@ struct ConeTables {
     DevBuf<float> vl2;     // [nviews * ncols]: (dx - sx)^2 + (dy - sy)^2
     DevBuf<float4> vsrc;   // [nviews]: source point (cone beam)
     DevBuf<float2> vpos;   // [nviews * ncols]: (x, y) of the column's rays' start (parallel beam)
+    // Cone beam: the largest panel patch (columns, rows) any view shows of a
+    // 16 x 16 column block of kConeNk[i] slices, and the most rows all views
+    // show of one; 0 columns: no patch form.
+    int patch_cols[2] = {0, 0}, patch_rows[2] = {0, 0}, patch_span[2] = {0, 0};
     int64_t nnz = -1;      // traced entries of all rays (-1: not counted yet)
 };
+constexpr int kConeNk[2] = {16, 8};   // back projection from panel patches: slices per workgroup
 
 void validate_cone(const mi_cone_geometry &g);
 // The context's tables for g (rebuilt when g differs from the cached one).
