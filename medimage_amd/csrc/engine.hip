@@ -776,6 +776,90 @@ __device__ __forceinline__ void line_fp_unit(const EngArgs<float> &a, const UG<f
     if (lane == 0) part_at(a, U, RESID ? SL_DF : SL_AD, wv)[lb] = mm;
 }
 
+// One image with its lines' zeros around it, row by row (px) and column by
+// column (py), from row-major pixels.
+__global__ __launch_bounds__(kBlock) void k_line_planes(const float *__restrict__ img, int nx, int ny,
+                                                        float *__restrict__ px, float *__restrict__ py) {
+    const int64_t ex = line_elems(nx, ny), ey = line_elems(ny, nx);
+    const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (e < ex) {
+        const int64_t i = e / line_stride(ny), j = e % line_stride(ny) - kLinePad;
+        px[e] = i < nx && j >= 0 && j < ny ? img[i * ny + j] : 0.0f;
+    } else if (e < ex + ey) {
+        const int64_t j = (e - ex) / line_stride(nx), i = (e - ex) % line_stride(nx) - kLinePad;
+        py[e - ex] = j < ny && i >= 0 && i < nx ? img[i * ny + j] : 0.0f;
+    }
+}
+
+// sino = A img over every view: the forward projection above without a
+// residual, for one image.  512 x 512 pixels, 720 views of 736 bins: a
+// whole call from and to host arrays 382 us, 1593 with a wave per ray that
+// reads the matrix (1332 of it, 2.7 GB); relative error against 64 bits 2.6e-8
+// and 3.2e-8.
+__global__ __launch_bounds__(kLineBlock) void k_line_project(
+    const float *px, const float *py, int nx, int ny, int nbins, int64_t groups, const double2 *__restrict__ mb,
+    const float *__restrict__ rinv, const double *__restrict__ rlen, const int32_t *__restrict__ drop,
+    const float *__restrict__ dlen, const int4 *__restrict__ rng, float *__restrict__ sino) {
+    __shared__ double lds[kLineWaves][kLineRays];
+    const int lane = threadIdx.x & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int64_t lb = xcd_block();
+    if (lb >= groups) return;
+    const int per = (nbins + kLineRays - 1) / kLineRays;
+    const int64_t view = lb / per;
+    const int bin = (int)(lb - view * per) * kLineRays + lane;
+    const int64_t row = view * nbins + bin;
+    const bool valid = bin < nbins;
+    double m = 0.0, b0 = 0.0, acc[1] = {0.0};
+    float inv = 0.0f;
+    if (valid) {
+        m = mb[row].x;
+        b0 = mb[row].y;
+        inv = rinv[row];
+    }
+    const int4 r = rng[lb];
+#pragma unroll
+    for (int ax = 0; ax < 2; ++ax) {
+        const int r0 = ax ? r.z : r.x, r1 = ax ? r.w : r.y;
+        if (r0 >= r1) continue;
+        const int run = ((r1 - r0 + kLineWaves - 1) / kLineWaves + 7) & ~7, c0 = r0 + wv * run;
+        if (c0 >= r1) continue;
+        const bool mine = valid && (inv < 0.0f) == (ax == 1);
+        line_run<1>((const GL float *)(ax ? py : px), ax ? ny : nx, ax ? nx : ny, c0, min(run, (r1 - c0 + 7) & ~7),
+                    mine ? m : 0.0, mine ? b0 : -64.0, mine ? fabsf(inv) : 0.0f, acc);
+    }
+    lds[wv][lane] = acc[0];
+    __syncthreads();
+    if (wv != 0 || !valid) return;
+    double tot = 0.0;
+#pragma unroll
+    for (int w = 0; w < kLineWaves; ++w) tot += lds[w][lane];
+    const double len = rlen[row];
+    const int dp = drop[row];
+    tot *= len;
+    if (dp >= 0) tot -= (double)dlen[row] * (double)px[(int64_t)(dp / ny) * line_stride(ny) + dp % ny + kLinePad];
+    if (!(fabs(tot) < INFINITY)) {
+        // Some pixel beside the ray or of its dropped piece may not be finite
+        // (weight 0 times it is not 0): only what the ray crosses counts.
+        const bool ay = inv < 0.0f;
+        const float *p = ay ? py : px;
+        const int nb = ay ? nx : ny, r0 = ay ? r.z : r.x, r1 = min(ay ? r.w : r.y, ay ? ny : nx);
+        tot = 0.0;
+        for (int a = r0; a < r1; ++a) {
+            const double pos = b0 + 0.5 * fabs(m) + m * a, jf = floor(pos);
+            if (!(jf >= 0.0 && jf <= (double)nb)) continue;
+            const int j = (int)jf;
+            const double w = fmin(1.0, (pos - jf) * (double)fabsf(inv));
+            for (int h = 0; h < 2; ++h) {   // pixels j - 1 and j of the line (both may be padding)
+                const int jj = j - 1 + h;
+                double part = (h ? w : 1.0 - w) * len;
+                if (dp == (ay ? jj * ny + a : a * ny + jj) && jj >= 0 && jj < nb) part -= (double)dlen[row];
+                if (part > 1e-6 * len) tot += part * (double)p[(int64_t)a * line_stride(nb) + jj + kLinePad];
+            }
+        }
+    }
+    sino[row] = (float)tot;
+}
+
 // K interleaved values at pixel (i, j), or `pad` outside the image.
 template <typename T, int K>
 __device__ __forceinline__ void ldn(const UG<T> &U, const GL T *arr, int i, int j, T (&o)[K], T pad) {
@@ -2047,6 +2131,17 @@ void eng_line_bp(hipStream_t st, const EngArgs<float> &a, const BlockMap &m, int
     if (kmax == 1) go(std::integral_constant<int, 1>{});
     else if (kmax <= 4) go(std::integral_constant<int, 4>{});
     else go(std::integral_constant<int, kMaxK>{});
+    MI_HIP(hipGetLastError());
+}
+
+void line_project(hipStream_t st, const Matrix &m, const float *img, float *px, float *py, float *sino) {
+    const mi_geometry &g = m.g;
+    const Lines &q = m.lines;
+    const int64_t groups = q.slice0.back() / 4;
+    k_line_planes<<<grid_of(line_elems(g.nx, g.ny) + line_elems(g.ny, g.nx)), kBlock, 0, st>>>(img, g.nx, g.ny, px, py);
+    MI_HIP(hipGetLastError());
+    k_line_project<<<grid8((int)groups), kLineBlock, 0, st>>>(px, py, g.nx, g.ny, g.n_bins, groups, q.mb.p, q.inv.p, q.len.p,
+                                                              q.drop.p, q.dlen.p, q.rng.p, sino);
     MI_HIP(hipGetLastError());
 }
 

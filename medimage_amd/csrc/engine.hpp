@@ -140,6 +140,9 @@ void eng_fp_sq(hipStream_t st, const EngArgs<T> &a, const BlockMap &rows, int s,
 // The two forward projections of units with lines (FP32): r = g - A_s u and
 // ||A_s d||^2, from the unit's projection images.
 void eng_line_fp(hipStream_t st, const EngArgs<float> &a, const BlockMap &m, int s, int kmax, bool resid);
+// sino = A img along the lines of a one-subset geometry's rays; px, py: scratch
+// of line_elems(nx, ny) and line_elems(ny, nx) floats.
+void line_project(hipStream_t st, const Matrix &m, const float *img, float *px, float *py, float *sino);
 // The back projection of units with lines, as eng_bp_grad; groups (1, 2 or 4,
 // line_groups of every unit): 256-lane groups that share a block's views.
 void eng_line_bp(hipStream_t st, const EngArgs<float> &a, const BlockMap &m, int s, int kmax, int groups);

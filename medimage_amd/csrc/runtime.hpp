@@ -61,7 +61,8 @@ struct GeomKey {
 };
 // The caller's per-view angle table as an owned copy (empty: none).
 std::vector<double> view_table(const mi_geometry &g);
-// layout: 0 = CSR / CSC (projector calls), 1 = sliced (AT engine).
+// layout: 0 = CSR / CSC (projector calls), 1 = sliced (AT engine), 2 = the
+// rays' lines alone (has_lines false: a ray has no such form).
 GeomKey make_key(const mi_geometry &g, int n_subsets, int layout = 0);
 void validate_geometry(const mi_geometry &g);
 
@@ -317,7 +318,7 @@ void build_sell(Matrix &m, hipStream_t st, bool drop_csr = false);
 // lengths.  Host-side GoldenC walk for MI_BEAM_GOLDENC, device tracers
 // otherwise.
 // otf: also record the checkpointed forward walk (fan beam only).
-std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, hipStream_t st, bool otf = false);
+std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, hipStream_t st, int layout = 0);
 // Subset order: bit-reversed subset indices (values >= S dropped).
 std::vector<int> subset_order(int S);
 

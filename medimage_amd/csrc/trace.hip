@@ -708,7 +708,7 @@ size_t Matrix::bytes() const {
            seq_bytes(seq.get());
 }
 
-std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, hipStream_t st, bool otf) {
+std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, hipStream_t st, int layout) {
     validate_geometry(g);
     MI_REQUIRE(S >= 1 && S <= g.n_views, MI_E_ARG, "n_subsets must be in [1, n_views]");
     auto m = std::make_unique<Matrix>();
@@ -834,7 +834,11 @@ std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, h
     // matrix; FP64 runs, and geometries with a ray that has no line form, re-run
     // the tracer from checkpoints and read the matrix.
     const bool fan = g.beam == MI_BEAM_FAN_FLAT || g.beam == MI_BEAM_FAN_ARC;
-    if (otf && fan && build_lines(*m, a, st) && !want64) {
+    if (layout != 0 && fan && build_lines(*m, a, st) && !want64) {
+        m->has_csr = false;
+        return m;
+    }
+    if (layout == 2) {
         m->has_csr = false;
         return m;
     }
@@ -852,7 +856,7 @@ std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, h
     MI_HIP(hipGetLastError());
     build_csc(*m, m->rowptr.p, m->idx.p, m->len32.p, want64 ? m->len64.p : nullptr, st);
     subset_counts(*m, st);
-    if (otf && fan) build_otf(*m, a, st);
+    if (layout == 1 && fan) build_otf(*m, a, st);
     return m;
 }
 
