@@ -3,9 +3,8 @@
 // reference program adds it, so results equal the reference's bit for bit:
 //   * A: one lane per ray sums its products in the order proj.c emits them;
 //   * AStar: one lane per pixel, likewise;
-//   * energies, norms, inner products: one workgroup per sum, whose result
-//     is the running double's after adding the terms one by one in
-//     row-major order (k_chains).
+//   * energies, norms, inner products: the running double's value after
+//     adding the terms one by one in row-major order (k_chain_scan).
 #include "ordered.hpp"
 #include "gc_stencil.hpp"
 
@@ -149,36 +148,100 @@ __device__ __forceinline__ void chain_term(const ChainSeg &s, const ChainArgs &a
     }
 }
 
-// One sequential sum per workgroup, 4096 terms a step.
+// Folding the terms in index order, rounding after every add as the
+// reference's loop does, need not be a serial chain.  While the running sum
+// acc stays inside one binade, adding a term t moves it by t rounded to acc's
+// own unit in the last place, whatever acc's bits are, unless t lies exactly
+// halfway between two multiples of it (then ties-to-even looks at acc).  So
+// per chunk of 64 terms the rounded terms are integers that may be added in
+// any order, and the chunks' sums are applied in order as long as (a) no term
+// is a tie, infinite, NaN or 2^50 units or more, and (b) acc plus the chunk's
+// positive terms stays below the binade's upper end and acc plus its negative
+// ones (each up to half a unit more than its rounded value) above the lower
+// end.
 //
-// The terms are computed by all lanes, and folding them in index order
-// (rounding after every add, as the reference's loop does) need not be a
-// serial chain.  While the running sum acc stays inside one binade, adding a
-// term t moves it by t rounded to acc's own unit in the last place, whatever
-// acc's bits are, unless t lies exactly halfway between two multiples of it
-// (then ties-to-even looks at acc).  So per 256 terms (one wave) the rounded
-// terms are integers that may be added in any order, and the 16 waves' sums
-// are applied in order as long as (a) no term is a tie, infinite, NaN or
-// 2^50 units or more, and (b) acc plus the wave's positive terms stays below
-// the binade's upper end and acc plus its negative ones (each up to half a
-// unit more than its rounded value) above the lower end.
-// A wave that fails this is folded term by term from LDS, after which the
-// waves behind it are rounded again for acc's new binade.  acc's binade
-// changes about log2(n) times, so a sum of 4e5 terms folds some 20 waves of
-// 1600 serially.
+// Three launches.  k_chain_terms computes all terms and their plain sums,
+// k_chain_records rounds each chunk for the binade that the plain sums put
+// acc in, and k_chain_scan, one wave per sum, applies the records, 64 x 1024
+// terms at a time where all of them hold.  A record whose binade is not acc's
+// (the plain sum may be off near a binade's end), or that fails (a) or (b), is
+// folded term by term; acc's binade changes about log2(n) times, so a sum of
+// 4e5 terms folds some 25 chunks of 6500.  The result does not depend on the
+// plain sums: they only choose which chunks are folded.
 //
-// Measured over the sums of one GoldenC alternation (2.6e5 to 5.2e5 terms):
-// 696 us a launch, against 5189 us (13 ns a term) with one wave per sum that
-// took each term from its lane and added it.
-constexpr int kChainThreads = 1024, kChainPer = 4, kChainStep = kChainThreads * kChainPer;
-constexpr int kChainWaves = kChainThreads / kWave, kChainSub = kWave * kChainPer;
+// Bounded by the scan's folds and their latency.  Measured over the sums of
+// one GoldenC alternation (2.6e5 to 5.2e5 terms): 63 us for the three
+// launches, against 696 us with one workgroup per sum (4096 terms a step)
+// and 5189 us (13 ns a term) with one wave that added each term from its lane.
+constexpr int kChunk = kWave, kSupChunks = 16, kSup = kChunk * kSupChunks;
+constexpr long long kUnit = (long long)1 << 52, kNoLow = (long long)1 << 61;
 
-struct ChainLds {
-    double term[kChainStep];
-    long long sum[kChainWaves], pos[kChainWaves], low[kChainWaves];   // low: bound of the negative terms, 0 without any
-    int bad[kChainWaves], zero[kChainWaves];
-    double acc;
+struct ChainRec {
+    long long sum, pos, low;   // sum; bounds of the partial sums above and below (kNoLow: no negative term)
+    int key;                   // sign and exponent of the running sum that it is rounded for
+    int flags;                 // REC_BAD: fold term by term; REC_ZERO: all terms are zero
 };
+enum { REC_BAD = 1, REC_ZERO = 2 };
+// Scratch of one sum (sups groups of kSup terms).
+struct ChainBuf {
+    double *terms, *chunk, *sup;   // the terms; plain sums per chunk and per group
+    ChainRec *rec, *srec;
+    int64_t sups;
+};
+struct ChainScratch {
+    ChainBuf c[4];
+};
+
+__device__ __forceinline__ int64_t chain_terms(const ChainSeg &s) { return s.term == CT_NABLA2 ? 2 * s.n : s.n; }
+
+__device__ __forceinline__ double chain_value(const ChainSeg &s, const ChainArgs &a, int64_t e) {
+    double t = 0.0, t1 = 0.0;
+    switch (s.term) {
+        case CT_SQDIFF: chain_term<CT_SQDIFF>(s, a, e, t, t1); return t;
+        case CT_SQ: chain_term<CT_SQ>(s, a, e, t, t1); return t;
+        case CT_DOT: chain_term<CT_DOT>(s, a, e, t, t1); return t;
+        case CT_REG_INT: chain_term<CT_REG_INT>(s, a, e, t, t1); return t;
+        case CT_NV: chain_term<CT_NV>(s, a, e, t, t1); return t;
+        case CT_NABLA2: chain_term<CT_NABLA2>(s, a, e >> 1, t, t1); return e & 1 ? t1 : t;
+        default: chain_term<CT_NDSQ>(s, a, e, t, t1); return t;
+    }
+}
+
+__device__ __forceinline__ bool chain_skip(const ChainArgs &a) {
+    return a.edge_c && (a.sc->edge_done || a.sc->converged);
+}
+
+// Workgroup (x, y): group x of sum y; wave w its chunks 4 w .. 4 w + 3, one
+// term per lane (zeros past the end: adding +0 leaves every running sum but
+// -0 as it is, and the sums start at +0).
+__global__ __launch_bounds__(kBlock) void k_chain_terms(ChainArgs a, ChainScratch q) {
+    __shared__ double lds[kBlock / kWave];
+    if (chain_skip(a)) return;
+    const ChainDesc &c = a.c[blockIdx.y];
+    const ChainBuf &b = q.c[blockIdx.y];
+    const int64_t g = blockIdx.x;
+    if (g >= b.sups) return;
+    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    const int64_t n0 = chain_terms(c.seg[0]), n = n0 + (c.nseg > 1 ? chain_terms(c.seg[1]) : 0);
+    constexpr int PER = kSupChunks / (kBlock / kWave);
+    double t[PER], all = 0.0;
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int64_t e = g * kSup + (wv * PER + k) * kChunk + lane;
+        t[k] = e >= n ? 0.0 : (e < n0 ? chain_value(c.seg[0], a, e) : chain_value(c.seg[1], a, e - n0));
+    }
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int64_t ch = g * kSupChunks + wv * PER + k;
+        b.terms[ch * kChunk + lane] = t[k];
+        const double s = group_sum<kWave>(t[k]);
+        if (lane == 0) b.chunk[ch] = s;
+        all += s;
+    }
+    if (lane == 0) lds[wv] = all;
+    __syncthreads();
+    if (threadIdx.x == 0) b.sup[g] = (lds[0] + lds[1]) + (lds[2] + lds[3]);
+}
 
 __device__ __forceinline__ long long wave_sum_i64(long long x) {
 #pragma unroll
@@ -186,135 +249,141 @@ __device__ __forceinline__ long long wave_sum_i64(long long x) {
     return x;
 }
 
-// The terms of lane slots first .. first + 3 of the segment (zeros past its
-// end; adding +0 leaves every running sum but -0 as it is, and the sums start
-// at +0).
-template <int TERM>
-__device__ __forceinline__ void chain_load(const ChainSeg &s, const ChainArgs &a, int64_t first, double (&t)[kChainPer]) {
-    if constexpr (TERM == CT_NABLA2) {
+__device__ __forceinline__ int chain_key(double acc) { return (int)(__double_as_longlong(acc) >> 52) & 0xfff; }
+// The scale 2^(52 - e) of a running sum of exponent e is a normal number too.
+__device__ __forceinline__ bool chain_normal(int key) { return (key & 0x7ff) >= 53 && (key & 0x7ff) <= 2000; }
+
+__global__ __launch_bounds__(kBlock) void k_chain_records(ChainArgs a, ChainScratch q) {
+    __shared__ double lds[kBlock / kWave];
+    __shared__ ChainRec recs[kSupChunks];
+    if (chain_skip(a)) return;
+    const ChainBuf &b = q.c[blockIdx.y];
+    const int64_t g = blockIdx.x;
+    if (g >= b.sups) return;
+    const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    constexpr int PER = kSupChunks / (kBlock / kWave);
+    double t[PER];
 #pragma unroll
-        for (int k = 0; k < kChainPer; k += 2) {
-            const int64_t e = (first + k) >> 1;
-            t[k] = t[k + 1] = 0.0;
-            if (e < s.n) chain_term<TERM>(s, a, e, t[k], t[k + 1]);
-        }
-    } else {
+    for (int k = 0; k < PER; ++k) t[k] = b.terms[(g * kSupChunks + wv * PER + k) * kChunk + lane];
+    double mine = 0.0;
+    for (int64_t i = threadIdx.x; i < g; i += kBlock) mine += b.sup[i];
+    mine = group_sum<kWave>(mine);
+    if (lane == 0) lds[wv] = mine;
+    __syncthreads();
+    double before = (lds[0] + lds[1]) + (lds[2] + lds[3]);
+    for (int k = 0; k < wv * PER; ++k) before += b.chunk[g * kSupChunks + k];
 #pragma unroll
-        for (int k = 0; k < kChainPer; ++k) {
-            double none = 0.0;
-            t[k] = 0.0;
-            if (first + k < s.n) chain_term<TERM>(s, a, first + k, t[k], none);
+    for (int k = 0; k < PER; ++k) {
+        const int key = chain_key(before);
+        const double scale = __longlong_as_double(((long long)(2098 - (key & 0x7ff)) << 52) | ((long long)(key >> 11) << 63));
+        constexpr double M = 6755399441055744.0;   // 1.5 2^52: adding it rounds to an integer
+        const double x = t[k] * scale, r = x + M;
+        const long long i = __double_as_longlong(r) - __double_as_longlong(M);
+        bool bad = !(fabs(x) < 1125899906842624.0) | (fabs(x - (r - M)) == 0.5) | !chain_normal(key);
+        const bool zero = __all(t[k] == 0.0);
+        bad = __any(bad);
+        ChainRec o{0, 0, kNoLow, key, zero ? REC_ZERO : (bad ? REC_BAD : 0)};
+        if (!zero && !bad) {
+            const long long p = wave_sum_i64(i > 0 ? i : 0), m = __any(x < 0.0) ? wave_sum_i64(i < 0 ? i : 0) : 0;
+            o.sum = p + m;
+            o.pos = p;
+            if (__any(x < 0.0)) o.low = m - kChunk;
+            if (p >= 2 * kUnit || m <= -2 * kUnit) {   // cannot stay in the binade
+                o = ChainRec{0, 0, kNoLow, key, REC_BAD};
+            }
         }
+        if (lane == 0) {
+            b.rec[g * kSupChunks + wv * PER + k] = o;
+            recs[wv * PER + k] = o;
+        }
+        before += b.chunk[g * kSupChunks + wv * PER + k];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {   // the group as one record, if its chunks are of one binade
+        ChainRec o{0, 0, kNoLow, 0, REC_ZERO};
+        for (int k = 0; k < kSupChunks; ++k) {
+            const ChainRec c = recs[k];
+            if (c.flags & REC_ZERO) continue;
+            if (o.flags & REC_ZERO) {
+                o.flags = 0;
+                o.key = c.key;
+            }
+            if ((c.flags & REC_BAD) || c.key != o.key) o.flags = REC_BAD;
+            o.pos = max(o.pos, o.sum + c.pos);
+            if (c.low != kNoLow) o.low = min(o.low, o.sum + c.low);
+            o.sum += c.sum;
+        }
+        if (o.pos >= 2 * kUnit || o.low <= -2 * kUnit) o.flags = REC_BAD;
+        if (o.flags & REC_BAD) o = ChainRec{0, 0, kNoLow, o.key, REC_BAD};
+        b.srec[g] = o;
     }
 }
 
-template <int TERM>
-__device__ double chain_segment(const ChainSeg &s, const ChainArgs &a, double acc, ChainLds &L) {
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
-    const int64_t n = TERM == CT_NABLA2 ? 2 * s.n : s.n;
-    double t[kChainPer], nx[kChainPer];
-    chain_load<TERM>(s, a, (int64_t)tid * kChainPer, t);
-    for (int64_t b0 = 0; b0 < n; b0 += kChainStep) {
-        // the next step's terms load while this one is folded
-        chain_load<TERM>(s, a, b0 + kChainStep + (int64_t)tid * kChainPer, nx);
+// Applies the records of lanes from .. 63 to acc as far as they hold; returns
+// the first lane whose record does not (64: none).
+__device__ __forceinline__ int chain_apply(const ChainRec &r, int from, int lane, double &acc) {
+    const int key = chain_key(acc);
+    const long long bits = __double_as_longlong(acc), A = (bits & (kUnit - 1)) | kUnit;
+    const bool zero = lane < from || (r.flags & REC_ZERO);
+    long long run = zero ? 0 : r.sum;
 #pragma unroll
-        for (int k = 0; k < kChainPer; ++k) L.term[tid * kChainPer + k] = t[k];
-        const int waves = (int)min((int64_t)kChainWaves, (n - b0 + kChainSub - 1) / kChainSub);
-        for (int from = 0; from < waves;) {
-            // acc = +-A 2^(e - 52), 2^52 <= A < 2^53, where e is its exponent
-            const long long bits = __double_as_longlong(acc);
-            const int be = (int)((bits >> 52) & 0x7ff);
-            const bool normal = be >= 53 && be <= 2000;   // the scale 2^(52 - e) is a normal number too
-            const double scale = __longlong_as_double(((long long)(2098 - be) << 52) | (bits & ((long long)1 << 63)));
-            if (wv >= from && wv < waves) {
-                long long p = 0, q = 0;
-                bool bad = false, zero = true, below = false;
-                constexpr double M = 6755399441055744.0;   // 1.5 2^52: adding it rounds to an integer
-#pragma unroll
-                for (int k = 0; k < kChainPer; ++k) {
-                    const double x = t[k] * scale, r = x + M;
-                    const long long i = __double_as_longlong(r) - __double_as_longlong(M);
-                    bad |= !(fabs(x) < 1125899906842624.0) | (fabs(x - (r - M)) == 0.5);
-                    zero &= t[k] == 0.0;
-                    below |= x < 0.0;
-                    p += i > 0 ? i : 0;
-                    q += i < 0 ? i : 0;
-                }
-                bad |= !normal;
-                bad = __any(bad);
-                zero = __all(zero);
-                below = __any(below);
-                if (!bad) {
-                    p = wave_sum_i64(p);
-                    if (below) q = wave_sum_i64(q);
-                }
-                if (lane == 0) {
-                    L.sum[wv] = p + q;
-                    L.pos[wv] = p;
-                    L.low[wv] = below ? q - kChainSub : 0;
-                    L.bad[wv] = bad;
-                    L.zero[wv] = zero;
-                }
-            }
-            __syncthreads();
-            // every thread applies the waves' sums in order
-            constexpr long long kLo = (long long)1 << 52;
-            long long A = (bits & (kLo - 1)) | kLo;
-            int k = from;
-            for (; k < waves; ++k) {
-                if (L.zero[k]) continue;   // +-0 terms leave acc as it is
-                if (L.bad[k] || A + L.pos[k] >= 2 * kLo || (L.low[k] < 0 && A + L.low[k] <= kLo)) break;
-                A += L.sum[k];
-            }
-            if (normal) acc = __longlong_as_double((bits & ~(kLo - 1)) | (A & (kLo - 1)));
-            if (k < waves) {
-                // wave k term by term, by one wave (all lanes alike)
-                if (wv == 0) {
-                    const int m = (int)min((int64_t)kChainSub, n - b0 - (int64_t)k * kChainSub);
-                    const double *q = L.term + k * kChainSub;
-                    int i = 0;
-                    for (; i + 16 <= m; i += 16) {
-                        double x[16];
-#pragma unroll
-                        for (int j = 0; j < 16; ++j) x[j] = q[i + j];
-#pragma unroll
-                        for (int j = 0; j < 16; ++j) acc = acc + x[j];
-                    }
-                    for (; i < m; ++i) acc = acc + q[i];
-                    if (lane == 0) L.acc = acc;
-                }
-                ++k;
-                __syncthreads();
-                acc = L.acc;
-            }
-            from = k;
-            __syncthreads();   // the tables (and, at the end, the terms) are written again
-        }
-#pragma unroll
-        for (int k = 0; k < kChainPer; ++k) t[k] = nx[k];
+    for (int o = 1; o < kWave; o <<= 1) {
+        const long long up = __shfl_up(run, o, kWave);
+        if (lane >= o) run += up;
     }
-    return acc;
+    const long long at = A + run - (zero ? 0 : r.sum);
+    const bool holds = zero || (!(r.flags & REC_BAD) && r.key == key && chain_normal(key) && at + r.pos < 2 * kUnit &&
+                                (r.low == kNoLow || at + r.low > kUnit));
+    const unsigned long long fail = __ballot(!holds);
+    const int f = fail ? __ffsll((long long)fail) - 1 : kWave;
+    const long long to = f < kWave ? __shfl(at, f, kWave) : __shfl(A + run, kWave - 1, kWave);
+    if (chain_normal(key)) acc = __longlong_as_double((bits & ~(kUnit - 1)) | (to & (kUnit - 1)));
+    return f;
 }
 
-// One workgroup per sum.
-__global__ __launch_bounds__(kChainThreads) void k_chains(ChainArgs a) {
-    __shared__ ChainLds L;
-    if (a.edge_c && (a.sc->edge_done || a.sc->converged)) return;
-    const ChainDesc &c = a.c[blockIdx.x];
+// One wave per sum.
+__global__ __launch_bounds__(kWave) void k_chain_scan(ChainArgs a, ChainScratch q) {
+    __shared__ double lt[kSup];
+    if (chain_skip(a)) return;
+    const ChainBuf &b = q.c[blockIdx.x];
+    const int lane = threadIdx.x;
+    const ChainRec none{0, 0, kNoLow, 0, REC_ZERO};
     double acc = 0.0;
-    for (int k = 0; k < c.nseg; ++k) {
-        const ChainSeg &s = c.seg[k];
-        switch (s.term) {
-            case CT_SQDIFF: acc = chain_segment<CT_SQDIFF>(s, a, acc, L); break;
-            case CT_SQ: acc = chain_segment<CT_SQ>(s, a, acc, L); break;
-            case CT_DOT: acc = chain_segment<CT_DOT>(s, a, acc, L); break;
-            case CT_REG_INT: acc = chain_segment<CT_REG_INT>(s, a, acc, L); break;
-            case CT_NV: acc = chain_segment<CT_NV>(s, a, acc, L); break;
-            case CT_NABLA2: acc = chain_segment<CT_NABLA2>(s, a, acc, L); break;
-            default: acc = chain_segment<CT_NDSQ>(s, a, acc, L); break;
+    ChainRec next = lane < b.sups ? b.srec[lane] : none;
+    for (int64_t g0 = 0; g0 < b.sups; g0 += kWave) {
+        const ChainRec r = next;
+        next = g0 + kWave + lane < b.sups ? b.srec[g0 + kWave + lane] : none;
+        for (int from = 0;;) {
+            const int f = chain_apply(r, from, lane, acc);
+            if (f >= kWave) break;
+            // group f chunk by chunk
+            const int64_t g = g0 + f;
+            const ChainRec c = lane < kSupChunks ? b.rec[g * kSupChunks + lane] : none;
+            double t[kSupChunks];
+#pragma unroll
+            for (int k = 0; k < kSupChunks; ++k) t[k] = b.terms[g * kSup + k * kChunk + lane];
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < kSupChunks; ++k) lt[k * kChunk + lane] = t[k];
+            __syncthreads();
+            for (int at = 0;;) {
+                const int k = chain_apply(c, at, lane, acc);
+                if (k >= kWave) break;
+                const double *x = lt + k * kChunk;   // term by term (all lanes alike)
+#pragma unroll 1
+                for (int i = 0; i < kChunk; i += 16) {
+                    double y[16];
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) y[j] = x[i + j];
+#pragma unroll
+                    for (int j = 0; j < 16; ++j) acc = acc + y[j];
+                }
+                at = k + 1;
+            }
+            from = f + 1;
         }
     }
-    if (threadIdx.x == 0) *c.out = acc;
+    if (lane == 0) *a.c[blockIdx.x].out = acc;
 }
 
 // The edge step from its three sums (main.c:329).
@@ -324,9 +393,40 @@ __global__ void k_chain_edge(ChainArgs a) {
     sc->e_c = sc->e_nd / (a.alpha * sc->e_nd2 + a.beta * a.eps * sc->e_nnd + (a.beta / (4 * a.eps)) * sc->e_nd);
 }
 
-void launch_chains(hipStream_t st, const ChainArgs &a) {
+// buf: scratch of the sums, grown as needed (the job's, on its stream).
+void launch_chains(hipStream_t st, const ChainArgs &a, DevBuf<unsigned char> &buf) {
     MI_REQUIRE(a.nchains >= 1 && a.nchains <= 4, MI_E_ARG, "1 to 4 sums per launch");
-    k_chains<<<a.nchains, kChainThreads, 0, st>>>(a);
+    ChainScratch q{};
+    int64_t sups[4] = {}, all = 0, most = 1;
+    for (int i = 0; i < a.nchains; ++i) {
+        int64_t n = 0;
+        for (int k = 0; k < a.c[i].nseg; ++k) n += (a.c[i].seg[k].term == CT_NABLA2 ? 2 : 1) * a.c[i].seg[k].n;
+        sups[i] = std::max<int64_t>(1, (n + kSup - 1) / kSup);
+        all += sups[i];
+        most = std::max(most, sups[i]);
+    }
+    constexpr size_t kPer = sizeof(double) * (kSup + kSupChunks + 1) + sizeof(ChainRec) * (kSupChunks + 1);
+    if (buf.n < all * kPer) buf.alloc(all * kPer);
+    unsigned char *p = buf.p;
+    auto take = [&](size_t bytes) {
+        unsigned char *r = p;
+        p += bytes;
+        return r;
+    };
+    for (int i = 0; i < a.nchains; ++i) {
+        q.c[i].sups = sups[i];
+        q.c[i].terms = (double *)take(sups[i] * kSup * sizeof(double));
+        q.c[i].chunk = (double *)take(sups[i] * kSupChunks * sizeof(double));
+        q.c[i].sup = (double *)take(sups[i] * sizeof(double));
+        q.c[i].rec = (ChainRec *)take(sups[i] * kSupChunks * sizeof(ChainRec));
+        q.c[i].srec = (ChainRec *)take(sups[i] * sizeof(ChainRec));
+    }
+    const dim3 grid((unsigned)most, a.nchains);
+    k_chain_terms<<<grid, kBlock, 0, st>>>(a, q);
+    MI_HIP(hipGetLastError());
+    k_chain_records<<<grid, kBlock, 0, st>>>(a, q);
+    MI_HIP(hipGetLastError());
+    k_chain_scan<<<a.nchains, kWave, 0, st>>>(a, q);
     MI_HIP(hipGetLastError());
     if (a.edge_c) {
         k_chain_edge<<<1, 1, 0, st>>>(a);
@@ -492,7 +592,7 @@ int gc_image_step_ordered(mi_context *ctx, Matrix &m, JobState<double> &js, doub
     auto energy = [&] {
         ca.nchains = 1;
         ca.c[0] = chain(&sc->gen[0], seg(CT_SQDIFF, nrows, js.af.p, js.g.p), seg(CT_REG_INT, nint, js.u.p, js.v.p));
-        launch_chains(st, ca);
+        launch_chains(st, ca, js.chain);
     };
     int reason = 0, ran = 0;
 
@@ -509,7 +609,7 @@ int gc_image_step_ordered(mi_context *ctx, Matrix &m, JobState<double> &js, doub
         ca.c[0] = chain(&sc->gen[3], seg(CT_NV, npix, js.p.p, js.v.p));
         ca.c[1] = chain(&sc->gen[4], seg(CT_DOT, npix, js.p.p, js.d.p));
         ca.c[2] = chain(&sc->gen[2], seg(CT_SQ, nrows, js.q.p));
-        launch_chains(st, ca);
+        launch_chains(st, ca, js.chain);
         h = js.read_scalars(st);
         const double nap = h.gen[2];
         const double c1 = h.gen[4] / (nap + alpha * h.gen[3]);
@@ -548,7 +648,7 @@ int gc_image_step_ordered(mi_context *ctx, Matrix &m, JobState<double> &js, doub
         seq_forward(st, q, js.d.p, js.af.p);
         ca.nchains = 1;
         ca.c[0] = chain(&sc->gen[6], seg(CT_DOT, nrows, js.af.p, js.q.p));
-        launch_chains(st, ca);
+        launch_chains(st, ca, js.chain);
         h = js.read_scalars(st);
         const double c2 = -h.gen[6] / nap;
         launch_xpby<double>(st, npix, js.p.p, js.d.p, c2);
@@ -581,7 +681,7 @@ void gc_edge_step_ordered(mi_context *ctx, JobState<double> &js, double alpha, d
     launch_pass_begin(st, js.sc.p);
     for (int k = 0; k < iter_edge; ++k) {
         launch_edge_grad_n<double>(st, nx, ny, js.u.p, js.v.p, js.d.p, js.w.p, alpha, beta, eps, js.sc.p);
-        launch_chains(st, ca);
+        launch_chains(st, ca, js.chain);
         launch_edge_update<double>(st, js.rb(), nx, ny, js.v.p, js.d.p, js.sc.p);
     }
     MI_HIP(hipStreamSynchronize(st));
