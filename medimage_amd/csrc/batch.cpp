@@ -102,9 +102,6 @@ Batch<T>::Batch(mi_context *c, int n_subsets) : ctx(c), S(n_subsets) {
     MI_HIP(hipMemsetAsync(d_sc.p, 0, d_sc.bytes(), ctx->stream));
     MI_HIP(hipMemcpyAsync(d_jp.p, h_jp.data(), d_jp.bytes(), hipMemcpyHostToDevice, ctx->stream));
     MI_HIP(hipStreamSynchronize(ctx->stream));
-    MI_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
-    MI_HIP(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
-    MI_HIP(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
     t0 = std::chrono::steady_clock::now();
 }
 
@@ -583,7 +580,29 @@ void Batch<T>::rebuild() {
     args.part = d_part.p;
     args.nunits = (int)live.size();
     args.S = S;
+    // The second stream, where a phase has both classes (a stream costs 150 us
+    // to make and give back, a fifth of a 64 x 64 reconstruction's 0.8 ms).
+    if (!side && ((class_fp(0) && class_fp(1)) || (class_bp(0) && class_bp(1)))) {
+        MI_HIP(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
+        MI_HIP(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
+        MI_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
+    }
     dirty = false;
+}
+
+// Whether class c of a phase has launches.  The back projections along lines
+// of the K <= 4 units in one group a block are class 0, all others, smaller
+// images and K = 8, class 1.
+template <typename T>
+bool Batch<T>::class_fp(int c) const {
+    return rows[c].any() || ln[c].any();
+}
+template <typename T>
+bool Batch<T>::class_bp(int c) const {
+    bool y = bpl[c][0].any() || bpl[c][1].any() || bpg[c].any();
+    for (int k = 0; k < 2; ++k)
+        for (int l = 0; l < 3; ++l) y = y || ((c == 0) == (k == 0 && l == 0) && lnb[k][l].any());
+    return y;
 }
 
 // Algorithmic bytes of one launch summed over the live units (instrumented
@@ -620,14 +639,6 @@ void Batch<T>::record_pass(bool timed) {
             if (ln[c].any()) eng_line_fp(q, args, ln[c].map, s, ln[c].kmax, resid);
         }
     };
-    // ... and their back projection: the K <= 4 units in one group a block on
-    // one stream (branch 0), all others, smaller images and K = 8, beside it
-    auto any_lnb = [&](int c) {
-        bool y = false;
-        for (int k = 0; k < 2; ++k)
-            for (int l = 0; l < 3; ++l) y = y || ((c == 0) == (k == 0 && l == 0) && lnb[k][l].any());
-        return y;
-    };
     auto line_bp = [&](hipStream_t q, int c, int s) {
         if constexpr (sizeof(T) == 4) {
             for (int k = 0; k < 2; ++k)
@@ -649,7 +660,7 @@ void Batch<T>::record_pass(bool timed) {
                     line_fp(q, c, s, true);
                 };
             };
-            branches(one(0), one(1), rows[0].any() || ln[0].any(), rows[1].any() || ln[1].any());
+            branches(one(0), one(1), class_fp(0), class_fp(1));
         }
         {
             LaunchTimer lt(ctx, MI_K_BP, sum([&](const Unit<T> &U) {
@@ -663,8 +674,7 @@ void Batch<T>::record_pass(bool timed) {
                     line_bp(q, c, s);
                 };
             };
-            branches(one(0), one(1), bpl[0][0].any() || bpl[0][1].any() || bpg[0].any() || any_lnb(0),
-                     bpl[1][0].any() || bpl[1][1].any() || bpg[1].any() || any_lnb(1));
+            branches(one(0), one(1), class_bp(0), class_bp(1));
         }
         {
             LaunchTimer lt(ctx, MI_K_FPSQ, sum([&](const Unit<T> &U) {
@@ -676,7 +686,7 @@ void Batch<T>::record_pass(bool timed) {
                     line_fp(q, c, s, false);
                 };
             };
-            branches(one(0), one(1), rows[0].any() || ln[0].any(), rows[1].any() || ln[1].any());
+            branches(one(0), one(1), class_fp(0), class_fp(1));
         }
         {
             LaunchTimer lt(ctx, MI_K_STEP, sum([&](const Unit<T> &U) { return 5.0 * U.m->npix * sz * U.K; }));

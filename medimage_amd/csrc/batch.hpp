@@ -134,7 +134,9 @@ struct Batch {
     // 4; K = 1 units share the launch of larger ones, they would only run one
     // after the other).
     Launch rows[2], ln[2], lnb[2][3], bpl[2][2], bpg[2];   // bpl[K class][LDS class]
-    hipStream_t side = nullptr;   // the second class of a phase
+    bool class_fp(int c) const;   // the forward / back projection phase has launches of class c
+    bool class_bp(int c) const;
+    hipStream_t side = nullptr;   // the second class of a phase (made when a phase has both)
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     EngArgs<T> args{};
     int kmax = 1;
