@@ -545,20 +545,18 @@ void Batch<T>::rebuild() {
         D.bs_P = m.bs.P;
         D.job0 = U.uid * kMaxK;
         MI_REQUIRE(m.has_sell && (!f64 || m.has64), MI_E_STATE, "matrix lacks the engine's sliced layout");
+        auto put = [&](BlockMap &map, bool has, int64_t blocks) {
+            map.count[i] = has ? (int)blocks : 0;
+            map.start[i + 1] = map.start[i] + (map.count[i] + 7) / 8 * 8;
+        };
         for (int c = 0; c < 2; ++c) {
-            const int fb = c == rc ? (int)fp_blocks<T>(m) : 0;
-            rows[c].map.start[i + 1] = rows[c].map.start[i] + (lines ? 0 : fb);
-            ln[c].map.start[i + 1] = ln[c].map.start[i] + (lines ? fb : 0);
-            for (int l = 0; l < 2; ++l)
-                bpl[c][l].map.start[i + 1] =
-                    bpl[c][l].map.start[i] + (!lines && in_lds && c == bc && l == lc ? (int)bp_blocks(m) : 0);
-            bpg[c].map.start[i + 1] = bpg[c].map.start[i] + (!lines && !in_lds && c == bc ? (int)bp_blocks(m) : 0);
+            put(rows[c].map, !lines && c == rc, fp_blocks<T>(m));
+            put(ln[c].map, lines && c == rc, fp_blocks<T>(m));
+            for (int l = 0; l < 2; ++l) put(bpl[c][l].map, !lines && in_lds && c == bc && l == lc, bp_blocks(m));
+            put(bpg[c].map, !lines && !in_lds && c == bc, bp_blocks(m));
+            for (int l = 0; l < 3; ++l) put(lnb[c][l].map, lines && c == bc && l == ng, bp_blocks(m));
         }
-        for (int c = 0; c < 2; ++c)
-            for (int l = 0; l < 3; ++l)
-                lnb[c][l].map.start[i + 1] =
-                    lnb[c][l].map.start[i] + (lines && c == bc && l == ng ? (int)bp_blocks(m) : 0);
-        pix.start[i + 1] = pix.start[i] + (int)px_blocks(m);
+        put(pix, true, px_blocks(m));
         kmax = std::max(kmax, U.K);
         all_walk = all_walk && (lines || m.has_otf);
         for (int k = 0; k < U.K; ++k) {

@@ -219,14 +219,25 @@ __device__ __forceinline__ void group_sums(double (&v)[K], int P) {
         for (int j = 0; j < K; ++j) v[j] += __shfl_xor(v[j], o, kWave);
 }
 
-__device__ __forceinline__ int find_unit(const BlockMap &m, int b) {
+// This workgroup's unit and block of it.  Each XCD (workgroups go to the 8
+// XCDs in turn) takes an eighth of every unit's blocks, a contiguous one, unit
+// by unit: units differ tenfold in the cost of a block, and with the whole
+// launch cut into eight runs of blocks some XCDs had the costly units and the
+// others waited (64 slices of 17 geometries, K = 1 to 8: 2385 AT iterations/s,
+// now 3400; eight jobs of two geometries 27.5 and 25.8 ms).  A launch of one
+// unit is cut as before.  False for the padding.
+__device__ __forceinline__ bool unit_block(const BlockMap &m, int &ui, int &lb) {
+    const int x = (int)(blockIdx.x & 7), p = (int)(blockIdx.x >> 3) * 8;
+    if (p >= m.start[m.nunits]) return false;
     int lo = 0, hi = m.nunits;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
-        if (m.start[mid] <= b) lo = mid;
+        if (m.start[mid] <= p) lo = mid;
         else hi = mid;
     }
-    return lo;
+    ui = lo;
+    lb = (x * (m.start[lo + 1] - m.start[lo]) + (p - m.start[lo])) / 8;
+    return lb < m.count[lo];
 }
 
 template <typename T>
@@ -1715,24 +1726,20 @@ template <typename T, int KMAX, bool RESID, int FM>
 __global__ __launch_bounds__(kBlock) void k_eng_fp(EngArgs<T> a, BlockMap m, int s) {
     __shared__ double lds[kBlock / kWave * kMaxK];
     __shared__ double ldr[kBlock / kOtfPerWave * KMAX];
-    const int b = (int)xcd_block();
-    if (b >= m.start[m.nunits]) return;
-    const int ui = find_unit(m, b);
+    int ui, lb;
+    if (!unit_block(m, ui, lb)) return;
     const UG<T> U(a.units[ui]);
     if (unit_idle(a, U)) return;
-    const int lb = b - m.start[ui];
     MI_KSWITCH(KMAX, (fp_unit<T, K, RESID, FM>(a, U, s, lb, lds, ldr)))
 }
 
 template <int KMAX, bool RESID>
 __global__ __launch_bounds__(kLineBlock) void k_line_fp(EngArgs<float> a, BlockMap m, int s) {
     __shared__ double lds[kLineWaves * KMAX * kLineRays];
-    const int b = (int)xcd_block();
-    if (b >= m.start[m.nunits]) return;
-    const int ui = find_unit(m, b);
+    int ui, lb;
+    if (!unit_block(m, ui, lb)) return;
     const UG<float> U(a.units[ui]);
     if (unit_idle(a, U)) return;
-    const int lb = b - m.start[ui];
     MI_KSWITCH(KMAX, (line_fp_unit<K, RESID>(a, U, s, lb, lds)))
 }
 
@@ -1740,12 +1747,10 @@ template <int KMAX, int P>
 __global__ __launch_bounds__(P * kBlock) void k_line_bp(EngArgs<float> a, BlockMap m, int s, int cap) {
     __shared__ double lds[kBlock / kWave * kMaxK];
     extern __shared__ __align__(16) unsigned char ldr_raw[];
-    const int b = (int)xcd_block();
-    if (b >= m.start[m.nunits]) return;
-    const int ui = find_unit(m, b);
+    int ui, lb;
+    if (!unit_block(m, ui, lb)) return;
     const UG<float> U(a.units[ui]);
     if (unit_idle(a, U)) return;
-    const int lb = b - m.start[ui];
     MI_KSWITCH(KMAX, (line_bp_unit<K, P>(a, U, s, lb, cap, lds, (LDSP unsigned char *)ldr_raw)))
 }
 
@@ -1753,12 +1758,10 @@ template <typename T, int KMAX, bool LDS, bool SQ>
 __global__ __launch_bounds__(kBlock) void k_eng_bp(EngArgs<T> a, BlockMap m, int s, int sq_off) {
     __shared__ double lds[kBlock / kWave * kMaxK];
     extern __shared__ __align__(16) unsigned char ldr_raw[];   // LDS: the block's residual slots
-    const int b = (int)xcd_block();
-    if (b >= m.start[m.nunits]) return;
-    const int ui = find_unit(m, b);
+    int ui, lb;
+    if (!unit_block(m, ui, lb)) return;
     const UG<T> U(a.units[ui]);
     if (unit_idle(a, U)) return;
-    const int lb = b - m.start[ui];
     MI_KSWITCH(KMAX, (bp_unit<T, K, LDS, SQ>(a, U, s, lb, lds, (LDSP T *)ldr_raw, sq_off)))
 }
 
@@ -1933,12 +1936,10 @@ __global__ __launch_bounds__(kBlock) void k_eng_pix(EngArgs<T> a, BlockMap m, in
     // direction)
     constexpr int kStrips = OP == PX_EDGE_GRAD ? 2 : (OP == PX_MEDIAN || OP == PX_EDGE_NABLA || OP == PX_NV ? 1 : 0);
     __shared__ __align__(16) T L[kStrips ? kStrips * kHaloN * KMAX : 1];
-    const int b = (int)xcd_block();
-    if (b >= m.start[m.nunits]) return;
-    const int ui = find_unit(m, b);
+    int ui, lb;
+    if (!unit_block(m, ui, lb)) return;
     const UG<T> U(a.units[ui]);
     if (unit_idle(a, U)) return;
-    const int lb = b - m.start[ui];
     if constexpr (OP == PX_AXPY) { MI_KSWITCH(KMAX, (axpy_unit<T, K>(a, U, lb))) }
     else if constexpr (OP == PX_MEDIAN) { MI_KSWITCH(KMAX, (median_unit<T, K>(a, U, lb, L))) }
     else if constexpr (OP == PX_NV) { MI_KSWITCH(KMAX, (nv_unit<T, K>(a, U, lb, lds, L))) }

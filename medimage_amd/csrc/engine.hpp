@@ -106,7 +106,8 @@ struct UnitDesc {
 // Block ranges of one launch: unit u owns blocks [start[u], start[u+1]).
 struct BlockMap {
     int nunits;
-    int start[kMaxUnits + 1];
+    int start[kMaxUnits + 1];   // each unit's blocks, a multiple of 8
+    int count[kMaxUnits];       // ... of which it has
 };
 
 // Arguments common to the engine's launches.
