@@ -317,7 +317,9 @@ void build_sell(Matrix &m, hipStream_t st, bool drop_csr = false);
 // Builds the matrix for (g, S) on the stream; want64 also keeps double
 // lengths.  Host-side GoldenC walk for MI_BEAM_GOLDENC, device tracers
 // otherwise.
-// otf: also record the checkpointed forward walk (fan beam only).
+// layout as make_key's: 1 builds a fan beam's lines, which are all that FP32
+// then needs (has_csr false), else the checkpointed walk as well; 2 stops
+// behind the lines.
 std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, hipStream_t st, int layout = 0);
 // Subset order: bit-reversed subset indices (values >= S dropped).
 std::vector<int> subset_order(int S);
