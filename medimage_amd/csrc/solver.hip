@@ -42,12 +42,17 @@ CscView csc_view(const Matrix &m, int s, bool f64) {
 
 // Lanes per pixel column of the gather back projector: each lane takes four
 // entries per trip; aim at about three trips over the subset's mean column
-// length, within [4, 64].
+// length, within [4, 16].  At most 16: the four neighbouring pixels of a wave
+// then meet neighbouring rays, so that their gathers share lines.  A call with
+// 16 / 32 / 64 lanes: 400 x 400, 720 views FP64 1211 / 1307 / 3291 us; 300 x
+// 300, 359 views FP64 389 / 409 / 436; 120 x 120, 180 views FP64 74 / 76 / 80;
+// 512 x 512, 720 views FP32 1379 / 1510 / 1720; 60 x 60, 700 views FP64 85 / 79
+// / 84.
 int bp_lanes(const Matrix &m) {
     if (m.tune.bp_lanes) return m.tune.bp_lanes;
     const double mean = (double)m.nnz / ((double)m.S * (double)m.npix);
     int l = 4;
-    while (l < 64 && l * 12 < mean) l *= 2;
+    while (l < 16 && l * 12 < mean) l *= 2;
     return l;
 }
 
