@@ -1887,8 +1887,12 @@ __device__ __forceinline__ void fin_job(const EngArgs<T> &a, const UG<T> &U, int
             break;
         }
         case EF_EDGE_DONE:
-        case EF_EDGE_END:
-            if (!sc->edge_done && s < P.iter_edge) {
+        case EF_EDGE_END: {
+            // every wave has read the flag before EF_END below clears it
+            // (without the reduction no barrier stands between the two)
+            const bool stopped = sc->edge_done;
+            __syncthreads();
+            if (!stopped && s < P.iter_edge) {
                 const double mx = fin_reduce(part_at(a, U, SL_E3, j), npx, true, lds);
                 if (threadIdx.x == 0) {
                     sc->e_maxcd = mx;
@@ -1897,6 +1901,7 @@ __device__ __forceinline__ void fin_job(const EngArgs<T> &a, const UG<T> &U, int
             }
             if (op == EF_EDGE_DONE) break;
             [[fallthrough]];
+        }
         default: {  // EF_END
             if (threadIdx.x != 0) return;
             const double df = sc->df_pass;
