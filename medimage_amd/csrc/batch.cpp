@@ -468,8 +468,8 @@ void Batch<T>::rebuild() {
             D.ln_mb = m.lines.mb.p;
             D.ln_len = m.lines.len.p;
             D.ln_inv = m.lines.inv.p;
-            D.ln_dlen = m.lines.dlen.p;
             D.ln_drop = m.lines.drop.p;
+            D.ln_skip = m.lines.skip.p;
             D.ln_rng = m.lines.rng.p;
             D.ln_mx = m.lines.mx.p;
             D.ln_my = m.lines.my.p;

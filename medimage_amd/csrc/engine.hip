@@ -55,8 +55,8 @@ struct UG {
     const GL int32_t *ot_cx, *ot_cy, *ot_sg, *ot_cnt;
     const GL int64_t *ln_slice0;
     const GL double *ln_mb, *ln_len;
-    const GL float *ln_inv, *ln_dlen;
-    const GL int32_t *ln_drop, *ln_rng;
+    const GL double *ln_inv;
+    const GL int32_t *ln_drop, *ln_skip, *ln_rng;
     const GL double *ln_mx, *ln_my;
     const GL float *ln_ix, *ln_iy;
     const GL int64_t *ln_win0;
@@ -81,8 +81,8 @@ struct UG {
           ot_cx((const GL int32_t *)D.ot_cx), ot_cy((const GL int32_t *)D.ot_cy),
           ot_sg((const GL int32_t *)D.ot_sg), ot_cnt((const GL int32_t *)D.ot_cnt),
           ln_slice0((const GL int64_t *)D.ln_slice0), ln_mb((const GL double *)D.ln_mb),
-          ln_len((const GL double *)D.ln_len), ln_inv((const GL float *)D.ln_inv), ln_dlen((const GL float *)D.ln_dlen),
-          ln_drop((const GL int32_t *)D.ln_drop), ln_rng((const GL int32_t *)D.ln_rng), ln_mx((const GL double *)D.ln_mx),
+          ln_len((const GL double *)D.ln_len), ln_inv((const GL double *)D.ln_inv),
+          ln_drop((const GL int32_t *)D.ln_drop), ln_skip((const GL int32_t *)D.ln_skip), ln_rng((const GL int32_t *)D.ln_rng), ln_mx((const GL double *)D.ln_mx),
           ln_my((const GL double *)D.ln_my), ln_ix((const GL float *)D.ln_ix), ln_iy((const GL float *)D.ln_iy),
           ln_win0((const GL int64_t *)D.ln_win0), ln_views((const GL int32_t *)D.ln_views),
           sub_row0((const GL int64_t *)D.sub_row0), g((GL T *)D.g), r((GL T *)D.r), u((GL T *)D.u),
@@ -637,14 +637,19 @@ __device__ __forceinline__ void fp_unit(const EngArgs<T> &a, const UG<T> &U, int
 // waves cut the lines the group crosses into as many runs, one lane per ray.
 // At line a of the dominant axis a ray covers at most two neighbouring pixels
 // of that line, so a step is one 2K-value load from the projection image that
-// holds the line contiguously and the interpolation
+// holds the line contiguously and the two products
 //   w u[j] + (1 - w) u[j - 1],   w = min(1, frac(hi) / |m|),
-// with hi the upper end of the covered interval, j = floor(hi).  hi advances
+// with hi the upper end of the covered interval, j = floor(hi).  Weights and
+// products are double: a pixel that the ray does not meet has weight 0 or 1 - w
+// = 0 exactly and adds nothing, however large it is (as a difference in FP32 it
+// left 2^-24 of itself in the ray).  hi advances
 // by m, one double add, and is biased by 2^20 + 2^19 so that its low word is
 // frac(hi) 2^32 and its high word j plus a constant (rounded to 2^-33 pixel a
 // step, under 2^-24 over a run of 512 lines).  Positions outside the image
 // read the zero padding.  The run's sum is double; a ray's runs are added in
-// order, times the ray's length per line, less the piece the tracer drops.
+// order, times the ray's length per line.  The line in which the tracer leaves
+// out a piece (Lines) is not part of the runs: its other pixel is added last
+// (line_kept).
 //
 // What bounds it: the load, 17 accesses of the CU's L1 a line (four lanes an
 // access), beside 10 VALU instructions; a line brings the two pixels' entries
@@ -672,39 +677,47 @@ __device__ __forceinline__ void load_pair(__amdgpu_buffer_rsrc_t rs, uint32_t of
     }
 }
 
-// Adds this lane's ray over lines c0 .. c0 + n - 1 (n a multiple of 8) to acc.
+// Adds this lane's ray over lines c0 .. c0 + n - 1 (n a multiple of 8), without
+// line `skip`, to acc.
 template <int K>
 __device__ __forceinline__ void line_run(const GL float *img, int na, int nb, int c0, int n, double m, double b0,
-                                         float inv, double (&acc)[K]) {
+                                         double inv, int skip, double (&acc)[K]) {
     constexpr int OS = K <= 2 ? 8 : (K == 4 ? 4 : 2);
     const uint32_t lineb = (uint32_t)line_stride(nb) * K * 4;
     const __amdgpu_buffer_rsrc_t rs = make_rsrc((const void *)img, (uint32_t)line_elems(na, nb) * K * 4);
     double hi = b0 + 0.5 * fabs(m) + m * c0 + kLineBias;
-    const float sc = inv * 2.3283064365386963e-10f;   // 2^-32
+    const double sc = inv * 2.3283064365386963e-10;   // 2^-32
     uint32_t at = (uint32_t)c0 * lineb;
-    auto stage = [&](float (&w)[OS], float (&x)[OS][2 * K]) {
+    skip -= c0;
+    auto stage = [&](double (&w)[OS], float (&x)[OS][2 * K]) {
         uint32_t off[OS];
 #pragma unroll
         for (int k = 0; k < OS; ++k) {
             const int h = __double2hiint(hi);
-            w[k] = __builtin_amdgcn_fmed3f((float)(uint32_t)__double2loint(hi) * sc, 0.0f, 1.0f);
+            w[k] = fmin((double)(uint32_t)__double2loint(hi) * sc, 1.0);
             const int j = max(kLineHi0 - 1, min(h, kLineHi0 + nb + 1));   // zeros beyond
             off[k] = (uint32_t)(j - (kLineHi0 - 1)) * (4 * K);            // pixel j - 1, behind two of padding
             hi += m;
         }
+        if (__any((unsigned)skip < (unsigned)OS))
+#pragma unroll
+            for (int k = 0; k < OS; ++k) off[k] = skip == k ? 0u : off[k];   // zeros
+        skip -= OS;
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int k = 0; k < OS; ++k) load_pair<K>(rs, off[k], (int)(at + k * lineb), x[k]);
         at += OS * lineb;
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto consume = [&](const float (&w)[OS], const float (&x)[OS][2 * K]) {
+    auto consume = [&](const double (&w)[OS], const float (&x)[OS][2 * K]) {
 #pragma unroll
         for (int k = 0; k < OS; ++k)
 #pragma unroll
-            for (int j = 0; j < K; ++j) acc[j] += (double)__builtin_fmaf(w[k], x[k][K + j] - x[k][j], x[k][j]);
+            for (int j = 0; j < K; ++j)
+                acc[j] = __builtin_fma(w[k], (double)x[k][K + j], __builtin_fma(1.0 - w[k], (double)x[k][j], acc[j]));
     };
-    float wa[OS], wb[OS], xa[OS][2 * K], xb[OS][2 * K];
+    double wa[OS], wb[OS];
+    float xa[OS][2 * K], xb[OS][2 * K];
     const int ng = n / OS;
     stage(wa, xa);
     int g = 1;
@@ -723,6 +736,44 @@ __device__ __forceinline__ void line_run(const GL float *img, int na, int nb, in
     }
 }
 
+// Pixels j - 1 and j of line a that the ray (m, b0, inv) meets, and j's share.
+__device__ __forceinline__ int line_at(double m, double b0, double inv, int a, int nb, double &w) {
+    const double pos = b0 + 0.5 * fabs(m) + m * a, jf = floor(pos);
+    w = fmin(1.0, (pos - jf) * inv);
+    return (int)fmin(fmax(jf, -1.0), (double)(nb + 1));
+}
+
+// Value k of the K interleaved ones of the ray's left-out line, over the ray's
+// length per line: the pixel of the line that is not `drop`.  img: px or py, by
+// the ray's axis (yd: columns), lines of nb pixels.
+__device__ __forceinline__ double line_kept(const GL float *img, int nb, int ny, bool yd, double m, double b0, double inv,
+                                            int drop, int K, int k) {
+    const int i = drop / ny, jy = drop - i * ny, a = yd ? jy : i, gone = yd ? i : jy;
+    double w;
+    const int j = line_at(m, b0, inv, a, nb, w);
+    const GL float *p = img + ((int64_t)a * line_stride(nb) + j - 1 + kLinePad) * K + k;
+    return j == gone ? (1.0 - w) * (double)p[0] : j - 1 == gone ? w * (double)p[K] : (1.0 - w) * (double)p[0] + w * (double)p[K];
+}
+
+// The sum over lines r0 .. r1 - 1 again where it is not finite: some pixel beside the
+// ray, or its left-out one, may not be (0 times it is not 0).  Only what the
+// ray crosses counts.
+__device__ __forceinline__ double line_ray_again(const GL float *img, int nb, int ny, bool yd, double m, double b0, double inv,
+                                                 int r0, int r1, int drop, int K, int k) {
+    double tot = 0.0;
+    for (int a = r0; a < r1; ++a) {
+        double w;
+        const int j = line_at(m, b0, inv, a, nb, w);
+        for (int h = 0; h < 2; ++h) {   // pixels j - 1 and j of the line (both may be padding)
+            const int jj = j - 1 + h;
+            const double part = h ? w : 1.0 - w;
+            const bool gone = drop >= 0 && drop == (yd ? jj * ny + a : a * ny + jj) && jj >= 0 && jj < nb;
+            if (!gone && part > 1e-6) tot += part * (double)img[((int64_t)a * line_stride(nb) + jj + kLinePad) * K + k];
+        }
+    }
+    return tot;
+}
+
 // RESID: r = g - A u, stored times the ray's length per line (what the back
 // projection weighs), partial sum r^2; else partial sum (A d)^2.
 template <int K, bool RESID>
@@ -734,13 +785,14 @@ __device__ __forceinline__ void line_fp_unit(const EngArgs<float> &a, const UG<f
     const int view = lb / per, bin = (lb - view * per) * kLineRays + lane;
     const int64_t row = U.sub_row0[s] + (int64_t)view * U.nbins + bin;
     const GL int32_t *rng = U.ln_rng + 4 * (g0 + lb);
-    double m = 0.0, b0 = 0.0;
-    float inv = 0.0f;
+    double m = 0.0, b0 = 0.0, inv = 0.0;
+    int skip = -1;
     const bool valid = bin < U.nbins;
     if (valid) {
         m = U.ln_mb[2 * row];
         b0 = U.ln_mb[2 * row + 1];
         inv = U.ln_inv[row];
+        skip = U.ln_skip[row];
     }
     double acc[K];
 #pragma unroll
@@ -753,9 +805,9 @@ __device__ __forceinline__ void line_fp_unit(const EngArgs<float> &a, const UG<f
         // there (its rays have left the image)
         const int run = ((r1 - r0 + kLineWaves - 1) / kLineWaves + 7) & ~7, c0 = r0 + wv * run;
         if (c0 >= r1) continue;
-        const bool mine = valid && (inv < 0.0f) == (ax == 1);
+        const bool mine = valid && (inv < 0.0) == (ax == 1);
         line_run<K>(ax ? U.py : U.px, ax ? U.ny : U.nx, ax ? U.nx : U.ny, c0, min(run, (r1 - c0 + 7) & ~7),
-                    mine ? m : 0.0, mine ? b0 : -64.0, mine ? fabsf(inv) : 0.0f, acc);
+                    mine ? m : 0.0, mine ? b0 : -64.0, mine ? fabs(inv) : 0.0, mine ? skip : -1, acc);
     }
     // thread (job k, ray): the ray's runs in order
 #pragma unroll
@@ -768,12 +820,14 @@ __device__ __forceinline__ void line_fp_unit(const EngArgs<float> &a, const UG<f
     double mm = 0.0;
     if (valid) {
         const double len = U.ln_len[row];
+        const bool yd = inv < 0.0;
+        const GL float *img = yd ? U.py : U.px;
+        const int nb = yd ? U.nx : U.ny, drop = skip >= 0 ? U.ln_drop[row] : -1;
+        if (skip >= 0) tot += line_kept(img, nb, U.ny, yd, m, b0, fabs(inv), drop, K, wv);
+        if (!(fabs(tot) < INFINITY))
+            tot = line_ray_again(img, nb, U.ny, yd, m, b0, fabs(inv), rng[2 * yd], min(rng[2 * yd + 1], yd ? U.ny : U.nx),
+                                 drop, K, wv);
         tot *= len;
-        const int dp = U.ln_drop[row];
-        if (dp >= 0) {
-            const int i = dp / U.ny, j = dp - i * U.ny;
-            tot -= (double)U.ln_dlen[row] * (double)U.px[((int64_t)i * line_stride(U.ny) + j + kLinePad) * K + wv];
-        }
         if (RESID) {
             const double res = (double)U.g[row * K + wv] - tot;
             U.r[row * K + wv] = (float)(res * len);
@@ -809,8 +863,8 @@ __global__ __launch_bounds__(kBlock) void k_line_planes(const float *__restrict_
 // and 3.2e-8.
 __global__ __launch_bounds__(kLineBlock) void k_line_project(
     const float *px, const float *py, int nx, int ny, int nbins, int64_t groups, const double2 *__restrict__ mb,
-    const float *__restrict__ rinv, const double *__restrict__ rlen, const int32_t *__restrict__ drop,
-    const float *__restrict__ dlen, const int4 *__restrict__ rng, float *__restrict__ sino) {
+    const double *__restrict__ rinv, const double *__restrict__ rlen, const int32_t *__restrict__ rdrop,
+    const int32_t *__restrict__ rskip, const int4 *__restrict__ rng, float *__restrict__ sino) {
     __shared__ double lds[kLineWaves][kLineRays];
     const int lane = threadIdx.x & (kWave - 1), wv = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int64_t lb = xcd_block();
@@ -820,12 +874,13 @@ __global__ __launch_bounds__(kLineBlock) void k_line_project(
     const int bin = (int)(lb - view * per) * kLineRays + lane;
     const int64_t row = view * nbins + bin;
     const bool valid = bin < nbins;
-    double m = 0.0, b0 = 0.0, acc[1] = {0.0};
-    float inv = 0.0f;
+    double m = 0.0, b0 = 0.0, inv = 0.0, acc[1] = {0.0};
+    int skip = -1;
     if (valid) {
         m = mb[row].x;
         b0 = mb[row].y;
         inv = rinv[row];
+        skip = rskip[row];
     }
     const int4 r = rng[lb];
 #pragma unroll
@@ -834,9 +889,9 @@ __global__ __launch_bounds__(kLineBlock) void k_line_project(
         if (r0 >= r1) continue;
         const int run = ((r1 - r0 + kLineWaves - 1) / kLineWaves + 7) & ~7, c0 = r0 + wv * run;
         if (c0 >= r1) continue;
-        const bool mine = valid && (inv < 0.0f) == (ax == 1);
+        const bool mine = valid && (inv < 0.0) == (ax == 1);
         line_run<1>((const GL float *)(ax ? py : px), ax ? ny : nx, ax ? nx : ny, c0, min(run, (r1 - c0 + 7) & ~7),
-                    mine ? m : 0.0, mine ? b0 : -64.0, mine ? fabsf(inv) : 0.0f, acc);
+                    mine ? m : 0.0, mine ? b0 : -64.0, mine ? fabs(inv) : 0.0, mine ? skip : -1, acc);
     }
     lds[wv][lane] = acc[0];
     __syncthreads();
@@ -844,31 +899,13 @@ __global__ __launch_bounds__(kLineBlock) void k_line_project(
     double tot = 0.0;
 #pragma unroll
     for (int w = 0; w < kLineWaves; ++w) tot += lds[w][lane];
-    const double len = rlen[row];
-    const int dp = drop[row];
-    tot *= len;
-    if (dp >= 0) tot -= (double)dlen[row] * (double)px[(int64_t)(dp / ny) * line_stride(ny) + dp % ny + kLinePad];
-    if (!(fabs(tot) < INFINITY)) {
-        // Some pixel beside the ray or of its dropped piece may not be finite
-        // (weight 0 times it is not 0): only what the ray crosses counts.
-        const bool ay = inv < 0.0f;
-        const float *p = ay ? py : px;
-        const int nb = ay ? nx : ny, r0 = ay ? r.z : r.x, r1 = min(ay ? r.w : r.y, ay ? ny : nx);
-        tot = 0.0;
-        for (int a = r0; a < r1; ++a) {
-            const double pos = b0 + 0.5 * fabs(m) + m * a, jf = floor(pos);
-            if (!(jf >= 0.0 && jf <= (double)nb)) continue;
-            const int j = (int)jf;
-            const double w = fmin(1.0, (pos - jf) * (double)fabsf(inv));
-            for (int h = 0; h < 2; ++h) {   // pixels j - 1 and j of the line (both may be padding)
-                const int jj = j - 1 + h;
-                double part = (h ? w : 1.0 - w) * len;
-                if (dp == (ay ? jj * ny + a : a * ny + jj) && jj >= 0 && jj < nb) part -= (double)dlen[row];
-                if (part > 1e-6 * len) tot += part * (double)p[(int64_t)a * line_stride(nb) + jj + kLinePad];
-            }
-        }
-    }
-    sino[row] = (float)tot;
+    const bool yd = inv < 0.0;
+    const GL float *img = (const GL float *)(yd ? py : px);
+    const int nb = yd ? nx : ny, drop = skip >= 0 ? rdrop[row] : -1;
+    if (skip >= 0) tot += line_kept(img, nb, ny, yd, m, b0, fabs(inv), drop, 1, 0);
+    if (!(fabs(tot) < INFINITY))
+        tot = line_ray_again(img, nb, ny, yd, m, b0, fabs(inv), yd ? r.z : r.x, min(yd ? r.w : r.y, yd ? ny : nx), drop, 1, 0);
+    sino[row] = (float)(tot * rlen[row]);
 }
 
 // K interleaved values at pixel (i, j), or `pad` outside the image.
@@ -2147,7 +2184,7 @@ void line_project(hipStream_t st, const Matrix &m, const float *img, float *px, 
     k_line_planes<<<grid_of(line_elems(g.nx, g.ny) + line_elems(g.ny, g.nx)), kBlock, 0, st>>>(img, g.nx, g.ny, px, py);
     MI_HIP(hipGetLastError());
     k_line_project<<<grid8((int)groups), kLineBlock, 0, st>>>(px, py, g.nx, g.ny, g.n_bins, groups, q.mb.p, q.inv.p, q.len.p,
-                                                              q.drop.p, q.dlen.p, q.rng.p, sino);
+                                                              q.drop.p, q.skip.p, q.rng.p, sino);
     MI_HIP(hipGetLastError());
 }
 

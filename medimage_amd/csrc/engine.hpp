@@ -79,9 +79,8 @@ struct UnitDesc {
     // rays as lines (FP32 fan beams; null otherwise), see Lines
     const int64_t *ln_slice0;
     const double2 *ln_mb;
-    const double *ln_len;
-    const float *ln_inv, *ln_dlen;
-    const int32_t *ln_drop;
+    const double *ln_len, *ln_inv;
+    const int32_t *ln_drop, *ln_skip;
     const int4 *ln_rng;
     const double2 *ln_mx, *ln_my;
     const float *ln_ix, *ln_iy;

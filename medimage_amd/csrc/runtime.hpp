@@ -159,8 +159,8 @@ struct Otf {
 // and meets at most two pixels.  The length in pixel (a, j) is
 //   len * min(1, max(0, ((1 + |m|) / 2 - |b0 + m a - j - 1/2|) / |m|)),
 // the tracer's own length up to its rounding, except that the tracer leaves
-// out a piece that begins within 0.05 mm of the exit: that pixel and length
-// are kept per ray (drop / dlen; at most one for pixels above 0.05 mm).
+// out a piece that begins within 0.05 mm of the exit: that pixel and its line
+// are kept per ray (drop / skip; at most one for pixels above 0.05 mm).
 // build_lines walks every ray with the tracer and checks each piece against
 // this form; a geometry where one differs keeps the stored matrix.
 //
@@ -201,9 +201,9 @@ struct Lines {
     DevBuf<int64_t> d_slice0;
     DevBuf<double2> mb;              // per row: m, b0
     DevBuf<double> len;              // per row: mm per line of the dominant axis (0: misses the image)
-    DevBuf<float> inv;               // per row: 1 / |m| (1e30 for a ray along the axis), negative when the axis is y
+    DevBuf<double> inv;              // per row: 1 / |m| (1e30 for a ray along the axis), negative when the axis is y
     DevBuf<int32_t> drop;            // per row: pixel (x ny + y) whose piece is left out, -1: none
-    DevBuf<float> dlen;              // per row: its length
+    DevBuf<int32_t> skip;            // per row: that pixel's line along the axis, -1: none
     DevBuf<int4> rng;                // per group: lines its x-dominant rays cross [x, y), its y-dominant ones [z, w)
     // Back projection.  The lines along x and along y of every ray (a ray far
     // from that axis, or past the view's last bin: weight 0 everywhere), views
@@ -222,7 +222,7 @@ struct Lines {
     int arc = 0;
     float sod = 0.f, k = 0.f, bin0 = 0.f;
     size_t bytes() const {
-        return d_slice0.bytes() + mb.bytes() + len.bytes() + inv.bytes() + drop.bytes() + dlen.bytes() + rng.bytes() +
+        return d_slice0.bytes() + mb.bytes() + len.bytes() + inv.bytes() + drop.bytes() + skip.bytes() + rng.bytes() +
                mx.bytes() + my.bytes() + ix.bytes() + iy.bytes() + d_win0.bytes() + views.bytes();
     }
 };

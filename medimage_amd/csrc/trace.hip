@@ -395,8 +395,8 @@ struct LineOut {
     double2 *mb, *mx, *my;
     float *ix, *iy;
     double *len;
-    float *inv, *dlen;
-    int32_t *drop;
+    double *inv;
+    int32_t *drop, *skip;
     int4 *rng;
     unsigned *bad;
     unsigned long long *nnz;   // per subset: the tracer's entries
@@ -420,8 +420,7 @@ __global__ __launch_bounds__(kLineRays) void k_lines_fill(TraceArgs a, const int
         ray_endpoints(g, a.fcos[view], a.fsin[view], a.dcos, a.dsin, bin, sx, sy, dx, dy);
         const double rx = dx - sx, ry = dy - sy, L = sqrt(rx * rx + ry * ry);
         double m = 0.0, b0 = -64.0, len = 0.0, inv = 1e30;
-        int drop = -1;
-        float dlen = 0.0f;
+        int drop = -1, skip = -1;
         SiddonState st;
         if (siddon_init(sx, sy, dx, dy, g.nx, g.ny, g.vx, g.vy, st)) {
             yd = fabs(ry) > fabs(rx);
@@ -462,7 +461,7 @@ __global__ __launch_bounds__(kLineRays) void k_lines_fill(TraceArgs a, const int
                     bad |= !(fabs(w - rem) <= 1e-5 * v);
                     if (w > 0.0) {
                         drop = st.cx * g.ny + st.cy;
-                        dlen = (float)w;
+                        skip = yd ? st.cy : st.cx;
                     }
                 } else {
                     bad |= rem > 1e-5 * v;
@@ -471,9 +470,9 @@ __global__ __launch_bounds__(kLineRays) void k_lines_fill(TraceArgs a, const int
         }
         o.mb[row] = make_double2(m, b0);
         o.len[row] = len;
-        o.inv[row] = yd ? -(float)inv : (float)inv;
+        o.inv[row] = yd ? -inv : inv;
         o.drop[row] = drop;
-        o.dlen[row] = dlen;
+        o.skip[row] = skip;
         // Both lines.  Turned, m -> 1 / m: the length in a pixel stays len times
         // min(1, max(0, ((1 + |m|) / 2 - |..|) / min(1, |m|))) with |m| > 1.  Only
         // rays near the diagonal are looked at along their other axis.
@@ -631,7 +630,7 @@ bool try_lines(Matrix &m, const TraceArgs &a, hipStream_t st) {
     q.len.alloc(m.nrows);
     q.inv.alloc(m.nrows);
     q.drop.alloc(m.nrows + kLineEmpty);   // read past a view's last bin
-    q.dlen.alloc(m.nrows);
+    q.skip.alloc(m.nrows);
     q.rng.alloc(groups);
     for (auto *b : {&q.mx, &q.my}) b->alloc(entries);
     for (auto *b : {&q.ix, &q.iy}) b->alloc(entries);
@@ -652,7 +651,7 @@ bool try_lines(Matrix &m, const TraceArgs &a, hipStream_t st) {
     MI_HIP(hipMemsetAsync(q.views.p, 0, q.views.bytes(), st));
     DevBuf<unsigned long long> nnz(m.S);
     MI_HIP(hipMemsetAsync(nnz.p, 0, nnz.bytes(), st));
-    const LineOut o{q.mb.p, q.mx.p, q.my.p, q.ix.p, q.iy.p, q.len.p, q.inv.p, q.dlen.p, q.drop.p, q.rng.p,
+    const LineOut o{q.mb.p, q.mx.p, q.my.p, q.ix.p, q.iy.p, q.len.p, q.inv.p, q.drop.p, q.skip.p, q.rng.p,
                     (unsigned *)flags.p, nnz.p};
     k_lines_fill<<<(unsigned)groups, kLineRays, 0, st>>>(a, m.d_sub_row0.p, q.d_slice0.p, m.S, o);
     MI_HIP(hipGetLastError());
