@@ -652,13 +652,14 @@ __device__ __forceinline__ void fp_unit(const EngArgs<T> &a, const UG<T> &U, int
 // (line_kept).
 //
 // What bounds it: the load, 17 accesses of the CU's L1 a line (four lanes an
-// access), beside 10 VALU instructions; a line brings the two pixels' entries
+// access), beside 11 VALU instructions, eight of them on doubles at half rate; a
+// line brings the two pixels' entries
 // (1.4 entries of the matrix on average), where the checkpointed walk spends 26
 // VALU instructions and such a load on each entry.  512 x 512 pixels, 60 views
-// of 736 bins: 17.5 us (residual) and 17.0 us, against 32.4 and 32.1 us of the
-// walk; 4 waves a group 18.1 / 17.5 us, 16 waves 21.5 / 20.9, four lines in
-// flight instead of eight 18.0 / 17.4.  The run length is a multiple of 8
-// whatever K is, so a ray's sum does not depend on K.
+// of 736 bins: 18.8 us (residual) and 18.4 us, against 32.4 and 32.1 us of the
+// walk (17.4 and 17.0 with the interpolation in FP32).  Four lines in flight keep
+// eight waves a SIMD; eight of them and four waves: 20.2 / 19.9.  The run length
+// is a multiple of 8 whatever K is, so a ray's sum does not depend on K.
 constexpr int kLineWaves = 8, kLineBlock = kLineWaves * kWave;
 constexpr double kLineBias = 1572864.0;                    // 2^20 + 2^19
 constexpr int kLineHi0 = (0x413 << 20) + (1 << 19);        // high word of kLineBias
@@ -682,19 +683,20 @@ __device__ __forceinline__ void load_pair(__amdgpu_buffer_rsrc_t rs, uint32_t of
 template <int K>
 __device__ __forceinline__ void line_run(const GL float *img, int na, int nb, int c0, int n, double m, double b0,
                                          double inv, int skip, double (&acc)[K]) {
-    constexpr int OS = K <= 2 ? 8 : (K == 4 ? 4 : 2);
+    constexpr int OS = K <= 2 ? 4 : (K == 4 ? 2 : 1);
     const uint32_t lineb = (uint32_t)line_stride(nb) * K * 4;
     const __amdgpu_buffer_rsrc_t rs = make_rsrc((const void *)img, (uint32_t)line_elems(na, nb) * K * 4);
     double hi = b0 + 0.5 * fabs(m) + m * c0 + kLineBias;
     const double sc = inv * 2.3283064365386963e-10;   // 2^-32
     uint32_t at = (uint32_t)c0 * lineb;
     skip -= c0;
-    auto stage = [&](double (&w)[OS], float (&x)[OS][2 * K]) {
+    // (the weight is made where it is used: the fraction is half its registers)
+    auto stage = [&](uint32_t (&f)[OS], float (&x)[OS][2 * K]) {
         uint32_t off[OS];
 #pragma unroll
         for (int k = 0; k < OS; ++k) {
             const int h = __double2hiint(hi);
-            w[k] = fmin((double)(uint32_t)__double2loint(hi) * sc, 1.0);
+            f[k] = (uint32_t)__double2loint(hi);
             const int j = max(kLineHi0 - 1, min(h, kLineHi0 + nb + 1));   // zeros beyond
             off[k] = (uint32_t)(j - (kLineHi0 - 1)) * (4 * K);            // pixel j - 1, behind two of padding
             hi += m;
@@ -709,14 +711,21 @@ __device__ __forceinline__ void line_run(const GL float *img, int na, int nb, in
         at += OS * lineb;
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto consume = [&](const double (&w)[OS], const float (&x)[OS][2 * K]) {
+    auto consume = [&](const uint32_t (&f)[OS], const float (&x)[OS][2 * K]) {
 #pragma unroll
-        for (int k = 0; k < OS; ++k)
+        for (int k = 0; k < OS; ++k) {
+            uint32_t fr = f[k];
+            asm volatile("" : "+v"(fr));   // (converted here, line by line, not all of them before)
+            const double w = fmin(fmax((double)fr * sc, 0.0), 1.0), w0 = 1.0 - w;
 #pragma unroll
-            for (int j = 0; j < K; ++j)
-                acc[j] = __builtin_fma(w[k], (double)x[k][K + j], __builtin_fma(1.0 - w[k], (double)x[k][j], acc[j]));
+            for (int j = 0; j < K; ++j) {
+                float x0 = x[k][j], x1 = x[k][K + j];
+                asm volatile("" : "+v"(x0), "+v"(x1));
+                acc[j] = __builtin_fma(w, (double)x1, __builtin_fma(w0, (double)x0, acc[j]));
+            }
+        }
     };
-    double wa[OS], wb[OS];
+    uint32_t wa[OS], wb[OS];
     float xa[OS][2 * K], xb[OS][2 * K];
     const int ng = n / OS;
     stage(wa, xa);
@@ -1131,7 +1140,10 @@ __device__ __forceinline__ void bp_unit(const EngArgs<T> &a, const UG<T> &U, int
 // bins whose rays can meet it, a superset; for each the exact length follows
 // from the ray's line in double,
 //   min(1, max(0, ((1 + |m|) / 2 - |b0 + m a - j - 1/2|) / |m|)),
-// times the residual, which holds the ray's length per line.
+// times the residual, which holds the ray's length per line.  Weight, product
+// and sum are double; 1 / |m| is rounded to FP32, once, as a stored length is (as
+// a double it costs 8 more bytes of LDS a slot).  A sum that is not finite is taken again over the rays
+// that cross the pixel (line_bp_again).
 //
 // A block's views come in windows of 64, sorted by axis and by candidates
 // (LineView, prepared with the geometry).  As many views as half of the
@@ -1142,10 +1154,12 @@ __device__ __forceinline__ void bp_unit(const EngArgs<T> &a, const UG<T> &U, int
 // views (view by view in turn) and their sums are added in order.  The order
 // of a pixel's sum depends on the geometry only, not on K or on the LDS slots.
 //
-// What bounds it: VALU, some 33 instructions a view and pixel (a quarter of the
-// issue slots go to LDS latency at four waves a SIMD).  512 x 512 pixels, 60
-// views: 37.4 us, against 35.4 of the staged matrix form (bp_unit, 179 MB a
-// launch); four jobs 40 against 58 us; 256 x 256, 360 views, one job: 75 us.
+// What bounds it: VALU at K = 1, some 32 instructions a view and pixel, half of
+// them on doubles at half rate (a quarter of the
+// issue slots go to LDS latency at four waves a SIMD), LDS reads at K = 4 (36
+// bytes a candidate).  512 x 512 pixels, 60
+// views: 40.1 us, against 35.4 of the staged matrix form (bp_unit, 179 MB a
+// launch) and 37.6 with weights and a view's products in FP32.
 // It needs no matrix at all: an 874 x 874 slice of 576 views is ready in 2 ms
 // (95 ms with the matrix), in 0.2 GB instead of 4.
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
@@ -1185,6 +1199,12 @@ struct LinePix {
     int id;                  // x ny + y
 };
 
+// The ray's share of pixel b - 1/2 of line a.
+__device__ __forceinline__ double line_weight(double m, double b0, float inv, double a, double b) {
+    const double D = __builtin_fma(m, a, b0) - b;
+    return fmin(fmax((__builtin_fma(fabs(m), 0.5, 0.5) - fabs(D)) * (double)inv, 0.0), 1.0);
+}
+
 // C candidates of one view (0: `cand` of them, two at a time) added to tot;
 // slot: the first one's, in the half.
 template <int K, bool EDGE, int C>
@@ -1192,23 +1212,18 @@ __device__ __forceinline__ void line_bp_view(const LineHalf<K> &h, uint32_t slot
                                              double (&tot)[K]) {
     constexpr int CC = C ? C : 2;
     for (int q = 0; q < (C ? C : cand); q += CC, slot += CC) {
-        float t[CC];
+        double t[CC];
 #pragma unroll
         for (int n = 0; n < CC; ++n) {
             const f64x2 mb = h.mb[slot + n];
-            const double m = mb.x, D = __builtin_fma(m, a, mb.y) - b;
-            const float e = (float)(__builtin_fma(fabs(m), 0.5, 0.5) - fabs(D));
-            t[n] = __builtin_amdgcn_fmed3f(e * h.inv[slot + n], 0.0f, 1.0f);
-            if (EDGE) t[n] = h.drop[slot + n] == id ? 0.0f : t[n];
+            t[n] = line_weight(mb.x, mb.y, h.inv[slot + n], a, b);
+            if (EDGE) t[n] = h.drop[slot + n] == id ? 0.0 : t[n];
         }
         const LDSP float *r = h.r + slot * K;
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-            float x = t[0] * r[k];
+        for (int k = 0; k < K; ++k)
 #pragma unroll
-            for (int n = 1; n < CC; ++n) x = __builtin_fmaf(t[n], r[n * K + k], x);
-            tot[k] += (double)x;
-        }
+            for (int n = 0; n < CC; ++n) tot[k] = __builtin_fma(t[n], (double)r[n * K + k], tot[k]);
     }
 }
 
@@ -1241,6 +1256,30 @@ __device__ __forceinline__ void line_bp_run(const LDSP unsigned char *views, int
     }
 }
 
+// Job k's sum of one pixel again, straight from memory, over the rays that
+// cross the pixel: where it is not finite a residual beside the pixel may not
+// be (0 times it is not 0).  tab: the block's first window, windows `step`
+// views apart.
+template <bool ARC>
+__device__ __forceinline__ double line_bp_again(const UG<float> &U, const GL char *tab, int64_t step, int nv, int64_t row0,
+                                                const LinePix &p, double x, double y, int K, int k) {
+    double tot = 0.0;
+    for (int v = 0; v < nv; ++v) {
+        const GL LineView &w = ((const GL LineView *)tab)[v / kLineViews * step + v % kLineViews];
+        const float u = ARC ? line_bin_arc(p.X, p.Y, w.c, w.s, p.sod, p.k)
+                            : line_bin_flat(p.X, p.Y, p.Xk, p.Yk, w.c, w.s, p.sodk);
+        const int slot = (int)__builtin_amdgcn_fmed3f(u + w.lob, w.first, w.end);
+        const bool yd = line_axis(w.meta);
+        for (int n = slot; n < slot + line_cand(w.meta); ++n) {
+            const int64_t e = w.src + n, row = row0 + w.row + n;
+            const GL double *mb = (yd ? U.ln_my : U.ln_mx) + 2 * e;
+            const double t = line_weight(mb[0], mb[1], (yd ? U.ln_iy : U.ln_ix)[e], yd ? y : x, (yd ? x : y) + 0.5);
+            if (t > 1e-6 && U.ln_drop[row] != p.id) tot += t * (double)U.r[row * K + k];
+        }
+    }
+    return tot;
+}
+
 // d = S A_s^T r + alpha R(u, v) for the block's pixels; partial sum d^2.
 // P groups of 256 lanes; cap: slots of one half.
 template <int K, int P>
@@ -1260,22 +1299,22 @@ __device__ __forceinline__ void line_bp_unit(const EngArgs<float> &a, const UG<f
     double tot[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) tot[k] = 0.0;
+    const int64_t row0 = U.sub_row0[s];
+    const int nv = (int)((U.sub_row0[s + 1] - row0) / U.nbins);
+    const int64_t nblk = bp_blocks_of(tnx, U.tny);
+    LinePix p;
+    p.X = (i + 0.5f - 0.5f * U.nx) * U.ln_pix;
+    p.Y = (j + 0.5f - 0.5f * U.ny) * U.ln_pix;
+    p.k = U.ln_k;
+    p.sod = U.ln_sod;
+    p.Xk = p.X / p.k;
+    p.Yk = p.Y / p.k;
+    p.sodk = p.sod / p.k;
+    p.id = i * U.ny + j;
+    const double id = i, jd = j;
     if (j0 < U.ny) {   // else: only padding of the tile rows
-        const int64_t row0 = U.sub_row0[s];
-        const int nv = (int)((U.sub_row0[s + 1] - row0) / U.nbins);
-        const int64_t nblk = bp_blocks_of(tnx, U.tny);
         const int nwin = (nv + kLineViews - 1) / kLineViews;
         const bool edge = i0 == 0 || j0 == 0 || i0 + 16 >= U.nx || j0 + 16 >= U.ny;
-        LinePix p;
-        p.X = (i + 0.5f - 0.5f * U.nx) * U.ln_pix;
-        p.Y = (j + 0.5f - 0.5f * U.ny) * U.ln_pix;
-        p.k = U.ln_k;
-        p.sod = U.ln_sod;
-        p.Xk = p.X / p.k;
-        p.Yk = p.Y / p.k;
-        p.sodk = p.sod / p.k;
-        p.id = i * U.ny + j;
-        const double id = i, jd = j;
 
         // A window: lane l holds view l (its second half: end, meta, src, row;
         // and first), and the views up to the end of each class.
@@ -1363,8 +1402,8 @@ __device__ __forceinline__ void line_bp_unit(const EngArgs<float> &a, const UG<f
             if (nw < nwin) copy(W, nk0, nk1, noff, raw + (par ^ 1) * half);
             const LDSP unsigned char *vt = raw + par * half, *b = vt + VB;
             vt -= k0 * (int)sizeof(LineView);
-            const LineHalf<K> h{(const LDSP f64x2 *)b, (const LDSP float *)(b + cap * 16), (const LDSP float *)(b + cap * 20),
-                                (const LDSP int32_t *)(b + cap * (20 + 4 * K))};
+            const LineHalf<K> h{(const LDSP f64x2 *)b, (const LDSP float *)(b + cap * 16),
+                                (const LDSP float *)(b + cap * 20), (const LDSP int32_t *)(b + cap * (20 + 4 * K))};
             auto run = [&](auto arc, auto ed) {
                 auto one = [&](auto c, int e) {
                     constexpr int C = decltype(c)::value;
@@ -1410,6 +1449,14 @@ __device__ __forceinline__ void line_bp_unit(const EngArgs<float> &a, const UG<f
                 for (int k = 0; k < K; ++k) tot[k] += part[((g - 1) * K + k) * kBlock + threadIdx.x];
         __syncthreads();
     }
+    if (grp == 0 && real)
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            if (!(fabs(tot[k]) < INFINITY)) {
+                const GL char *tab = (const GL char *)U.ln_views + (U.ln_win0[s] * nblk + lb) * VB;
+                tot[k] = U.ln_arc ? line_bp_again<true>(U, tab, nblk * kLineViews, nv, row0, p, id, jd, K, k)
+                                  : line_bp_again<false>(U, tab, nblk * kLineViews, nv, row0, p, id, jd, K, k);
+            }
     LDSP float *Lu = (LDSP float *)raw, *Lv = Lu + kSqN * K;
     if (grp == 0) {
         put_square<float, K>(U, U.u, i0, j0, 0.0f, Lu);
@@ -1780,8 +1827,10 @@ __global__ __launch_bounds__(kLineBlock) void k_line_fp(EngArgs<float> a, BlockM
     MI_KSWITCH(KMAX, (line_fp_unit<K, RESID>(a, U, s, lb, lds)))
 }
 
+// The bounds keep the waves a SIMD that the LDS slots leave room for (six at K =
+// 1, five at K = 4, four at K = 8): unbounded, a few more registers cost one.
 template <int KMAX, int P>
-__global__ __launch_bounds__(P * kBlock) void k_line_bp(EngArgs<float> a, BlockMap m, int s, int cap) {
+__global__ __launch_bounds__(P * kBlock, KMAX == 1 ? 6 : KMAX == 4 ? 5 : 4) void k_line_bp(EngArgs<float> a, BlockMap m, int s, int cap) {
     __shared__ double lds[kBlock / kWave * kMaxK];
     extern __shared__ __align__(16) unsigned char ldr_raw[];
     int ui, lb;
