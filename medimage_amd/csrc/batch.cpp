@@ -25,8 +25,11 @@ bool use_lines(const Matrix &m) {
 template <typename T>
 int64_t unit_state_bytes(const Matrix &m, int K) {
     int64_t e = 2 * m.nrows + kLineEmpty + 4 * m.npix_t;
-    if (use_lines<T>(m)) e += line_elems(m.g.nx, m.g.ny) + line_elems(m.g.ny, m.g.nx);
-    return (int64_t)K * e * (int64_t)sizeof(T);
+    int64_t b = e * (int64_t)sizeof(T);
+    if (use_lines<T>(m))
+        b += m.npix_t * (int64_t)sizeof(T) +
+             (line_elems(m.g.nx, m.g.ny) + line_elems(m.g.ny, m.g.nx)) * (int64_t)(sizeof(T) + line_part_bytes(K));
+    return K * b;
 }
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
@@ -77,13 +80,16 @@ void Unit<T>::alloc(hipStream_t st) {
     if (use_lines<T>(*m)) {
         px.n = (size_t)line_elems(m->g.nx, m->g.ny) * K;
         py.n = (size_t)line_elems(m->g.ny, m->g.nx) * K;
+        qx.n = (px.n * line_part_bytes(K) + sizeof(T) - 1) / sizeof(T);   // parts are counted in T
+        qy.n = (py.n * line_part_bytes(K) + sizeof(T) - 1) / sizeof(T);
+        ul.n = (size_t)m->npix_t * K;
     }
     constexpr size_t kAlign = 256 / sizeof(T);   // each part starts on a 256-byte line, as an allocation of its own does
     size_t at = 0;
-    for (Part *b : {&g, &r, &u, &v, &d, &w, &px, &py}) at += (b->n + kAlign - 1) / kAlign * kAlign;
+    for (Part *b : {&g, &r, &u, &v, &d, &w, &px, &py, &qx, &qy, &ul}) at += (b->n + kAlign - 1) / kAlign * kAlign;
     state.alloc(at);
     at = 0;
-    for (Part *b : {&g, &r, &u, &v, &d, &w, &px, &py}) {
+    for (Part *b : {&g, &r, &u, &v, &d, &w, &px, &py, &qx, &qy, &ul}) {
         if (b->n) b->p = state.p + at;
         at += (b->n + kAlign - 1) / kAlign * kAlign;
     }
@@ -225,6 +231,12 @@ Unit<T> *Batch<T>::place(BatchJob<T> &j, int group) {
 }
 
 template <typename T>
+void Batch<T>::spread(const Unit<T> &U) {
+    const Matrix &m = *U.m;
+    eng_spread<T>(ctx->stream, U.u.p, U.ul.p, (float *)U.px.p, (float *)U.py.p, U.qx.p, U.qy.p, U.K, m.g.nx, m.g.ny, m.tny);
+}
+
+template <typename T>
 void Batch<T>::load_job(BatchJob<T> &j) {
     Unit<T> &U = *units[j.uid];
     const Matrix &m = *U.m;
@@ -242,7 +254,10 @@ void Batch<T>::load_job(BatchJob<T> &j) {
     } else {
         eng_put_img<T>(st, U.u.p, U.K, j.slot, nx, ny, m.tny, nullptr, T(0));
     }
-    if (U.px.p) eng_spread<T>(st, U.u.p, U.px.p, U.py.p, U.K, nx, ny, m.tny);
+    if (U.ul.p) {
+        eng_put_img<T>(st, U.ul.p, U.K, j.slot, nx, ny, m.tny, nullptr, T(0));
+        spread(U);
+    }
     if (!j.v0.empty()) {
         MI_HIP(hipMemcpyAsync(stage.p, j.v0.data(), m.npix * sizeof(T), hipMemcpyHostToDevice, st));
         eng_put_img<T>(st, U.v.p, U.K, j.slot, nx, ny, m.tny, stage.p, T(1));
@@ -345,7 +360,7 @@ int Batch<T>::admit(bool require) {
 
 // Repacks the jobs of each matrix into units of 8 plus one unit of the
 // next power of two above the remainder, when that needs fewer slots than
-// the current units.  Job state (g, u, v, scalars) moves with the job; r, d
+// the current units.  Job state (g, u and its remainder, v, scalars) moves with the job; r, d
 // and w are scratch that every pass rewrites.
 template <typename T>
 void Batch<T>::compact() {
@@ -401,6 +416,7 @@ void Batch<T>::compact() {
                 const int from = j.uid * kMaxK + j.slot, to = uid * kMaxK + k;
                 eng_move<T>(st, U->g.p, K, k, src->g.p, src->K, j.slot, mp->nrows);
                 eng_move<T>(st, U->u.p, K, k, src->u.p, src->K, j.slot, mp->npix_t);
+                if (U->ul.p) eng_move<T>(st, U->ul.p, K, k, src->ul.p, src->K, j.slot, mp->npix_t);
                 eng_move<T>(st, U->v.p, K, k, src->v.p, src->K, j.slot, mp->npix_t);
                 MI_HIP(hipMemcpyAsync(d_sc.p + to, sc_old.p + from, sizeof(Scalars), hipMemcpyDeviceToDevice, st));
                 h_jp[to] = jp_old[from];
@@ -408,7 +424,7 @@ void Batch<T>::compact() {
                 j.uid = uid;
                 j.slot = k;
             }
-            if (U->px.p) eng_spread<T>(st, U->u.p, U->px.p, U->py.p, K, mp->g.nx, mp->g.ny, mp->tny);
+            if (U->ul.p) spread(*U);
             units[uid] = std::move(U);
             live.push_back(uid);
         }
@@ -482,8 +498,12 @@ void Batch<T>::rebuild() {
             D.ln_bin0 = m.lines.bin0;
             D.ln_pix = (float)m.g.pixel_mm;
             D.ln_arc = m.lines.arc;
-            D.px = U.px.p;
-            D.py = U.py.p;
+            D.px = (float *)U.px.p;
+            D.py = (float *)U.py.p;
+            D.qx = U.qx.p;
+            D.qy = U.qy.p;
+            D.ul = U.ul.p;
+            D.dl = U.w.p;   // w is the edge steps' and the median's
         }
         D.fs_slice0 = m.has_otf ? m.otf.d_slice0.p : m.fs.d_slice0.p;
         if (m.has_otf) {

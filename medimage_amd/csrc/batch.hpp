@@ -39,7 +39,7 @@ struct Unit {
     };
     DevBuf<T> state;
     Part g, r, u, v, d, w;
-    Part px, py;                   // projection images (units with lines)
+    Part px, py, qx, qy, ul;       // units with lines: projection images, what u's rounding leaves over
     void alloc(hipStream_t st);
     int used() const {
         int n = 0;
@@ -183,6 +183,7 @@ struct Batch {
 
     // Internals (also used by the launch-shape tuner).
     Unit<T> *place(BatchJob<T> &j, int group_size);
+    void spread(const Unit<T> &U);   // u and its remainder into the projection images
     void load_job(BatchJob<T> &j);
     void retire(BatchJob<T> &j);
     void free_slot(BatchJob<T> &j);

@@ -93,8 +93,11 @@ struct UnitDesc {
     T *u, *v, *d, *w;                      // npix_t * K
     // projection images of a unit with lines: the image to be projected next
     // (u, or d between the back projection and the update), row by row and
-    // column by column, zero-padded (line_stride / line_elems), K interleaved
-    T *px, *py;
+    // column by column, zero-padded (line_stride / line_elems), K interleaved:
+    // px, py in FP32; qx, qy u's second part (LineForm)
+    float *px, *py;
+    void *qx, *qy;
+    T *ul, *dl;                            // what the FP32 rounding of u, and of d until the update, leaves over
     int64_t npix_t, nrows;
     int64_t part_off, cap;                 // partials: part + part_off + (slot * K + j) * cap
     int nx, ny, tny, K, fs_P, bs_P;
@@ -150,9 +153,12 @@ void eng_line_bp(hipStream_t st, const EngArgs<float> &a, const BlockMap &m, int
 // 256 lanes put four waves on every SIMD.  Two groups at 1024 blocks: 38.1 us
 // against 37.4.
 inline int line_groups(int64_t blocks) { return blocks <= 320 ? 4 : (blocks <= 640 ? 2 : 1); }
-// Writes u into the unit's projection images.
+// Writes u and its remainder into the unit's projection images.
 template <typename T>
-void eng_spread(hipStream_t st, const T *u, T *px, T *py, int K, int nx, int ny, int tny);
+void eng_spread(hipStream_t st, const T *u, const T *ul, float *px, float *py, void *qx, void *qy, int K, int nx, int ny,
+                int tny);
+// Bytes of a value's second part in qx / qy for units of K jobs.
+inline int line_part_bytes(int K) { return K <= 2 ? 8 : 2; }
 template <typename T>
 void eng_nv(hipStream_t st, const EngArgs<T> &a, const BlockMap &pix, int kmax);
 template <typename T>
