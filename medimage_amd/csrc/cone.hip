@@ -685,12 +685,30 @@ __global__ __launch_bounds__(kBlock) void k_cone_bp(ConeDev g, const float *cs, 
 // 0.94; 64^3 x 100: 0.91 and 0.30.  Against 64-bit sums of the exact lengths
 // both are off by 4.9e-7 of the largest voxel at 128^3.
 constexpr int kConeRun = 24, kConeStep = 4;   // rows of a patch column per lane: at most, a multiple of
+constexpr float kConeRange = 7.62939453125e-6f;   // 2^-17
 constexpr int kConeBatch = 5;                 // planes whose LDS reads are issued together (9: 4% slower at C4)
 struct ConeView {
     int col0, ncol, r0, nr;       // the patch: panel columns, rows
     int run, cand;                // rows per lane; candidate columns of a voxel column
     float hw, icol;               // half width of a voxel column's shadow, 1 / ncol
 };
+
+// The largest x >= 0 of the wave's lanes.
+__device__ __forceinline__ float wave_top(float x) {
+    auto step = [&](auto ctrl, auto rows) {
+        const int o = __builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, decltype(rows)::value, 0xf, true);
+        x = fmaxf(x, __int_as_float(o));
+    };
+    using std::integral_constant;
+    const integral_constant<int, 0xf> all;
+    step(integral_constant<int, 0x111>{}, all);   // row_shr:1, 2, 4, 8
+    step(integral_constant<int, 0x112>{}, all);
+    step(integral_constant<int, 0x114>{}, all);
+    step(integral_constant<int, 0x118>{}, all);
+    step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});   // row_bcast:15, 31
+    step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+}
 
 // A value that all lanes hold, in scalar registers.
 __device__ __forceinline__ double uniform(double x) {
@@ -809,7 +827,8 @@ __device__ __forceinline__ void cone_bp_block(
     // this lane's part of view iv's patch, into registers (rows behind its
     // run are other lanes', rows behind the panel read as 0)
     int v0 = 0;
-    bool bad = false;   // a sum of this lane was not finite
+    bool bad = false;   // a sum of this lane was not finite, or the values differ too much
+    float top = 0.0f, low = INFINITY;   // largest value of the wave's lanes in any view, the least such of a well filled view
     auto load = [&](int iv) {
         const ConeView w = info[iv];
         const int seg = (int)(((float)tid + 0.5f) * w.icol), col = tid - seg * w.ncol;   // tid / ncol
@@ -870,6 +889,7 @@ __device__ __forceinline__ void cone_bp_block(
             const int r = seg * w.run;
             const bool any = r < w.nr;
             double sum = 0.0;
+            float most = 0.0f;   // largest value of this lane's run
             if (any) {
                 const float *w2 = w2s + (w.r0 - rbase + r + 1);
 #pragma unroll
@@ -879,10 +899,21 @@ __device__ __forceinline__ void cone_bp_block(
                         for (int h = i; h < i + kConeStep; ++h) {
                             raw[h] *= __builtin_amdgcn_sqrtf(w2[h] + l2);
                             sum += (double)raw[h];
+                            most = fmaxf(most, fabsf(raw[h]));
                             asm volatile("" : "+v"(raw[h]));   // (converted again below: not 24 doubles kept)
                         }
             }
             bad |= !(fabs(sum) < INFINITY);
+            // A few values far above the others would take the others' last
+            // bits in the running sums and the planes' (some 3e-13 of the
+            // largest over 720 views): a sixteenth of a wave's runs below
+            // 2^-17 of its largest, or views that differ so, and the block's
+            // voxels go ray by ray.
+            const float wtop = wave_top(most);
+            const int filled = __popcll(__ballot(most > 0.0f));
+            bad |= 16 * __popcll(__ballot(most > 0.0f && most < wtop * kConeRange)) > filled;
+            top = fmaxf(top, wtop);
+            if (filled >= kWave / 2) low = fminf(low, wtop);
             tots[tid] = sum;
             // a ray along an axis: all or nothing on the other, by a huge finite
             // inverse (0 x infinity has no value)
@@ -959,9 +990,11 @@ __device__ __forceinline__ void cone_bp_block(
             __syncthreads();   // the patch is written again
         }
     }
+    bad |= low < top * kConeRange;
     if (__syncthreads_or(bad)) {
-        // A value that is not finite would reach every row behind it through
-        // the running sums: the block's voxels ray by ray instead.
+        // A value that is not finite, or far above the others, would reach every
+        // row behind it through the running sums: the block's voxels ray by ray
+        // instead.
         const int zend = min(z0 + NK, g.nz);
         for (int z = z0; z < zend; z += kZc) {
             if (x >= g.nx || y >= g.ny) break;
