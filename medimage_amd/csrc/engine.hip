@@ -67,7 +67,7 @@ struct UG {
     GL char *qx, *qy;
     int64_t npix_t, nrows, part_off, cap;
     int nx, ny, tny, K, fs_P, bs_P, job0, nbins, ln_arc;
-    float ln_sod, ln_k, ln_bin0, ln_pix;
+    float ln_sod, ln_k, ln_pix;
     template <typename Desc>   // UnitDesc<T>, of any address space
     __device__ __forceinline__ explicit UG(Desc &D)
         : fs_slice0((const GL int64_t *)D.fs_slice0), fs_base((const GL int64_t *)D.fs_base),
@@ -92,7 +92,7 @@ struct UG {
           v((GL T *)D.v), d((GL T *)D.d), w((GL T *)D.w), ul((GL T *)D.ul), dl((GL T *)D.dl), px((GL float *)D.px), py((GL float *)D.py), qx((GL char *)D.qx), qy((GL char *)D.qy),
           npix_t(D.npix_t), nrows(D.nrows),
           part_off(D.part_off), cap(D.cap), nx(D.nx), ny(D.ny), tny(D.tny), K(D.K), fs_P(D.fs_P), bs_P(D.bs_P),
-          job0(D.job0), nbins(D.nbins), ln_arc(D.ln_arc), ln_sod(D.ln_sod), ln_k(D.ln_k), ln_bin0(D.ln_bin0),
+          job0(D.job0), nbins(D.nbins), ln_arc(D.ln_arc), ln_sod(D.ln_sod), ln_k(D.ln_k),
           ln_pix(D.ln_pix) {}
     // Tiled index of pixel (i, j), or -1 outside the image.
     __device__ __forceinline__ int64_t at(int i, int j) const {

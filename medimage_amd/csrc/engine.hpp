@@ -86,7 +86,7 @@ struct UnitDesc {
     const float *ln_ix, *ln_iy;
     const int64_t *ln_win0;
     const LineView *ln_views;
-    float ln_sod, ln_k, ln_bin0, ln_pix;   // Lines, pixel size in mm
+    float ln_sod, ln_k, ln_pix;            // Lines, pixel size in mm
     int ln_arc;
     const int64_t *sub_row0;               // S + 1 row offsets
     T *g, *r;                              // rows * K

@@ -220,7 +220,7 @@ struct Lines {
     DevBuf<int64_t> d_win0;
     DevBuf<LineView> views;
     int arc = 0;
-    float sod = 0.f, k = 0.f, bin0 = 0.f;
+    float sod = 0.f, k = 0.f;
     size_t bytes() const {
         return d_slice0.bytes() + mb.bytes() + len.bytes() + inv.bytes() + drop.bytes() + skip.bytes() + rng.bytes() +
                mx.bytes() + my.bytes() + ix.bytes() + iy.bytes() + d_win0.bytes() + views.bytes();

@@ -503,7 +503,8 @@ __global__ __launch_bounds__(kLineRays) void k_lines_fill(TraceArgs a, const int
 // at the block's centre.
 struct LineGeo {
     int nx, ny, nbins, arc;
-    float pix, sod, k, bin0;
+    float pix, sod, k;
+    double bin0;
 };
 __device__ __forceinline__ void line_view(const LineGeo &g, float c, float s, int i0, int j0, int &b0, int &cnt, float &hw,
                                           int &axis) {
@@ -531,13 +532,16 @@ __device__ __forceinline__ void line_view(const LineGeo &g, float c, float s, in
         }
     }
     // first order in the pixel; the arc's least distance may lie between the
-    // corners; the float rounding, and the arc tangent's error on the arc
+    // corners; the float rounding (a few units of the position's last place,
+    // more where the distance to the source is a small difference; the slot,
+    // below 2^15, has its own), and the arc tangent's error on the arc
     const float step = g.arc ? sqrtf(rn) * p : rn * p;
     const float near = g.arc ? 1.0f + 256.0f * step * step : 1.0f;
-    hw = 0.5f * p * (ax + ay) * rn * near * (1.0f + 2.0f * step) + 0.01f + (g.arc ? 1.2e-5f * k : 0.0f);
-    b0 = max(0, (int)ceilf(lo + g.bin0 - hw - 0.01f));
-    cnt = max(0, min(g.nbins - 1, (int)floorf(hi + g.bin0 + hw + 1.01f)) - b0 + 1);
-    b0 = min(b0, g.nbins);
+    const float err = fmaxf(fabsf(lo), fabsf(hi)) * 2.4e-7f * (1.0f + 2.0f * sod / p * step);
+    hw = 0.5f * p * (ax + ay) * rn * near * (1.0f + 2.0f * step) + 0.01f + err + (g.arc ? 1.2e-5f * k : 0.0f);
+    // (the bins counted from an offset that float does not hold: in double)
+    b0 = (int)fmin(fmax(ceil(lo + g.bin0 - hw - 0.01), 0.0), (double)g.nbins);
+    cnt = max(0, (int)fmin(floor(hi + g.bin0 + hw + 1.01), g.nbins - 1.0) - b0 + 1);
     const float Xc = X0 + 8 * p, Yc = Y0 + 8 * p;
     axis = g.arc ? fabsf(Yc - sod * s) > fabsf(Xc - sod * c) : fabsf(Yc + sod * c) > fabsf(Xc - sod * s);
 }
@@ -590,7 +594,7 @@ __global__ __launch_bounds__(kLineViews) void k_line_windows(LineGeo g, int tnx,
         LineView w;
         w.c = c;
         w.s = sn;
-        w.lob = g.bin0 - hw + 1.0f + (float)(off - b0);   // + 1: the conversion to a slot rounds down
+        w.lob = (float)(g.bin0 - hw + 1.0 + (off - b0));   // + 1: the conversion to a slot rounds down
         w.first = (float)off;
         w.end = (float)(off + cnt);
         w.meta = line_meta(off + size, cand, axis);
@@ -613,7 +617,6 @@ bool try_lines(Matrix &m, const TraceArgs &a, hipStream_t st) {
     q.arc = g.beam == MI_BEAM_FAN_ARC;
     q.sod = (float)g.sod_mm;
     q.k = (float)(q.arc ? 180.0 / (M_PI * g.bin_mm) : g.sdd_mm / g.bin_mm);
-    q.bin0 = (float)(q.arc ? g.n_bins / 2 - g.det_offset : g.n_bins / 2 - 0.5 - g.det_offset);
     // every corner of a block, also one that reaches past the image, lies in
     // front of the source
     const double rad = 0.5 * g.pixel_mm * std::hypot((double)g.nx, (double)g.ny), blk = 16 * M_SQRT2 * g.pixel_mm;
@@ -655,7 +658,8 @@ bool try_lines(Matrix &m, const TraceArgs &a, hipStream_t st) {
                     (unsigned *)flags.p, nnz.p};
     k_lines_fill<<<(unsigned)groups, kLineRays, 0, st>>>(a, m.d_sub_row0.p, q.d_slice0.p, m.S, o);
     MI_HIP(hipGetLastError());
-    const LineGeo lg{g.nx, g.ny, g.n_bins, q.arc, (float)g.pixel_mm, q.sod, q.k, q.bin0};
+    const double bin0 = q.arc ? g.n_bins / 2 - g.det_offset : g.n_bins / 2 - 0.5 - g.det_offset;
+    const LineGeo lg{g.nx, g.ny, g.n_bins, q.arc, (float)g.pixel_mm, q.sod, q.k, bin0};
     k_line_windows<<<(unsigned)wins, kLineViews, 0, st>>>(lg, tnx, tny, nblk, a.fcos, a.fsin, a.vlist, m.d_sub_row0.p,
                                                          q.d_win0.p, m.S, q.views.p, flags.p + 1);
     MI_HIP(hipGetLastError());

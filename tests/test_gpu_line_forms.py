@@ -1,0 +1,40 @@
+"""Fan-beam reconstructions along lines at the limits of that form against the
+FP64 oracle.  The bar is that of the line form's other comparison (2e-6 after
+12 updates)."""
+import numpy as np
+import pytest
+
+import medimage_amd as mi
+import oracle_py as O
+from test_gpu_lines import _fan
+
+pytestmark = pytest.mark.gpu
+
+EDGE = {
+    # seven or eight rays a pixel, the most that the back projection takes
+    "eight_rays": _fan(96, 96, 3.0, 20, 330, 1.8),
+    # a source just behind the least distance (2% of it beyond the image and a block)
+    "near_source": _fan(64, 64, 4.0, 40, 137, 6.0, sod=279.0, sdd=480.0),
+    # an arc just inside its 45 degrees
+    "wide_arc": mi.arc_geometry(96, 3.0, 48, 76, 1.2, 295.0, 600.0, 1.75),
+    # a detector so long that a float does not hold its bins' places
+    "long_detector": _fan(48, 48, 4.0, 2, 16000001, 4.0, off=0.3),
+    "view_pairs": _fan(80, 80, 3.0, 9, 111, 3.3),
+}
+
+@pytest.mark.parametrize("name,subsets", [("eight_rays", 4), ("near_source", 4), ("wide_arc", 4), ("long_detector", 1),
+                                          ("view_pairs", 9), ("view_pairs", 8), ("view_pairs", 4)])
+def test_line_limits_match_oracle(ctx, name, subsets):
+    g = EDGE[name]
+    rng = np.random.default_rng(len(name))
+    img = rng.random((g.nx, g.ny)) * 0.02 / g.pixel_mm
+    of = O.fan_from(g)
+    sino = O.fan_fp(of, img)
+    sino32 = np.where(sino > 0, sino + 0.01 * rng.random(sino.shape), 0.0).astype(np.float32)
+    p = mi.at_params(1e-3, 1e-4, 1e-2, n_subsets=subsets, max_iters=3)
+    u, v, rep = ctx.at_reconstruct(g, sino32, p)
+    ou, ov, _, hist = O.os_at(O.op_fan(of), sino32.astype(np.float64), 1e-3, 1e-4, 1e-2, subsets, 3)
+    eu, ev = (float(np.linalg.norm(a - b) / np.linalg.norm(b)) for a, b in ((u, ou), (v, ov)))
+    print(f"[line limits {name} {subsets}] u {eu:.1e} v {ev:.1e}", flush=True)
+    assert eu < 2e-6 and ev < 2e-6
+    assert abs(rep.data_fidelity - hist[-1]) <= 1e-5 * hist[-1]
