@@ -495,6 +495,7 @@ void Batch<T>::rebuild() {
             D.ln_views = m.lines.views.p;
             D.ln_sod = m.lines.sod;
             D.ln_k = m.lines.k;
+            D.ln_vstride = m.lines.vstride;
             D.ln_pix = (float)m.g.pixel_mm;
             D.ln_arc = m.lines.arc;
             D.px = (float *)U.px.p;

@@ -113,47 +113,62 @@ std::shared_ptr<Matrix> get_matrix(mi_context *ctx, const mi_geometry &g, int S,
     return m;
 }
 
-// The lines of g's rays (has_lines false: they have no such form).
-std::shared_ptr<Matrix> get_lines(mi_context *ctx, const mi_geometry &g) {
-    const GeomKey key = make_key(g, 1, 2);
-    auto it = ctx->matrices.find(key);
-    if (it == ctx->matrices.end())
-        it = ctx->matrices.emplace(key, std::shared_ptr<Matrix>(build_matrix(g, 1, false, ctx->stream, 2).release())).first;
-    it->second->last_use = ++ctx->tick;
-    return it->second;
-}
-
-std::shared_ptr<Matrix> find_engine_matrix(mi_context *ctx, const mi_geometry &g, int S, bool want64) {
-    auto it = ctx->matrices.find(make_key(g, S, 1));
-    if (it == ctx->matrices.end() || (want64 && !it->second->has64)) return nullptr;
-    return it->second;
-}
-
-std::shared_ptr<Matrix> get_engine_matrix(mi_context *ctx, const mi_geometry &g, int S, bool want64) {
-    const GeomKey key = make_key(g, S, 1);
-    auto it = ctx->matrices.find(key);
-    if (it != ctx->matrices.end() && (!want64 || it->second->has64)) {
-        it->second->last_use = ++ctx->tick;
-        return it->second;
-    }
-    if (it != ctx->matrices.end()) ctx->matrices.erase(it);
+// Builds (g, S, layout) and keeps it.  Out of device memory: drops idle cached
+// matrices (least recently used first) and builds once more.
+std::shared_ptr<Matrix> build_kept(mi_context *ctx, const mi_geometry &g, int S, bool want64, int layout) {
     std::shared_ptr<Matrix> m;
     for (int attempt = 0;; ++attempt) {
         try {
-            m.reset(build_matrix(g, S, want64, ctx->stream, 1).release());
-            build_sell(*m, ctx->stream, true);
+            m.reset(build_matrix(g, S, want64, ctx->stream, layout).release());
+            if (layout == 1 || (layout == 3 && m->has_lines)) build_sell(*m, ctx->stream, true);
             break;
         } catch (const Error &e) {
-            // Out of device memory: drop idle cached matrices (least recently
-            // used first) and build once more.
             (void)hipGetLastError();
             m.reset();
             if (e.code != MI_E_NOMEM || attempt > 0 || evict_idle(ctx, -1) <= 0) throw;
         }
     }
     m->last_use = ++ctx->tick;
-    ctx->matrices[key] = m;
+    ctx->matrices[make_key(g, S, layout)] = m;
     return m;
+}
+
+bool fan_beam(const mi_geometry &g) { return g.beam == MI_BEAM_FAN_FLAT || g.beam == MI_BEAM_FAN_ARC; }
+
+// The lines of a fan beam (layout 2 or 3).  A geometry without them keeps that
+// answer, so that it is looked at once.
+std::shared_ptr<Matrix> get_lines(mi_context *ctx, const mi_geometry &g, int S, int layout) {
+    auto it = ctx->matrices.find(make_key(g, S, layout));
+    if (it == ctx->matrices.end()) return build_kept(ctx, g, S, false, layout);
+    it->second->last_use = ++ctx->tick;
+    return it->second;
+}
+
+std::shared_ptr<Matrix> find_engine_matrix(mi_context *ctx, const mi_geometry &g, int S, bool want64) {
+    if (!want64 && fan_beam(g)) {
+        auto it = ctx->matrices.find(make_key(g, S, 3));
+        if (it == ctx->matrices.end()) return nullptr;
+        if (it->second->has_lines) return it->second;
+    }
+    auto it = ctx->matrices.find(make_key(g, S, 1));
+    if (it == ctx->matrices.end() || (want64 && !it->second->has64)) return nullptr;
+    return it->second;
+}
+
+std::shared_ptr<Matrix> get_engine_matrix(mi_context *ctx, const mi_geometry &g, int S, bool want64) {
+    // FP32 runs of a fan beam along lines: beside a matrix that an FP64 run of
+    // the geometry may have built, so that neither depends on the other
+    if (!want64 && fan_beam(g)) {
+        const std::shared_ptr<Matrix> l = get_lines(ctx, g, S, 3);
+        if (l->has_lines) return l;
+    }
+    auto it = ctx->matrices.find(make_key(g, S, 1));
+    if (it != ctx->matrices.end() && (!want64 || it->second->has64)) {
+        it->second->last_use = ++ctx->tick;
+        return it->second;
+    }
+    if (it != ctx->matrices.end()) ctx->matrices.erase(it);
+    return build_kept(ctx, g, S, want64, 1);
 }
 
 int64_t evict_idle(mi_context *ctx, int64_t bytes) {
@@ -331,8 +346,8 @@ void forward_impl(mi_context *ctx, const mi_geometry *g, const T *img, T *sino) 
     if constexpr (sizeof(T) == 4) {
         // A fan beam along its rays' lines: no matrix to build and to read
         // (512 x 512 pixels, 720 views of 736 bins: 2.7 GB in 1332 us).
-        if (g->beam == MI_BEAM_FAN_FLAT || g->beam == MI_BEAM_FAN_ARC) {
-            const std::shared_ptr<Matrix> l = get_lines(ctx, *g);
+        if (fan_beam(*g)) {
+            const std::shared_ptr<Matrix> l = get_lines(ctx, *g, 1, 2);
             if (l->has_lines) {
                 const Matrix &m = *l;
                 const int64_t ex = line_elems(g->nx, g->ny), ey = line_elems(g->ny, g->nx);

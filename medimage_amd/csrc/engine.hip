@@ -66,7 +66,7 @@ struct UG {
     GL float *px, *py;
     GL char *qx, *qy;
     int64_t npix_t, nrows, part_off, cap;
-    int nx, ny, tny, K, fs_P, bs_P, job0, nbins, ln_arc;
+    int nx, ny, tny, K, fs_P, bs_P, job0, nbins, ln_arc, ln_vstride;
     float ln_sod, ln_k, ln_pix;
     template <typename Desc>   // UnitDesc<T>, of any address space
     __device__ __forceinline__ explicit UG(Desc &D)
@@ -92,7 +92,7 @@ struct UG {
           v((GL T *)D.v), d((GL T *)D.d), w((GL T *)D.w), ul((GL T *)D.ul), dl((GL T *)D.dl), px((GL float *)D.px), py((GL float *)D.py), qx((GL char *)D.qx), qy((GL char *)D.qy),
           npix_t(D.npix_t), nrows(D.nrows),
           part_off(D.part_off), cap(D.cap), nx(D.nx), ny(D.ny), tny(D.tny), K(D.K), fs_P(D.fs_P), bs_P(D.bs_P),
-          job0(D.job0), nbins(D.nbins), ln_arc(D.ln_arc), ln_sod(D.ln_sod), ln_k(D.ln_k),
+          job0(D.job0), nbins(D.nbins), ln_arc(D.ln_arc), ln_vstride(D.ln_vstride), ln_sod(D.ln_sod), ln_k(D.ln_k),
           ln_pix(D.ln_pix) {}
     // Tiled index of pixel (i, j), or -1 outside the image.
     __device__ __forceinline__ int64_t at(int i, int j) const {
@@ -1371,7 +1371,7 @@ __device__ __forceinline__ void line_bp_run(const LDSP unsigned char *views, int
 // Job k's sum of one pixel again, straight from memory, over the rays that
 // cross the pixel: where it is not finite a residual beside the pixel may not
 // be (0 times it is not 0).  tab: the block's first window, windows `step`
-// views apart.
+// table entries apart.
 template <bool ARC>
 __device__ __forceinline__ double line_bp_again(const UG<float> &U, const GL char *tab, int64_t step, int s, int i, int j,
                                                 int K, int k) {
@@ -1435,7 +1435,7 @@ __device__ __forceinline__ void line_bp_unit(const EngArgs<float> &a, const UG<f
         };
         auto load = [&](int w) {
             Window W;
-            W.tab = (const GL char *)U.ln_views + ((U.ln_win0[s] + w) * nblk + lb) * VB;
+            W.tab = (const GL char *)U.ln_views + ((U.ln_win0[s] + w) * nblk + lb) * (U.ln_vstride * (int64_t)sizeof(LineView));
             W.n = min(kLineViews, nv - w * kLineViews);
             W.b = i32x4{0, 0, 0, 0};
             W.first = 0.0f;
@@ -1568,9 +1568,10 @@ __device__ __forceinline__ void line_bp_unit(const EngArgs<float> &a, const UG<f
 #pragma unroll
         for (int k = 0; k < K; ++k)
             if (!(fabs(tot[k]) < INFINITY)) {
-                const GL char *tab = (const GL char *)V.ln_views + (V.ln_win0[s] * nblk + lb) * VB;
-                tot[k] = V.ln_arc ? line_bp_again<true>(V, tab, nblk * kLineViews, s, i, j, K, k)
-                                  : line_bp_again<false>(V, tab, nblk * kLineViews, s, i, j, K, k);
+                const GL char *tab =
+                    (const GL char *)V.ln_views + (V.ln_win0[s] * nblk + lb) * (V.ln_vstride * (int64_t)sizeof(LineView));
+                tot[k] = V.ln_arc ? line_bp_again<true>(V, tab, nblk * V.ln_vstride, s, i, j, K, k)
+                                  : line_bp_again<false>(V, tab, nblk * V.ln_vstride, s, i, j, K, k);
             }
     LDSP float *Lu = (LDSP float *)raw, *Lv = Lu + kSqN * K;
     if (grp == 0) {

@@ -87,7 +87,7 @@ struct UnitDesc {
     const int64_t *ln_win0;
     const LineView *ln_views;
     float ln_sod, ln_k, ln_pix;            // Lines, pixel size in mm
-    int ln_arc;
+    int ln_arc, ln_vstride;
     const int64_t *sub_row0;               // S + 1 row offsets
     T *g, *r;                              // rows * K
     T *u, *v, *d, *w;                      // npix_t * K

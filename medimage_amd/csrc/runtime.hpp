@@ -62,7 +62,9 @@ struct GeomKey {
 // The caller's per-view angle table as an owned copy (empty: none).
 std::vector<double> view_table(const mi_geometry &g);
 // layout: 0 = CSR / CSC (projector calls), 1 = sliced (AT engine), 2 = the
-// rays' lines alone (has_lines false: a ray has no such form).
+// rays' lines alone (FP32 forward projection), 3 = the lines and the back
+// projection's tables (FP32 AT engine); 2 and 3 with has_lines false: the
+// geometry has no such form.
 GeomKey make_key(const mi_geometry &g, int n_subsets, int layout = 0);
 void validate_geometry(const mi_geometry &g);
 
@@ -215,10 +217,11 @@ struct Lines {
     //   flat: bin k (c X + s Y) / (sod - s X + c Y) + bin0, k = sdd / bin_mm
     //   arc:  bin -k atan((c Y - s X) / (sod - c X - s Y)) + bin0, k = 1 / (radians per bin)
     // and, per block and window of kLineViews views, the views by line_class:
-    // window w of subset s and block b at ((win0[s] + w) nblk + b) kLineViews.
+    // window w of subset s and block b at ((win0[s] + w) nblk + b) vstride.
     std::vector<int64_t> win0;
     DevBuf<int64_t> d_win0;
     DevBuf<LineView> views;
+    int vstride = 0;                 // views a window has room for
     int arc = 0;
     float sod = 0.f, k = 0.f;
     size_t bytes() const {
@@ -317,9 +320,8 @@ void build_sell(Matrix &m, hipStream_t st, bool drop_csr = false);
 // Builds the matrix for (g, S) on the stream; want64 also keeps double
 // lengths.  Host-side GoldenC walk for MI_BEAM_GOLDENC, device tracers
 // otherwise.
-// layout as make_key's: 1 builds a fan beam's lines, which are all that FP32
-// then needs (has_csr false), else the checkpointed walk as well; 2 stops
-// behind the lines.
+// layout as make_key's: 1 also builds a fan beam's checkpointed walk, 2 and 3 no
+// matrix at all (has_csr false).
 std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, hipStream_t st, int layout = 0);
 // Subset order: bit-reversed subset indices (values >= S dropped).
 std::vector<int> subset_order(int S);

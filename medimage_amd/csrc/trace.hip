@@ -476,14 +476,16 @@ __global__ __launch_bounds__(kLineRays) void k_lines_fill(TraceArgs a, const int
         // Both lines.  Turned, m -> 1 / m: the length in a pixel stays len times
         // min(1, max(0, ((1 + |m|) / 2 - |..|) / min(1, |m|))) with |m| > 1.  Only
         // rays near the diagonal are looked at along their other axis.
-        const int64_t e = row / a.nbins * (a.nbins + kLineEmpty) + bin;
-        const bool near = fabs(m) > 0.25;
-        const double2 own = make_double2(m, b0), no = make_double2(0.0, -64.0);
-        const double2 other = near ? make_double2(1.0 / m, 0.5 + (0.5 - b0) / m) : no;
-        o.mx[e] = yd ? other : own;
-        o.my[e] = yd ? own : other;
-        o.ix[e] = yd ? (near ? 1.0f : 0.0f) : (float)inv;
-        o.iy[e] = yd ? (float)inv : (near ? 1.0f : 0.0f);
+        if (o.mx) {
+            const int64_t e = row / a.nbins * (a.nbins + kLineEmpty) + bin;
+            const bool near = fabs(m) > 0.25;
+            const double2 own = make_double2(m, b0), no = make_double2(0.0, -64.0);
+            const double2 other = near ? make_double2(1.0 / m, 0.5 + (0.5 - b0) / m) : no;
+            o.mx[e] = yd ? other : own;
+            o.my[e] = yd ? own : other;
+            o.ix[e] = yd ? (near ? 1.0f : 0.0f) : (float)inv;
+            o.iy[e] = yd ? (float)inv : (near ? 1.0f : 0.0f);
+        }
     }
     int x0 = yd ? INT32_MAX : r0, x1 = yd ? 0 : r1, y0 = yd ? r0 : INT32_MAX, y1 = yd ? r1 : 0;
     for (int w = kWave / 2; w > 0; w >>= 1) {
@@ -552,7 +554,7 @@ __device__ __forceinline__ void line_view(const LineGeo &g, float c, float s, in
 __global__ __launch_bounds__(kLineViews) void k_line_windows(LineGeo g, int tnx, int tny, int64_t nblk, const double *fcos,
                                                              const double *fsin, const int *vlist,
                                                              const int64_t *sub_row0, const int64_t *win0, int S,
-                                                             LineView *views, int *most) {
+                                                             int vstride, LineView *views, int *most) {
     const int64_t at = blockIdx.x;   // window * nblk + block
     const int64_t win = at / nblk;
     const int lb = (int)(at % nblk), lane = threadIdx.x;
@@ -600,68 +602,83 @@ __global__ __launch_bounds__(kLineViews) void k_line_windows(LineGeo g, int tnx,
         w.meta = line_meta(off + size, cand, axis);
         w.src = (vs + v) * (g.nbins + kLineEmpty) + b0 - off;
         w.row = v * g.nbins + b0 - off;
-        views[at * kLineViews + pos] = w;
+        views[at * vstride + pos] = w;
         if (i0 < g.nx && j0 < g.ny) atomicMax(most, cand > kLineEmpty ? INT32_MAX : size);
     }
 }
 
-// The line form of every ray; false (and nothing kept) when the geometry has
-// a ray without it, an image or sinogram beyond the kernels' 32-bit offsets, a
+// The line form of every ray; false when the geometry has a ray without it, or
+// an image or sinogram beyond the kernels' 32-bit offsets and the fixed point of
+// their positions.  windows: and the back projection's tables; false also for a
 // source too near (for the arc: the 45 degrees of its arc tangent), or bins so
 // fine that the rays of one view through a 16 x 16 pixel block do not fit the
 // back projection's LDS slots.
-bool try_lines(Matrix &m, const TraceArgs &a, hipStream_t st) {
+bool try_lines(Matrix &m, const TraceArgs &a, bool windows, hipStream_t st) {
     const mi_geometry &g = m.g;
-    if (!(g.pixel_mm > 0.0501) || (int64_t)(g.nx + 64) * (g.ny + 64) >= (int64_t)1 << 26) return false;
+    if (!(g.pixel_mm > 0.0501) || (int64_t)(g.nx + 64) * (g.ny + 64) >= (int64_t)1 << 26 || std::max(g.nx, g.ny) >= 1 << 18)
+        return false;
     Lines &q = m.lines;
     q.arc = g.beam == MI_BEAM_FAN_ARC;
     q.sod = (float)g.sod_mm;
     q.k = (float)(q.arc ? 180.0 / (M_PI * g.bin_mm) : g.sdd_mm / g.bin_mm);
-    // every corner of a block, also one that reaches past the image, lies in
-    // front of the source
-    const double rad = 0.5 * g.pixel_mm * std::hypot((double)g.nx, (double)g.ny), blk = 16 * M_SQRT2 * g.pixel_mm;
-    if (!(g.sod_mm - rad - blk > 0.02 * g.sod_mm)) return false;
     if (m.nrows + (int64_t)g.n_views * kLineEmpty >= (int64_t)1 << 30) return false;
-    if (q.arc && !(1.42 * (rad + g.pixel_mm) < g.sod_mm)) return false;
+    // the windows' blocks: every corner, also one that reaches past the image,
+    // lies in front of the source
+    const int tnx = (g.nx + kTileH - 1) / kTileH, tny = tiled_ny(g.ny);
+    const int64_t nblk = bp_blocks_of(tnx, tny);
+    int64_t wins = 0;
+    if (windows) {
+        const double rad = 0.5 * g.pixel_mm * std::hypot((double)g.nx, (double)g.ny), blk = 16 * M_SQRT2 * g.pixel_mm;
+        if (!(g.sod_mm - rad - blk > 0.02 * g.sod_mm)) return false;
+        if (q.arc && !(1.42 * (rad + g.pixel_mm) < g.sod_mm)) return false;
+        q.win0.assign(m.S + 1, 0);
+        int64_t most = 0;
+        for (int s = 0; s < m.S; ++s) {
+            const int64_t nv = (m.sub_row0[s + 1] - m.sub_row0[s]) / g.n_bins;
+            most = std::max(most, nv);
+            q.win0[s + 1] = q.win0[s] + (nv + kLineViews - 1) / kLineViews;
+        }
+        // small subsets: windows as short as the longest (720 subsets of one view
+        // at 512 x 512: 24 MB, 1.5 GB with windows of 64)
+        q.vstride = (int)std::min<int64_t>(most, kLineViews);
+        wins = q.win0.back() * nblk;
+        if (wins >= INT32_MAX / 8) return false;
+    }
     const int64_t per = (g.n_bins + kLineRays - 1) / kLineRays;
     q.slice0.assign(m.S + 1, 0);
     for (int s = 0; s < m.S; ++s) q.slice0[s + 1] = q.slice0[s] + 4 * per * ((m.sub_row0[s + 1] - m.sub_row0[s]) / g.n_bins);
     const int64_t groups = q.slice0.back() / 4;
     upload(q.d_slice0, q.slice0, st);
-    const int64_t entries = (int64_t)g.n_views * (g.n_bins + kLineEmpty);
     q.mb.alloc(m.nrows);
     q.len.alloc(m.nrows);
     q.inv.alloc(m.nrows);
     q.drop.alloc(m.nrows + kLineEmpty);   // read past a view's last bin
     q.skip.alloc(m.nrows);
     q.rng.alloc(groups);
-    for (auto *b : {&q.mx, &q.my}) b->alloc(entries);
-    for (auto *b : {&q.ix, &q.iy}) b->alloc(entries);
     MI_HIP(hipMemsetAsync(q.drop.p, 0xff, q.drop.bytes(), st));
-    // the empty entries: any finite line with weight 0
-    for (auto *b : {&q.mx, &q.my}) MI_HIP(hipMemsetAsync(b->p, 0, b->bytes(), st));
-    for (auto *b : {&q.ix, &q.iy}) MI_HIP(hipMemsetAsync(b->p, 0, b->bytes(), st));
-    q.win0.assign(m.S + 1, 0);
-    for (int s = 0; s < m.S; ++s)
-        q.win0[s + 1] = q.win0[s] + ((m.sub_row0[s + 1] - m.sub_row0[s]) / g.n_bins + kLineViews - 1) / kLineViews;
-    upload(q.d_win0, q.win0, st);
-    const int tnx = (g.nx + kTileH - 1) / kTileH, tny = tiled_ny(g.ny);
-    const int64_t nblk = bp_blocks_of(tnx, tny), wins = q.win0.back() * nblk;
-    if (wins >= INT32_MAX / 8) return false;
-    q.views.alloc(wins * kLineViews);
     DevBuf<int> flags(2);   // a ray without the form; the largest slot count
     MI_HIP(hipMemsetAsync(flags.p, 0, flags.bytes(), st));
-    MI_HIP(hipMemsetAsync(q.views.p, 0, q.views.bytes(), st));
+    if (windows) {
+        const int64_t entries = (int64_t)g.n_views * (g.n_bins + kLineEmpty);
+        for (auto *b : {&q.mx, &q.my}) b->alloc(entries);
+        for (auto *b : {&q.ix, &q.iy}) b->alloc(entries);
+        // the empty entries: any finite line with weight 0
+        for (auto *b : {&q.mx, &q.my}) MI_HIP(hipMemsetAsync(b->p, 0, b->bytes(), st));
+        for (auto *b : {&q.ix, &q.iy}) MI_HIP(hipMemsetAsync(b->p, 0, b->bytes(), st));
+        upload(q.d_win0, q.win0, st);
+        q.views.alloc(wins * q.vstride);
+        MI_HIP(hipMemsetAsync(q.views.p, 0, q.views.bytes(), st));
+        const double bin0 = q.arc ? g.n_bins / 2 - g.det_offset : g.n_bins / 2 - 0.5 - g.det_offset;
+        const LineGeo lg{g.nx, g.ny, g.n_bins, q.arc, (float)g.pixel_mm, q.sod, q.k, bin0};
+        k_line_windows<<<(unsigned)wins, kLineViews, 0, st>>>(lg, tnx, tny, nblk, a.fcos, a.fsin, a.vlist, m.d_sub_row0.p,
+                                                             q.d_win0.p, m.S, q.vstride, q.views.p, flags.p + 1);
+        MI_HIP(hipGetLastError());
+    }
     DevBuf<unsigned long long> nnz(m.S);
     MI_HIP(hipMemsetAsync(nnz.p, 0, nnz.bytes(), st));
     const LineOut o{q.mb.p, q.mx.p, q.my.p, q.ix.p, q.iy.p, q.len.p, q.inv.p, q.drop.p, q.skip.p, q.rng.p,
                     (unsigned *)flags.p, nnz.p};
     k_lines_fill<<<(unsigned)groups, kLineRays, 0, st>>>(a, m.d_sub_row0.p, q.d_slice0.p, m.S, o);
-    MI_HIP(hipGetLastError());
-    const double bin0 = q.arc ? g.n_bins / 2 - g.det_offset : g.n_bins / 2 - 0.5 - g.det_offset;
-    const LineGeo lg{g.nx, g.ny, g.n_bins, q.arc, (float)g.pixel_mm, q.sod, q.k, bin0};
-    k_line_windows<<<(unsigned)wins, kLineViews, 0, st>>>(lg, tnx, tny, nblk, a.fcos, a.fsin, a.vlist, m.d_sub_row0.p,
-                                                         q.d_win0.p, m.S, q.views.p, flags.p + 1);
     MI_HIP(hipGetLastError());
     int h[2] = {0, 0};
     std::vector<unsigned long long> n(m.S);
@@ -672,12 +689,6 @@ bool try_lines(Matrix &m, const TraceArgs &a, hipStream_t st) {
     m.sub_nnz.assign(n.begin(), n.end());
     m.nnz = std::accumulate(m.sub_nnz.begin(), m.sub_nnz.end(), (int64_t)0);
     return m.has_lines = true;
-}
-
-bool build_lines(Matrix &m, const TraceArgs &a, hipStream_t st) {
-    if (try_lines(m, a, st)) return true;
-    m.lines = Lines{};
-    return false;
 }
 
 // Entries of each subset's rows, from the device row pointer.
@@ -833,15 +844,12 @@ std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, h
         a.psin = psin.p;
     }
 
-    // FP32 engine runs of a fan beam project along the lines and need no
-    // matrix; FP64 runs, and geometries with a ray that has no line form, re-run
+    // FP32 projections and engine runs of a fan beam go along the lines and need
+    // no matrix; FP64 runs, and geometries with a ray that has no line form, re-run
     // the tracer from checkpoints and read the matrix.
     const bool fan = g.beam == MI_BEAM_FAN_FLAT || g.beam == MI_BEAM_FAN_ARC;
-    if (layout != 0 && fan && build_lines(*m, a, st) && !want64) {
-        m->has_csr = false;
-        return m;
-    }
-    if (layout == 2) {
+    if (layout >= 2) {
+        if (!fan || !try_lines(*m, a, layout == 3, st)) m->lines = Lines{};
         m->has_csr = false;
         return m;
     }

@@ -1,12 +1,16 @@
-"""Fan-beam reconstructions along lines at the limits of that form against the
-FP64 oracle.  The bar is that of the line form's other comparison (2e-6 after
-12 updates)."""
+"""Which fan-beam geometries go along lines, at the limits of that form; what
+its tables hold; and its results there against the FP64 oracle.
+
+The form shows in the context's memory: a stored matrix holds at least 8 bytes
+an entry (index and length), the lines some 100 bytes a ray and 32 bytes a
+block and view.  The bar of a reconstruction is that of the line form's other
+comparison (2e-6 after 12 updates)."""
 import numpy as np
 import pytest
 
 import medimage_amd as mi
 import oracle_py as O
-from test_gpu_lines import _fan
+from test_gpu_lines import GEOMS, _fan
 
 pytestmark = pytest.mark.gpu
 
@@ -21,6 +25,19 @@ EDGE = {
     "long_detector": _fan(48, 48, 4.0, 2, 16000001, 4.0, off=0.3),
     "view_pairs": _fan(80, 80, 3.0, 9, 111, 3.3),
 }
+LINES = ["square", "wide", "half_turn", "two_groups", "one_group", "arc", "coarse_bins", "eight_rays", "near_source", "wide_arc",
+         "view_pairs"]
+MATRIX = ["source_in_corner", "fine_pixels", "arc_wide", "fine_bins"]
+
+
+@pytest.mark.parametrize("name", LINES + MATRIX)
+def test_line_form(ctx, name):
+    g = {**GEOMS, **EDGE}[name]
+    ctx.trim()
+    nnz, mem = ctx.prepare(g, 4), ctx.mem_bytes()
+    print(f"[line form {name}] {nnz} entries, {mem} bytes", flush=True)
+    assert (mem < 8 * nnz) == (name in LINES)
+
 
 @pytest.mark.parametrize("name,subsets", [("eight_rays", 4), ("near_source", 4), ("wide_arc", 4), ("long_detector", 1),
                                           ("view_pairs", 9), ("view_pairs", 8), ("view_pairs", 4)])
@@ -38,3 +55,39 @@ def test_line_limits_match_oracle(ctx, name, subsets):
     print(f"[line limits {name} {subsets}] u {eu:.1e} v {ev:.1e}", flush=True)
     assert eu < 2e-6 and ev < 2e-6
     assert abs(rep.data_fidelity - hist[-1]) <= 1e-5 * hist[-1]
+
+
+def test_line_tables(ctx):
+    """Subsets of one view need no more room than larger ones; a forward
+    projection none of the back projection's tables; an FP64 run no lines."""
+    g = mi.fan_geometry(512, 0.7, 720, 736, 1.0)
+    rows = g.n_views * g.n_bins
+    ctx.trim()
+    ctx.prepare(g, 12)
+    few = ctx.mem_bytes()
+    ctx.trim()
+    ctx.prepare(g, 720)
+    many = ctx.mem_bytes()
+    print(f"[line tables] 12 subsets {few}, 720 subsets {many} bytes", flush=True)
+    assert many < 1.1 * few
+    ctx.trim()
+    ctx.forward(g, np.zeros((512, 512), np.float32))
+    one = ctx.mem_bytes()
+    print(f"[line tables] forward {one} bytes", flush=True)
+    assert one < 60 * rows
+    ctx.trim()
+    small = GEOMS["square"]
+    nnz = ctx.prepare(small, 4)
+    lines = ctx.mem_bytes()
+    sino = np.random.default_rng(1).random((small.n_views, small.n_bins))
+    p32 = mi.at_params(n_subsets=4, max_iters=2)
+    p64 = mi.at_params(n_subsets=4, max_iters=2, precision=mi.MI_FP64)
+    before = ctx.at_reconstruct(small, sino.astype(np.float32), p32)
+    ctx.at_reconstruct(small, sino, p64)
+    both = ctx.mem_bytes()
+    after = ctx.at_reconstruct(small, sino.astype(np.float32), p32)
+    assert ctx.mem_bytes() == both > lines
+    assert np.array_equal(before[0], after[0]) and np.array_equal(before[1], after[1])
+    ctx.trim()
+    ctx.at_reconstruct(small, sino, p64)
+    assert ctx.mem_bytes() == both - lines
