@@ -685,30 +685,13 @@ __global__ __launch_bounds__(kBlock) void k_cone_bp(ConeDev g, const float *cs, 
 // 0.94; 64^3 x 100: 0.91 and 0.30.  Against 64-bit sums of the exact lengths
 // both are off by 4.9e-7 of the largest voxel at 128^3.
 constexpr int kConeRun = 24, kConeStep = 4;   // rows of a patch column per lane: at most, a multiple of
-constexpr float kConeRange = 7.62939453125e-6f;   // 2^-17
+constexpr double kConeBits = 9.313225746154785e-10;   // 2^-30
 constexpr int kConeBatch = 5;                 // planes whose LDS reads are issued together (9: 4% slower at C4)
 struct ConeView {
     int col0, ncol, r0, nr;       // the patch: panel columns, rows
     int run, cand;                // rows per lane; candidate columns of a voxel column
     float hw, icol;               // half width of a voxel column's shadow, 1 / ncol
 };
-
-// The largest x >= 0 of the wave's lanes.
-__device__ __forceinline__ float wave_top(float x) {
-    auto step = [&](auto ctrl, auto rows) {
-        const int o = __builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, decltype(rows)::value, 0xf, true);
-        x = fmaxf(x, __int_as_float(o));
-    };
-    using std::integral_constant;
-    const integral_constant<int, 0xf> all;
-    step(integral_constant<int, 0x111>{}, all);   // row_shr:1, 2, 4, 8
-    step(integral_constant<int, 0x112>{}, all);
-    step(integral_constant<int, 0x114>{}, all);
-    step(integral_constant<int, 0x118>{}, all);
-    step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});   // row_bcast:15, 31
-    step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
-}
 
 // A value that all lanes hold, in scalar registers.
 __device__ __forceinline__ double uniform(double x) {
@@ -782,12 +765,14 @@ __global__ __launch_bounds__(kWave) void k_cone_patch(ConeDev g, const float *cs
 
 // LDS of a workgroup: the running sums (column major; one entry before the
 // first row and one behind the last), 1 / w and w^2 of the rows its views
-// see, 1 / (d - s) per column, the lanes' totals, the views.
+// see, 1 / (d - s) per column, the lanes' totals and absolute totals, the
+// columns' absolute totals, the views.
 constexpr int kConeViews = 36;
 __host__ __device__ __forceinline__ int cone_patch_stride(int rows) { return (rows + 3) | 1; }
 __host__ __device__ __forceinline__ size_t cone_patch_lds(int cols, int rows, int span) {
     const size_t sums = ((size_t)cols * cone_patch_stride(rows) + 1) & ~(size_t)1;
-    const size_t need = 8 * (sums + 2 * (size_t)cols + kBlock + span + 2) + 4 * (size_t)(span + 2) + kConeViews * sizeof(ConeView);
+    const size_t need = 8 * (sums + 2 * (size_t)cols + kBlock + span + 2) + 4 * (size_t)(span + 2 + kBlock + cols) +
+                        kConeViews * sizeof(ConeView);
     return need > kZc * kBlock * 8 ? need : kZc * kBlock * 8;   // (the sums of the ray by ray form)
 }
 
@@ -805,7 +790,7 @@ __device__ __forceinline__ void cone_bp_block(
     double2 *irs = (double2 *)(PS + ((cols * stride + 1) & ~1));
     double *tots = (double *)(irs + cols), *iws = tots + kBlock;
     ConeView *info = (ConeView *)(iws + span_rows + 2);
-    float *w2s = (float *)(info + kConeViews);
+    float *w2s = (float *)(info + kConeViews), *atots = w2s + span_rows + 2, *acols = atots + kBlock;
     __shared__ int sh_r0, sh_r1;
     const float kcol = g.sdd / g.pixel, kz = g.sample / g.pixel, sodv = g.sod / g.sample, h5 = (float)g.halfdet - 0.5f;
     const float px = (float)x + 0.5f - g.nx / 2.0f, py = (float)y + 0.5f - g.ny / 2.0f;
@@ -827,8 +812,8 @@ __device__ __forceinline__ void cone_bp_block(
     // this lane's part of view iv's patch, into registers (rows behind its
     // run are other lanes', rows behind the panel read as 0)
     int v0 = 0;
-    bool bad = false;   // a sum of this lane was not finite, or the values differ too much
-    float top = 0.0f, low = INFINITY;   // largest value of the wave's lanes in any view, the least such of a well filled view
+    bool bad = false;   // a sum of this lane was not finite, or one of its voxels lost too many bits
+    float size = 0.0f;  // what the planes' sums may have held: the columns' absolute sums, by the chords
     auto load = [&](int iv) {
         const ConeView w = info[iv];
         const int seg = (int)(((float)tid + 0.5f) * w.icol), col = tid - seg * w.ncol;   // tid / ncol
@@ -889,7 +874,7 @@ __device__ __forceinline__ void cone_bp_block(
             const int r = seg * w.run;
             const bool any = r < w.nr;
             double sum = 0.0;
-            float most = 0.0f;   // largest value of this lane's run
+            float mag = 0.0f;
             if (any) {
                 const float *w2 = w2s + (w.r0 - rbase + r + 1);
 #pragma unroll
@@ -899,29 +884,23 @@ __device__ __forceinline__ void cone_bp_block(
                         for (int h = i; h < i + kConeStep; ++h) {
                             raw[h] *= __builtin_amdgcn_sqrtf(w2[h] + l2);
                             sum += (double)raw[h];
-                            most = fmaxf(most, fabsf(raw[h]));
+                            mag += fabsf(raw[h]);
                             asm volatile("" : "+v"(raw[h]));   // (converted again below: not 24 doubles kept)
                         }
             }
             bad |= !(fabs(sum) < INFINITY);
-            // A few values far above the others would take the others' last
-            // bits in the running sums and the planes' (some 3e-13 of the
-            // largest over 720 views): a sixteenth of a wave's runs below
-            // 2^-17 of its largest, or views that differ so, and the block's
-            // voxels go ray by ray.
-            const float wtop = wave_top(most);
-            const int filled = __popcll(__ballot(most > 0.0f));
-            bad |= 16 * __popcll(__ballot(most > 0.0f && most < wtop * kConeRange)) > filled;
-            top = fmaxf(top, wtop);
-            if (filled >= kWave / 2) low = fminf(low, wtop);
             tots[tid] = sum;
+            atots[tid] = mag;
             // a ray along an axis: all or nothing on the other, by a huge finite
             // inverse (0 x infinity has no value)
             if (tid < w.ncol) irs[tid] = make_double2(fmin(fmax(ir.x, -1e300), 1e300), fmin(fmax(ir.y, -1e300), 1e300));
             __syncthreads();
             if (any) {
                 double run = 0.0;
-                for (int i = 0; i < seg; ++i) run += tots[i * w.ncol + col];
+                for (int i = 0; i < seg; ++i) {
+                    run += tots[i * w.ncol + col];
+                    mag += atots[i * w.ncol + col];
+                }
                 double *P = PS + col * stride + 2 + r;   // P[i]: the rows up to r + i
                 if (seg == 0) P[-2] = P[-1] = 0.0;
 #pragma unroll
@@ -929,7 +908,10 @@ __device__ __forceinline__ void cone_bp_block(
                     if (i < w.run)
 #pragma unroll
                         for (int h = i; h < i + kConeStep; ++h) P[h] = run += (double)raw[h];
-                if (r + w.run == w.nr) P[w.run] = run;
+                if (r + w.run == w.nr) {
+                    P[w.run] = run;
+                    acols[col] = mag;
+                }
             }
             __syncthreads();
             if (iv + 1 < ng) load(iv + 1);
@@ -950,6 +932,7 @@ __device__ __forceinline__ void cone_bp_block(
                 const float span = (in && hi > lo) ? (float)(hi - lo) : 0.0f;
                 if (!__any(span > 0.0f)) continue;
                 const float inv = span > 0.0f ? (__builtin_amdgcn_rcpf((float)lo) + __builtin_amdgcn_rcpf((float)hi)) * (0.5f * kz) : 0.0f;
+                size = __builtin_fmaf(span, acols[lc], size);
                 const double spand = (double)span, nlo = -lo, base = over ? hi : nlo;
                 const double *P = PS + lc * stride;
                 const float last = (float)(w.nr + 1);
@@ -990,7 +973,15 @@ __device__ __forceinline__ void cone_bp_block(
             __syncthreads();   // the patch is written again
         }
     }
-    bad |= low < top * kConeRange;
+    // A voxel is the difference of two planes' sums, which keep some 47 bits of
+    // `size`: where it is below 2^-30 of it, a few values far above the others
+    // were in the sums.  (0 is exact: the two planes summed alike.)  Positive data
+    // has it at 2^-6, noise about 2^-11.
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+        const double d = fabs(A[k] - A[k + 1]);
+        bad |= x < g.nx && y < g.ny && z0 + k < g.nz && d != 0.0 && d < (double)size * kConeBits;
+    }
     if (__syncthreads_or(bad)) {
         // A value that is not finite, or far above the others, would reach every
         // row behind it through the running sums: the block's voxels ray by ray

@@ -66,3 +66,22 @@ def test_cone_patch_single_view_scale(ctx):
     assert (~hit).any()
     assert np.abs(dev - off)[~hit].max() < 1e-5 * np.abs(off).max()
     assert np.abs(dev - ref)[hit].max() < 1e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("value", [1e10, 1e25])
+def test_cone_patch_sparse(ctx, value):
+    """Two rays alone, one far larger: voxels on the smaller one's only."""
+    g = GEOMS[0]
+    print(f"cone back projection, two rays, {value}", flush=True)
+    at, to = (5, g.n_rows // 2 - 4, 30), (29, g.n_rows // 2 + 6, 33)
+    sino = np.zeros((g.n_views, g.n_rows, g.n_cols), np.float32)
+    sino[at] = 1.0
+    small = O.cone_bp(O.cone_from(g), sino.astype(np.float64))
+    sino[to] = value
+    dev = ctx.cone_backproject(g, sino).astype(np.float64)
+    sino[at] = 0.0
+    big = O.cone_bp(O.cone_from(g), sino.astype(np.float64))
+    only = (big == 0) & (small != 0)
+    assert only.any()
+    assert np.abs(dev - small)[only].max() < 1e-5 * small.max()
+    assert not dev[(big == 0) & (small == 0)].any()
