@@ -2,7 +2,7 @@
 
 Workload: the precision form (C2): 512 x 512 image, 0.7 mm pixels, 720 views
 over 360 degrees, 736 detector bins of 1.0 mm, flat fan beam (SOD 541 mm,
-SDD 949 mm), 12 ordered subsets, FP32 bulk with Kahan sums and FP64
+SDD 949 mm), 12 ordered subsets, FP32 images and sinogram, projections in FP64, FP64
 reductions.  One step = one AT iteration (a pass over all 12 subsets: forward
 projection, residual, gather back projection + image gradient, line search,
 image update; then one edge step) of one job whose sinogram and state are
@@ -31,6 +31,7 @@ sys.path.insert(0, str(ROOT))
 import numpy as np  # noqa: E402
 
 HBM_PEAK_GBS = 8000.0
+VALU_PEAK = 256 * 4 * 2.4 / 4   # G wave instructions/s: one every four clocks and SIMD
 METRIC = "AT iters/sec & rays/sec (512², 720 views) plain vs batched; p50/p99 job latency"
 
 
@@ -692,12 +693,21 @@ def main():
     # HBM bytes per launch of the same kernel on the same workload, from the
     # rocprofv3 FETCH_SIZE / WRITE_SIZE runs (calibrated against a plain copy
     # kernel) recorded next to the kernel statistics.
-    traffic = None
+    # The projectors along lines stream nothing: they are measured against the
+    # vector units' issue rate, by the wave instructions of a launch (SQ_INSTS_VALU
+    # of the same profile) over this run's launch time.
+    tk = None
     tfile = ROOT / "profiles" / "c2_plain_traffic.json"
     if tfile.exists():
         tk = json.loads(tfile.read_text())["kernels"].get(kernel_symbol[dom])
-        if tk:
-            traffic = tk["traffic_bytes"]
+    traffic = tk["traffic_bytes"] if tk else None
+    if tk and tk.get("valu_instructions"):
+        rate = tk["valu_instructions"] / (avg_ms * 1e-3) / 1e9
+        roof = {"bound": "valu", "kernel": kernel_symbol[dom], "achieved": rate, "peak": VALU_PEAK,
+                "unit": "G wave instructions/s", "frac": rate / VALU_PEAK}
+    else:
+        roof = {"bound": "hbm", "kernel": kernel_symbol[dom], "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                "frac": achieved / HBM_PEAK_GBS}
     rays = g.n_views * g.n_bins
     out = {
         "metric": METRIC,
@@ -716,10 +726,9 @@ def main():
                                "SOD 541 mm, SDD 949 mm, 12 ordered subsets, alpha 1e-3, beta 1e-4, eps 1e-2",
                    "rays": rays, "nnz": nnz, "subsets": 12},
         "rays_per_s": rays * args.steps / elapsed,
-        "roofline": {"bound": "hbm", "kernel": kernel_symbol[dom], "achieved": achieved, "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "traffic_source": "profiles/c2_plain_traffic.json" if traffic else None,
-                     "bytes_per_launch": bytes_per, "avg_launch_us": avg_ms * 1e3,
+        "roofline": {**roof, "traffic": traffic,
+                     "counters": "profiles/c2_plain_traffic.json" if tk else None,
+                     "bytes_per_launch": bytes_per, "GBps": achieved, "avg_launch_us": avg_ms * 1e3,
                      "launches_timed": s.launches},
         "kernels": per_kernel,
     }

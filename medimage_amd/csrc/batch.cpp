@@ -623,8 +623,9 @@ bool Batch<T>::class_bp(int c) const {
     return y;
 }
 
-// Algorithmic bytes of one launch summed over the live units (instrumented
-// runs only).
+// Bytes of one launch summed over the live units (instrumented runs only):
+// each array that the launch reads or writes counted once; of a stored matrix
+// its entries (index and length), also where they are recomputed by the walk.
 template <typename T>
 void Batch<T>::record_pass(bool timed) {
     const hipStream_t st = ctx->stream;
@@ -651,6 +652,21 @@ void Batch<T>::record_pass(bool timed) {
             if (has1) launch1(st);
         }
     };
+    // Units with lines read their rays' numbers instead of a matrix.
+    auto fp_bytes = [&](const Unit<T> &U, int s, bool resid) {
+        const Matrix &m = *U.m;
+        const double nr = (double)(m.sub_row0[s + 1] - m.sub_row0[s]);
+        if (!use_lines<T>(m))
+            return m.sub_nnz[s] * (4 + sz) + m.npix * sz * U.K + (resid ? 2 * nr * sz * U.K : 0.0);
+        return line_ray_bytes(nr) + m.npix * (resid ? (U.K <= 2 ? 8.0 : 6.0) : 4.0) * U.K + (resid ? 2 * nr * sz * U.K : 0.0);
+    };
+    auto bp_bytes = [&](const Unit<T> &U, int s) {
+        const Matrix &m = *U.m;
+        const double nr = (double)(m.sub_row0[s + 1] - m.sub_row0[s]);
+        if (!use_lines<T>(m)) return m.sub_nnz[s] * (4 + sz) + nr * sz * U.K + 3.0 * m.npix * sz * U.K;
+        // a line and 1 / |m| a ray, the blocks' views, r; u, v, d, its remainder, two projection images
+        return nr * 20.0 + (nr / m.g.n_bins) * (double)bp_blocks(m) * sizeof(LineView) + nr * sz * U.K + 6.0 * m.npix * sz * U.K;
+    };
     // the units with lines (FP32) of class c
     auto line_fp = [&](hipStream_t q, int c, int s, bool resid) {
         if constexpr (sizeof(T) == 4) {
@@ -666,12 +682,8 @@ void Batch<T>::record_pass(bool timed) {
         }
     };
     for (int s = 0; s < S; ++s) {
-        auto nnz_s = [&](const Unit<T> &U) { return (double)U.m->sub_nnz[s]; };
-        auto nr_s = [&](const Unit<T> &U) { return (double)(U.m->sub_row0[s + 1] - U.m->sub_row0[s]); };
         {
-            LaunchTimer lt(ctx, MI_K_FP, sum([&](const Unit<T> &U) {
-                return nnz_s(U) * (4 + sz) + U.m->npix * sz * U.K + 2 * nr_s(U) * sz * U.K;
-            }), true);
+            LaunchTimer lt(ctx, MI_K_FP, sum([&](const Unit<T> &U) { return fp_bytes(U, s, true); }), true);
             auto one = [&](int c) {
                 return [&, c](hipStream_t q) {
                     if (rows[c].any()) eng_fp_resid<T>(q, args, rows[c].map, s, rows[c].kmax, all_walk);
@@ -681,9 +693,7 @@ void Batch<T>::record_pass(bool timed) {
             branches(one(0), one(1), class_fp(0), class_fp(1));
         }
         {
-            LaunchTimer lt(ctx, MI_K_BP, sum([&](const Unit<T> &U) {
-                return nnz_s(U) * (4 + sz) + nr_s(U) * sz * U.K + 3.0 * U.m->npix * sz * U.K;
-            }), true);
+            LaunchTimer lt(ctx, MI_K_BP, sum([&](const Unit<T> &U) { return bp_bytes(U, s); }), true);
             auto one = [&](int c) {
                 return [&, c](hipStream_t q) {
                     for (const Launch &L : bpl[c])
@@ -695,9 +705,7 @@ void Batch<T>::record_pass(bool timed) {
             branches(one(0), one(1), class_bp(0), class_bp(1));
         }
         {
-            LaunchTimer lt(ctx, MI_K_FPSQ, sum([&](const Unit<T> &U) {
-                return nnz_s(U) * (4 + sz) + U.m->npix * sz * U.K;
-            }), true);
+            LaunchTimer lt(ctx, MI_K_FPSQ, sum([&](const Unit<T> &U) { return fp_bytes(U, s, false); }), true);
             auto one = [&](int c) {
                 return [&, c](hipStream_t q) {
                     if (rows[c].any()) eng_fp_sq<T>(q, args, rows[c].map, s, rows[c].kmax, all_walk);

@@ -354,7 +354,7 @@ void forward_impl(mi_context *ctx, const mi_geometry *g, const T *img, T *sino) 
                 DevBuf<float> buf(m.npix + ex + ey), out(m.nrows);
                 MI_HIP(hipMemcpyAsync(buf.p, img, m.npix * sizeof(T), hipMemcpyHostToDevice, st));
                 {
-                    LaunchTimer lt(ctx, MI_K_FP, fp_bytes(m, m.nrows, sizeof(T), FP_WRITE));
+                    LaunchTimer lt(ctx, MI_K_FP, line_ray_bytes(m.nrows) + 4.0 * (m.npix + m.nrows));
                     line_project(st, m, buf.p, buf.p + m.npix, buf.p + m.npix + ex, out.p);
                 }
                 MI_HIP(hipMemcpyAsync(sino, out.p, m.nrows * sizeof(T), hipMemcpyDeviceToHost, st));

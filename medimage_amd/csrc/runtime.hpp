@@ -230,6 +230,10 @@ struct Lines {
     }
 };
 
+// What a forward projection reads of `rows` rays: m, b0, 1 / |m|, the length and
+// the left-out line.
+inline double line_ray_bytes(double rows) { return rows * (16 + 8 + 8 + 4); }
+
 constexpr int kGroup = 4;
 __host__ __device__ __forceinline__ int64_t sell_pos(int64_t base, int t, int lane) {
     return base + (int64_t)(t >> 2) * (kGroup * 64) + lane * kGroup + (t & 3);

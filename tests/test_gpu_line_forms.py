@@ -91,3 +91,26 @@ def test_line_tables(ctx):
     ctx.trim()
     ctx.at_reconstruct(small, sino, p64)
     assert ctx.mem_bytes() == both - lines
+
+
+def test_line_bytes(ctx):
+    """A timed launch reports what it reads and writes, not a matrix's entries."""
+    g = mi.fan_geometry(256, 1.4, 360, 512, 1.44)
+    ctx.trim()
+    nnz = ctx.prepare(g, 1)
+    job = ctx.job(g, np.ones((g.n_views, g.n_bins), np.float32), mi.at_params(n_subsets=1, max_iters=2))
+    ctx.stats_reset()
+    ctx.stats_enable(True)
+    job.enqueue(1)
+    job.synchronize()
+    ctx.forward(g, np.ones((256, 256), np.float32))
+    ctx.stats_enable(False)
+    fp, bp, sq = (ctx.stats(k) for k in (mi.MI_K_FP, mi.MI_K_BP, mi.MI_K_FPSQ))
+    job.close()
+    rows, pix = g.n_views * g.n_bins, g.nx * g.ny
+    print(f"[line bytes] {nnz} entries; {fp.bytes} {bp.bytes} {sq.bytes}", flush=True)
+    assert (fp.launches, bp.launches, sq.launches) == (2, 1, 1)
+    assert sq.bytes == 36.0 * rows + 4 * pix
+    assert fp.bytes == 36.0 * rows + 8 * pix + 8 * rows + 36.0 * rows + 4 * (pix + rows)
+    assert bp.bytes == 24.0 * rows + 32.0 * 256 * g.n_views + 24 * pix
+    assert max(fp.bytes, bp.bytes, sq.bytes) < 4 * nnz
