@@ -46,6 +46,7 @@
 
 #include <mutex>
 
+#include <cfloat>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -519,6 +520,7 @@ __device__ __forceinline__ void cone_bp_voxels(const ConeDev &g, const float *cs
     // nk <= kZc: the slices from z0.
     // carry: the double sums of the earlier view chunks of a back projection
     // split into several launches (nullptr for a single launch).
+    // vol nullptr: the sums stay in acc.
 #pragma unroll
     for (int k = 0; k < kZc; ++k)
         acc[k][threadIdx.x] = (carry && !first && k < nk) ? carry[((size_t)(z0 + k) * g.nx + x) * g.ny + y] : 0.0;
@@ -620,6 +622,7 @@ __device__ __forceinline__ void cone_bp_voxels(const ConeDev &g, const float *cs
             }
         }
     }
+    if (vol == nullptr) return;
     for (int k = 0; k < nk; ++k) {
         const size_t i = ((size_t)(z0 + k) * g.nx + x) * g.ny + y;
         if (carry && !last) carry[i] = acc[k][threadIdx.x];
@@ -679,13 +682,16 @@ __global__ __launch_bounds__(kBlock) void k_cone_bp(ConeDev g, const float *cs, 
 // everything else is fixed by the geometry.
 //
 // Bounded by LDS reads (24 bytes per lane, plane and column, 12 clocks of a
-// CU per wave) and vector issue in about equal parts; two or three workgroups
-// per CU, which the patches' LDS allows.  512^3, 720 views of 1024 x 768: 508
-// ms ray by ray, 152 so; 256^3 x 360: 35.5 and 10.1; 128^3 x 180: 3.83 and
-// 0.94; 64^3 x 100: 0.91 and 0.30.  Against 64-bit sums of the exact lengths
+// CU per wave: 64% of the clocks) and vector issue (75%); two or three
+// workgroups per CU, which the patches' LDS allows.  512^3, 720 views of 1024
+// x 768: 508 ms ray by ray, 177 so; 256^3 x 360: 35.5 and 13.0; 128^3 x 180:
+// 3.83 and 1.04; 64^3 x 100: 0.91 and 0.33.  Against 64-bit sums of the exact lengths
 // both are off by 4.9e-7 of the largest voxel at 128^3.
 constexpr int kConeRun = 24, kConeStep = 4;   // rows of a patch column per lane: at most, a multiple of
 constexpr double kConeBits = 9.313225746154785e-10;   // 2^-30
+constexpr double kConeUlp = 8.881784197001252e-16;    // 2^-50
+constexpr int kConeMany = 8;                  // voxels that lost bits, from which on 0 counts as one
+constexpr int kConeFew = 512;                 // voxels of a block done again one by one, at most
 constexpr int kConeBatch = 5;                 // planes whose LDS reads are issued together (9: 4% slower at C4)
 struct ConeView {
     int col0, ncol, r0, nr;       // the patch: panel columns, rows
@@ -773,15 +779,38 @@ __host__ __device__ __forceinline__ size_t cone_patch_lds(int cols, int rows, in
     const size_t sums = ((size_t)cols * cone_patch_stride(rows) + 1) & ~(size_t)1;
     const size_t need = 8 * (sums + 2 * (size_t)cols + kBlock + span + 2) + 4 * (size_t)(span + 2 + kBlock + cols) +
                         kConeViews * sizeof(ConeView);
-    return need > kZc * kBlock * 8 ? need : kZc * kBlock * 8;   // (the sums of the ray by ray form)
+    const size_t again = kZc * kBlock * 8 + kConeFew * 4;   // (the sums of the ray by ray form, the voxels it does)
+    return need > again ? need : again;
 }
 
+struct ConePatchArgs {
+    ConeDev g;
+    const float *cs;
+    const double *rowtab;
+    const double2 *vinv;
+    const float *vl2;
+    const float4 *vsrc;
+    const int *views;
+    const float *sino;
+    float *vol;
+    int nv, cols, rows, span_rows;
+};
+
+// The planes' sums A of a block's voxel columns, what they may have held
+// (size); true if a sum of this lane was not finite.
 // CROSS: the source's height lies within the block's slices.
 template <int NK, bool CROSS>
-__device__ __forceinline__ void cone_bp_block(
-    const ConeDev &g, const float *cs, const double *rowtab, const double2 *__restrict__ vinv, const float *__restrict__ vl2,
-    const float4 *__restrict__ vsrc, const int *views, int nv, const float *__restrict__ sino, float *__restrict__ vol,
-    int cols, int rows, int span_rows, int x0, int y0, int z0) {
+__device__ __forceinline__ bool cone_bp_block(const ConePatchArgs &t, int x0, int y0, int z0, double (&A)[NK + 1],
+                                              float &size) {
+    const ConeDev &g = t.g;
+    const float *cs = t.cs;
+    const double *rowtab = t.rowtab;
+    const double2 *__restrict__ vinv = t.vinv;
+    const float *__restrict__ vl2 = t.vl2;
+    const float4 *__restrict__ vsrc = t.vsrc;
+    const float *__restrict__ sino = t.sino;
+    const int *views = t.views;
+    const int nv = t.nv, cols = t.cols, rows = t.rows, span_rows = t.span_rows;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int x = x0 + (wv >> 1) * 8 + (lane >> 3), y = y0 + (wv & 1) * 8 + (lane & 7);
     extern __shared__ double smem[];
@@ -800,7 +829,7 @@ __device__ __forceinline__ void cone_bp_block(
     const float dz0 = (float)z0 - g.nz / 2.0f;
     const bool over = dz0 >= 0.0f;
     const int kover = __builtin_amdgcn_readfirstlane((int)floorf(-dz0) + 1);   // the first plane over the source
-    double A[NK + 1], mdZ[NK + 1];
+    double mdZ[NK + 1];
 #pragma unroll
     for (int k = 0; k <= NK; ++k) {
         A[k] = 0.0;
@@ -812,8 +841,8 @@ __device__ __forceinline__ void cone_bp_block(
     // this lane's part of view iv's patch, into registers (rows behind its
     // run are other lanes', rows behind the panel read as 0)
     int v0 = 0;
-    bool bad = false;   // a sum of this lane was not finite, or one of its voxels lost too many bits
-    float size = 0.0f;  // what the planes' sums may have held: the columns' absolute sums, by the chords
+    bool bad = false;   // a sum of this lane was not finite
+    size = 0.0f;        // the columns' absolute sums, by the chords
     auto load = [&](int iv) {
         const ConeView w = info[iv];
         const int seg = (int)(((float)tid + 0.5f) * w.icol), col = tid - seg * w.ncol;   // tid / ncol
@@ -910,7 +939,7 @@ __device__ __forceinline__ void cone_bp_block(
                         for (int h = i; h < i + kConeStep; ++h) P[h] = run += (double)raw[h];
                 if (r + w.run == w.nr) {
                     P[w.run] = run;
-                    acols[col] = mag;
+                    acols[col] = fminf(mag, FLT_MAX);   // (times 0: 0)
                 }
             }
             __syncthreads();
@@ -973,53 +1002,120 @@ __device__ __forceinline__ void cone_bp_block(
             __syncthreads();   // the patch is written again
         }
     }
-    // A voxel is the difference of two planes' sums, which keep some 47 bits of
-    // `size`: where it is below 2^-30 of it, a few values far above the others
-    // were in the sums.  (0 is exact: the two planes summed alike.)  Positive data
-    // has it at 2^-6, noise about 2^-11.
-#pragma unroll
-    for (int k = 0; k < NK; ++k) {
-        const double d = fabs(A[k] - A[k + 1]);
-        bad |= x < g.nx && y < g.ny && z0 + k < g.nz && d != 0.0 && d < (double)size * kConeBits;
-    }
-    if (__syncthreads_or(bad)) {
-        // A value that is not finite, or far above the others, would reach every
-        // row behind it through the running sums: the block's voxels ray by ray
-        // instead.
-        const int zend = min(z0 + NK, g.nz);
-        for (int z = z0; z < zend; z += kZc) {
-            if (x >= g.nx || y >= g.ny) break;
-            cone_bp_voxels<false, false>(g, cs, rowtab, vinv, vl2, vsrc, nullptr, views, nv, sino, nullptr, 1, 1, vol, x, y,
-                                         z, min(kZc, zend - z), nullptr, (double(*)[kBlock])smem);
-        }
-        return;
-    }
-    if (x >= g.nx || y >= g.ny) return;
-    const int nk = min(NK, g.nz - z0);
-#pragma unroll
-    for (int k = 0; k < NK; ++k)
-        if (k < nk) {
-            const size_t i = ((size_t)(z0 + k) * g.nx + x) * g.ny + y;
-            vol[i] = (float)(A[k] - A[k + 1]);
-        }
+    return bad;
 }
 
 template <int NK>
-__global__ __launch_bounds__(kBlock) void k_cone_bp_patch(
-    ConeDev g, const float *cs, const double *rowtab, const double2 *__restrict__ vinv, const float *__restrict__ vl2,
-    const float4 *__restrict__ vsrc, const int *views, int nv, const float *__restrict__ sino, float *__restrict__ vol,
-    int cols, int rows, int span_rows) {
-    const int tx = (g.nx + 15) / 16, ty = (g.ny + 15) / 16;
+__global__ __launch_bounds__(kBlock) void k_cone_bp_patch(ConePatchArgs args) {
     const unsigned blk = xcd_block();
-    const int z0 = (int)(blk / (tx * ty)) * NK, tile = (int)(blk % (tx * ty));
-    if (z0 >= g.nz) return;
+    const int ty = (args.g.ny + 15) / 16, txy = (args.g.nx + 15) / 16 * ty;
+    const int z0 = (int)(blk / txy) * NK, tile = (int)(blk % txy);
+    if (z0 >= args.g.nz) return;
     const int x0 = (tile / ty) * 16, y0 = (tile % ty) * 16;
-    if (2 * z0 < g.nz && 2 * (z0 + NK) > g.nz)
-        cone_bp_block<NK, true>(g, cs, rowtab, vinv, vl2, vsrc, views, nv, sino, vol, cols, rows, span_rows,
-                                x0, y0, z0);
-    else
-        cone_bp_block<NK, false>(g, cs, rowtab, vinv, vl2, vsrc, views, nv, sino, vol, cols, rows, span_rows,
-                                 x0, y0, z0);
+    double A[NK + 1];
+    float size;
+    bool bad = 2 * z0 < args.g.nz && 2 * (z0 + NK) > args.g.nz ? cone_bp_block<NK, true>(args, x0, y0, z0, A, size)
+                                                               : cone_bp_block<NK, false>(args, x0, y0, z0, A, size);
+    // The arguments are read again from here: kept over the views' loop they
+    // had scalar registers going to and fro in it (512^3 x 720: 186 ms, now
+    // 177; 256^3 x 360: 13.6 and 13.0; 128^3 x 180: 1.055 and 1.038).
+    uint64_t at = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(at));
+    const ConePatchArgs t = *(const ConePatchArgs *)(const __attribute__((address_space(4))) ConePatchArgs *)at;
+    const ConeDev &g = t.g;
+    const float *cs = t.cs;
+    const double *rowtab = t.rowtab;
+    const int *views = t.views;
+    const float *sino = t.sino;
+    float *vol = t.vol;
+    const int nv = t.nv, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int x = x0 + (wv >> 1) * 8 + (lane >> 3), y = y0 + (wv & 1) * 8 + (lane & 7);
+    extern __shared__ double smem[];
+    __shared__ int sh_again, sh_few;
+    __shared__ unsigned sh_least;
+    // A voxel is the difference of two planes' sums, which keep some 47 bits of
+    // `size`: one that is below 2^-30 of it is done again ray by ray, for a few
+    // values far above its own may have been in the sums.  Positive data has it
+    // at 2^-6, so there is none; noise about 0 cancels so far in one voxel of
+    // some thousands, and where a few values do lie far above the others, the
+    // voxels off their rays have it.  0 is exact (no value lies between the two
+    // planes) unless the smaller values were lost whole: where the smallest one,
+    // over a voxel's width, is below 2^-50 of `size`, or several voxels of the
+    // block are small without being 0.  (Looked up here, in blocks that hold
+    // zeros, and not kept in the views' loop, which every call pays for.)
+    if (tid == 0) {
+        sh_again = sh_few = 0;
+        sh_least = UINT_MAX;
+    }
+    __syncthreads();
+    const double small = (double)size * kConeBits;
+    int few = 0;
+    bool none = false;
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+        const double d = fabs(A[k] - A[k + 1]);
+        const bool lower = x < g.nx && y < g.ny && z0 + k < g.nz && d < small;
+        few += lower && d != 0.0;
+        none |= lower && d == 0.0;
+    }
+    if (few > 0) atomicAdd(&sh_few, few);
+    none = __syncthreads_or(none);
+    bool lost = sh_few >= kConeMany;
+    if (none && !lost) {
+        // The smallest non-zero value of the patches: a wave a view.
+        unsigned least = UINT_MAX;   // its bits 2 x - 1 (0: the largest)
+        for (int iv = wv; iv < nv; iv += kBlock / kWave) {
+            const int v = views[iv];
+            const ConeView w = cone_view(g, cs[2 * v], cs[2 * v + 1], x0, y0, z0, NK);
+            const int nr = __builtin_amdgcn_readfirstlane(min(w.nr, g.nrows - w.r0));
+            const float *from = sino + ((size_t)v * g.nrows + w.r0) * g.ncols + w.col0;
+            for (int col = lane; col < w.ncol; col += kWave)
+                for (int r = 0; r < nr; ++r)
+                    least = min(least, (__builtin_bit_cast(unsigned, from[(size_t)r * g.ncols + col]) << 1) - 1u);
+        }
+        atomicMin(&sh_least, least);
+        __syncthreads();
+        lost = (double)__builtin_bit_cast(float, (sh_least + 1u) >> 1) < (double)size * kConeUlp;
+    }
+    int *list = (int *)(smem + kZc * kBlock);
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+        if (x < g.nx && y < g.ny && z0 + k < g.nz) {
+            const double d = A[k] - A[k + 1];
+            if (fabs(d) < small && (d != 0.0 || lost)) {
+                const int n = atomicAdd(&sh_again, 1);
+                if (n < kConeFew) list[n] = k * kBlock + tid;
+            } else {
+                vol[((size_t)(z0 + k) * g.nx + x) * g.ny + y] = (float)d;
+            }
+        }
+    bad = __syncthreads_or(bad);
+    const int again = sh_again;
+    double(*acc)[kBlock] = (double(*)[kBlock])smem;
+    if (bad || again > kConeFew) {
+        // The whole block (a value that is not finite reached every row behind
+        // it through the running sums).
+        const int zend = min(z0 + NK, g.nz);
+        for (int z = z0; z < zend; z += kZc) {
+            if (x >= g.nx || y >= g.ny) break;
+            cone_bp_voxels<false, false>(g, cs, rowtab, t.vinv, t.vl2, t.vsrc, nullptr, views, nv, sino, nullptr, 1, 1, vol, x, y,
+                                         z, min(kZc, zend - z), nullptr, acc);
+        }
+        return;
+    }
+    // A wave a voxel, its lanes some of the views each: one of noise costs a
+    // block some microseconds, where the whole block would take three times as
+    // long as all before.
+    for (int i = wv; i < again; i += kBlock / kWave) {
+        const int id = __builtin_amdgcn_readfirstlane(list[i]), w = id % kBlock / kWave, l = id % kWave;
+        const int vx = x0 + (w >> 1) * 8 + (l >> 3), vy = y0 + (w & 1) * 8 + (l & 7), vz = z0 + id / kBlock;
+        const int from = (int)((int64_t)lane * nv / kWave), to = (int)((int64_t)(lane + 1) * nv / kWave);
+        cone_bp_voxels<false, false>(g, cs, rowtab, t.vinv, t.vl2, t.vsrc, nullptr, views + from, to - from, sino, nullptr, 1, 1,
+                                     nullptr, vx, vy, vz, 1, nullptr, acc);
+        double sum = acc[0][tid];
+        for (int o = kWave / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+        if (lane == 0) vol[((size_t)vz * g.nx + vx) * g.ny + vy] = (float)sum;
+    }
 }
 
 unsigned grid8(size_t blocks) { return (unsigned)((blocks + 7) / 8 * 8); }
@@ -1200,9 +1296,10 @@ void cone_bp_views(hipStream_t st, const ConeTables &t, const int *views, int nv
     if (t.patch_cols[1] > 0 && (patch < 0 || grid(kConeNk[0]) < 512)) patch = 1;
     if (patch >= 0) {
         const int pc = t.patch_cols[patch], pr = t.patch_rows[patch], ps = t.patch_span[patch];
+        const ConePatchArgs args{t.d,      t.cs.p, t.rows.p, t.vinv.p, t.vl2.p, t.vsrc.p,
+                                 views,    sino,   vol,      nv,       pc,      pr,       ps};
         launch(patch == 0 ? k_cone_bp_patch<kConeNk[0]> : k_cone_bp_patch<kConeNk[1]>, dim3(grid8(grid(kConeNk[patch]))),
-               dim3(kBlock), (uint32_t)cone_patch_lds(pc, pr, ps), st, t.d, t.cs.p, t.rows.p, t.vinv.p, t.vl2.p, t.vsrc.p,
-               views, nv, sino, vol, pc, pr, ps);
+               dim3(kBlock), (uint32_t)cone_patch_lds(pc, pr, ps), st, args);
         MI_HIP(hipGetLastError());
         return;
     }

@@ -85,3 +85,43 @@ def test_cone_patch_sparse(ctx, value):
     assert only.any()
     assert np.abs(dev - small)[only].max() < 1e-5 * small.max()
     assert not dev[(big == 0) & (small == 0)].any()
+
+
+@pytest.mark.parametrize("gi", [0, 1, 4])
+def test_cone_patch_noise(ctx, gi):
+    """Noise about 0, with rows of values 2e4 times as large: voxels that cancel by chance."""
+    g = GEOMS[gi]
+    print(f"cone back projection of noise {g}", flush=True)
+    sino = np.random.default_rng(4).standard_normal((g.n_views, g.n_rows, g.n_cols)).astype(np.float32)
+    sino[:, g.n_rows // 2 :] *= np.float32(2e4)
+    ref = O.cone_bp(O.cone_from(g), sino.astype(np.float64))
+    dev = ctx.cone_backproject(g, sino).astype(np.float64)
+    assert np.abs(dev - ref).max() < 1e-5 * np.abs(ref).max()
+    # an FP32 value of the sums' own: the voxels of the smaller values to as much
+    one = np.zeros_like(sino)
+    one[:, g.n_rows // 2 :] = 1.0
+    small = O.cone_bp(O.cone_from(g), one.astype(np.float64)) == 0
+    if small.any():
+        assert np.abs(dev - ref)[small].max() < 1e-5 * np.abs(ref[small]).max()
+
+
+@pytest.mark.parametrize("value", [1e6, 1e13, 1e16, 1e22, 1e33])
+def test_cone_patch_large_row(ctx, value):
+    """A row of the panel in every view: no voxel's sums are free of it where they reach it."""
+    g = GEOMS[0]
+    print(f"cone back projection, large row {value}", flush=True)
+    big = np.zeros((g.n_views, g.n_rows, g.n_cols), np.float32)
+    big[:, g.n_rows // 3, :] = value
+    _check(ctx, g, big)
+
+
+@pytest.mark.parametrize("value", [1e13, 1e16, 1e20, 1e33])
+def test_cone_patch_large_anywhere(ctx, value):
+    """One large value at each of many places: at the edge of blocks too."""
+    g = GEOMS[0]
+    print(f"cone back projection, large value {value} at many rows", flush=True)
+    for row in range(1, g.n_rows - 1, 5):
+        big = np.zeros((g.n_views, g.n_rows, g.n_cols), np.float32)
+        big[row % g.n_views, row, g.n_cols // 2 + row % 5 - 2] = value
+        if (ctx.cone_backproject(g, (big != 0).astype(np.float32)) != 0).any():
+            _check(ctx, g, big)
