@@ -1062,7 +1062,9 @@ __global__ __launch_bounds__(kBlock) void k_cone_bp_patch(ConePatchArgs args) {
     none = __syncthreads_or(none);
     bool lost = sh_few >= kConeMany;
     if (none && !lost) {
-        // The smallest non-zero value of the patches: a wave a view.
+        // The smallest non-zero value of the patches: a wave a view, eight rows'
+        // loads together (the last row's again behind it; one at a time, 48^3 x
+        // 120 took 445 us, so 407, without the look 392).
         unsigned least = UINT_MAX;   // its bits 2 x - 1 (0: the largest)
         for (int iv = wv; iv < nv; iv += kBlock / kWave) {
             const int v = views[iv];
@@ -1070,8 +1072,13 @@ __global__ __launch_bounds__(kBlock) void k_cone_bp_patch(ConePatchArgs args) {
             const int nr = __builtin_amdgcn_readfirstlane(min(w.nr, g.nrows - w.r0));
             const float *from = sino + ((size_t)v * g.nrows + w.r0) * g.ncols + w.col0;
             for (int col = lane; col < w.ncol; col += kWave)
-                for (int r = 0; r < nr; ++r)
-                    least = min(least, (__builtin_bit_cast(unsigned, from[(size_t)r * g.ncols + col]) << 1) - 1u);
+                for (int r = 0; r < nr; r += 8) {
+                    float q[8];
+#pragma unroll
+                    for (int h = 0; h < 8; ++h) q[h] = from[(size_t)min(r + h, nr - 1) * g.ncols + col];
+#pragma unroll
+                    for (int h = 0; h < 8; ++h) least = min(least, (__builtin_bit_cast(unsigned, q[h]) << 1) - 1u);
+                }
         }
         atomicMin(&sh_least, least);
         __syncthreads();
@@ -1291,7 +1298,8 @@ void cone_bp_views(hipStream_t st, const ConeTables &t, const int *views, int nv
     // 8 where that leaves fewer workgroups than two per CU or 16 slices' patch
     // does not fit: 128^3 x 180 views (512 workgroups of 16) 0.94 ms with 16
     // and 1.22 with 8, 512^3 x 720 152 and 214, 64^3 x 100 (64 workgroups of
-    // 16) 0.40 and 0.30.
+    // 16) 0.40 and 0.30 (all before the voxels were tested for lost bits: 1.04,
+    // 177 and 0.33 with it).
     int patch = t.patch_cols[0] > 0 ? 0 : -1;
     if (t.patch_cols[1] > 0 && (patch < 0 || grid(kConeNk[0]) < 512)) patch = 1;
     if (patch >= 0) {
