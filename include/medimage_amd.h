@@ -160,7 +160,9 @@ int mi_matrix_export(mi_context *ctx, const mi_geometry *g, int64_t *rowptr, int
  * matrix.  mi_autotune times every candidate on the device and keeps the
  * fastest; mi_set_tuning installs a stored choice.  The AT engine (jobs and
  * batches) reads bp_lanes only; fp_vec / fp_grid / bp_grid shape the single
- * projector calls (mi_forward, mi_backproject and the GoldenC steps). */
+ * projector calls (mi_forward, mi_backproject and the GoldenC steps).  What
+ * projects along the rays' lines (mi_forward and the FP32 engine, for the fan
+ * beams that have them) reads none of them. */
 typedef struct mi_tuning {
     int32_t fp_vec;         /* forward projector: 1 = four consecutive entries
                                per lane (16-byte loads), 0 = lane-strided      */
@@ -186,9 +188,10 @@ int mi_get_tuning(mi_context *ctx, const mi_geometry *g, int n_subsets, mi_tunin
  * are part of the result's definition.  The reference has no such tuner. */
 typedef struct mi_engine_tuning {
     int32_t k_cap;            /* jobs per unit: 1, 2, 4 or 8; 0 = the default
-                                 rule (K images within one XCD's L2)          */
-    int32_t bp_lds;           /* -1 default rule (LDS up to 24 KiB of slots),
-                                 0 global gathers, 1 LDS up to 56 KiB         */
+                                 rule (8 up to 2^17 pixels, 4 above)          */
+    int32_t bp_lds;           /* -1 default rule (LDS up to 56 KiB of slots),
+                                 0 global gathers, 1 LDS up to 56 KiB; without
+                                 effect on jobs that project along lines      */
     double  us_per_job_pass;  /* measured: one AT iteration of one job        */
 } mi_engine_tuning;
 int mi_engine_autotune(mi_context *ctx, const mi_geometry *g, int n_subsets, int precision, mi_engine_tuning *out);
@@ -368,7 +371,10 @@ enum mi_kernel_id {
 typedef struct mi_kernel_stats {
     int64_t launches;
     double  total_ms;     /* sum of HIP-event durations of the launches      */
-    double  bytes;        /* algorithmic bytes moved by those launches       */
+    double  bytes;        /* algorithmic bytes moved by those launches: what
+                             each reads and writes once (the 2D projectors
+                             along lines their own tables, the others their
+                             matrix; the cone beam 8 bytes a traced entry)   */
 } mi_kernel_stats;
 /* Enable per-launch HIP-event timing of the kernels above (adds one event
  * pair per launch on the context's stream). */

@@ -83,7 +83,12 @@ struct Batch {
     // ways; small images also amortise the launches at K = 8.  Measured with
     // the engine tuner on the 20 C5 geometries (N = 256 .. 1024): K = 8 is
     // fastest per job for 256^2, K = 4 for 512^2 to 1024^2 (1024^2 x 2304
-    // views: 5.1 ms per job pass against 14.1 ms at K = 1).
+    // views: 5.1 ms per job pass against 14.1 ms at K = 1).  Units with lines
+    // share only the rays' tables and the steps along them, so they gain less
+    // and the line lies less sharply (8 jobs, us per job pass at K = 1 / 2 / 4
+    // / 8: 128^2 x 180 views 74 / 65 / 74 / 102, 256^2 x 360 253 / 187 / 154 /
+    // 163, 512^2 x 720 625 / 520 / 447 / 468, 1024^2 x 2304 5921 / 5698 / 4664
+    // / 4435).
     int k_cap(const Matrix &m) const {
         if (m.etune.k_cap > 0) return std::min(m.etune.k_cap, max_k);
         return std::min(m.npix <= (int64_t)1 << 17 ? 8 : 4, max_k);

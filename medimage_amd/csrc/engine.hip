@@ -1,24 +1,28 @@
 // Kernels of the batched ordered-subset AT engine (gfx950).
 //
-// One launch per phase serves every unit of a batch.  The global block index
-// is first renumbered so that each of the 8 XCDs owns a contiguous range
-// (xcd_block), then mapped to (unit, local block) through the BlockMap passed
-// by value.  K, the number of jobs of a unit, selects a code path compiled
-// for that K; a launch uses the kernel compiled for K <= 1, <= 4 or <= 8
-// that covers its units, so it keeps the register budget of that case.
+// One launch per phase serves every unit of a batch; units with lines and
+// units with matrices have projection kernels, and launches, of their own.
+// The global block index is mapped to (unit, local block) through the
+// BlockMap passed by value, each of the 8 XCDs owning a contiguous eighth of
+// each unit's blocks (unit_block).  K, the number of jobs of a unit, selects a
+// code path compiled for that K; a launch uses the kernel compiled for K <= 1,
+// <= 4 or <= 8 that covers its units, so it keeps the register budget of that
+// case.
 //
-// Forward projection of fan beams is the checkpointed walk (walk_otf): the
-// tracer re-run from stored per-segment states, a block holding 32
-// neighbouring rays x 8 segments.  Back projection (and the forward
-// projection of other geometries) reads the sliced matrices (Sell,
-// runtime.hpp): a lane owns one pixel column (back) or one segment of one
-// ray (forward) and walks it in entry order with a Kahan sum, four entries
-// per 16-byte load, a wave's loads contiguous; neighbouring lanes own
-// neighbouring rays / pixels, so one gather instruction touches few cache
-// lines.  The back projection stages each 16 x 16 pixel block's residual
-// values in LDS first where they fit (bp_unit).  Images are stored in 4 x 8
-// tiles (tile_index).  Partial sums of an item are combined in a fixed
-// order.
+// FP32 fan beams project along the rays' lines (Lines, runtime.hpp;
+// line_fp_unit, line_bp_unit, k_line_project): no matrix is read, a ray's
+// lengths follow from its position in each line of pixels.  The other fan
+// beams' forward projection is the checkpointed walk (walk_otf): the tracer
+// re-run from stored per-segment states, a block holding 32 neighbouring rays
+// x 8 segments.  Their back projection (and the forward projection of other
+// geometries) reads the sliced matrices (Sell, runtime.hpp): a lane owns one
+// pixel column (back) or one segment of one ray (forward) and walks it in
+// entry order with a Kahan sum, four entries per 16-byte load, a wave's loads
+// contiguous; neighbouring lanes own neighbouring rays / pixels, so one gather
+// instruction touches few cache lines.  The back projection stages each 16 x
+// 16 pixel block's residual values in LDS first where they fit (bp_unit).
+// Images are stored in 4 x 8 tiles (tile_index).  Partial sums of an item are
+// combined in a fixed order.
 #include "engine.hpp"
 #include "tracers.hpp"
 
