@@ -508,8 +508,8 @@ struct LineGeo {
     float pix, sod, k;
     double bin0;
 };
-__device__ __forceinline__ void line_view(const LineGeo &g, float c, float s, int i0, int j0, int &b0, int &cnt, float &hw,
-                                          int &axis) {
+__host__ __device__ __forceinline__ void line_view(const LineGeo &g, float c, float s, int i0, int j0, int &b0, int &cnt,
+                                                   float &hw, int &axis) {
     const float p = g.pix, sod = g.sod, k = g.k;
     const float X0 = (i0 - 0.5f * g.nx) * p, Y0 = (j0 - 0.5f * g.ny) * p;
     // the block's corners: extremes of the position (a monotonic function of
@@ -607,13 +607,39 @@ __global__ __launch_bounds__(kLineViews) void k_line_windows(LineGeo g, int tnx,
     }
 }
 
+// Bins too fine for a block's windows, seen from the blocks at the image's
+// corners, each in the view whose source comes nearest: such a geometry is
+// spared the attempt (allocations, the walk of every ray).  Only what is above
+// the limits by more than the device's rounding; k_line_windows has the rest.
+bool lines_too_fine(const LineGeo &g, const std::vector<double> &c, const std::vector<double> &s) {
+    for (int q = 0; q < 4; ++q) {
+        const int i0 = q & 1 ? (g.nx - 1) / 16 * 16 : 0, j0 = q >> 1 ? (g.ny - 1) / 16 * 16 : 0;
+        const double X = i0 + 8 - 0.5 * g.nx, Y = j0 + 8 - 0.5 * g.ny;
+        size_t at = 0;
+        double near = -1e300;
+        for (size_t v = 0; v < c.size(); ++v) {
+            const double d = g.arc ? c[v] * X + s[v] * Y : s[v] * X - c[v] * Y;
+            if (d > near) {
+                near = d;
+                at = v;
+            }
+        }
+        int b0, cnt, axis;
+        float hw;
+        line_view(g, (float)c[at], (float)s[at], i0, j0, b0, cnt, hw, axis);
+        if (2.0f * hw > kLineEmpty + 0.01f || cnt > kLineSlots) return true;
+    }
+    return false;
+}
+
 // The line form of every ray; false when the geometry has a ray without it, or
 // an image or sinogram beyond the kernels' 32-bit offsets and the fixed point of
 // their positions.  windows: and the back projection's tables; false also for a
 // source too near (for the arc: the 45 degrees of its arc tangent), or bins so
 // fine that the rays of one view through a 16 x 16 pixel block do not fit the
 // back projection's LDS slots.
-bool try_lines(Matrix &m, const TraceArgs &a, bool windows, hipStream_t st) {
+bool try_lines(Matrix &m, const TraceArgs &a, const std::vector<double> &vcos, const std::vector<double> &vsin, bool windows,
+               hipStream_t st) {
     const mi_geometry &g = m.g;
     if (!(g.pixel_mm > 0.0501) || (int64_t)(g.nx + 64) * (g.ny + 64) >= (int64_t)1 << 26 || std::max(g.nx, g.ny) >= 1 << 18)
         return false;
@@ -627,10 +653,13 @@ bool try_lines(Matrix &m, const TraceArgs &a, bool windows, hipStream_t st) {
     const int tnx = (g.nx + kTileH - 1) / kTileH, tny = tiled_ny(g.ny);
     const int64_t nblk = bp_blocks_of(tnx, tny);
     int64_t wins = 0;
+    const double bin0 = q.arc ? g.n_bins / 2 - g.det_offset : g.n_bins / 2 - 0.5 - g.det_offset;
+    const LineGeo lg{g.nx, g.ny, g.n_bins, q.arc, (float)g.pixel_mm, q.sod, q.k, bin0};
     if (windows) {
         const double rad = 0.5 * g.pixel_mm * std::hypot((double)g.nx, (double)g.ny), blk = 16 * M_SQRT2 * g.pixel_mm;
         if (!(g.sod_mm - rad - blk > 0.02 * g.sod_mm)) return false;
         if (q.arc && !(1.42 * (rad + g.pixel_mm) < g.sod_mm)) return false;
+        if (lines_too_fine(lg, vcos, vsin)) return false;
         q.win0.assign(m.S + 1, 0);
         int64_t most = 0;
         for (int s = 0; s < m.S; ++s) {
@@ -668,8 +697,6 @@ bool try_lines(Matrix &m, const TraceArgs &a, bool windows, hipStream_t st) {
         upload(q.d_win0, q.win0, st);
         q.views.alloc(wins * q.vstride);
         MI_HIP(hipMemsetAsync(q.views.p, 0, q.views.bytes(), st));
-        const double bin0 = q.arc ? g.n_bins / 2 - g.det_offset : g.n_bins / 2 - 0.5 - g.det_offset;
-        const LineGeo lg{g.nx, g.ny, g.n_bins, q.arc, (float)g.pixel_mm, q.sod, q.k, bin0};
         k_line_windows<<<(unsigned)wins, kLineViews, 0, st>>>(lg, tnx, tny, nblk, a.fcos, a.fsin, a.vlist, m.d_sub_row0.p,
                                                              q.d_win0.p, m.S, q.vstride, q.views.p, flags.p + 1);
         MI_HIP(hipGetLastError());
@@ -785,8 +812,9 @@ std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, h
     a.vlist = m->d_vlist.p;
     DevBuf<double> dcos, dsin, bcos, bsin;
     DevBuf<float> pcos, psin;
+    std::vector<double> vcos(g.n_views), vsin(g.n_views);   // fan beams: the views' cos and sin
     if (g.beam == MI_BEAM_FAN_FLAT) {
-        std::vector<double> c(g.n_views), s(g.n_views);
+        auto &c = vcos, &s = vsin;
         const double span = g.span_deg * (M_PI / 180.0);
         for (int v = 0; v < g.n_views; ++v) {
             double th = span * (double)v / (double)g.n_views;
@@ -803,7 +831,8 @@ std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, h
         // degrees -> cos(angle / 180 * pi); detector element j (from
         // -n_bins/2) -> cos((j + OFF_CENTER) * LENGTH_PER_DET * pi / 180 + pi)
         // (the angle of view v: the slice's _pos table, or uniform over span_deg)
-        std::vector<double> c(g.n_views), s(g.n_views), dc(g.n_bins), ds(g.n_bins);
+        auto &c = vcos, &s = vsin;
+        std::vector<double> dc(g.n_bins), ds(g.n_bins);
         for (int v = 0; v < g.n_views; ++v) {
             const double angle = g.view_deg ? g.view_deg[v] : g.span_deg * (double)v / (double)g.n_views;
             c[v] = std::cos(angle / 180.0 * M_PI);
@@ -849,7 +878,7 @@ std::unique_ptr<Matrix> build_matrix(const mi_geometry &g, int S, bool want64, h
     // the tracer from checkpoints and read the matrix.
     const bool fan = g.beam == MI_BEAM_FAN_FLAT || g.beam == MI_BEAM_FAN_ARC;
     if (layout >= 2) {
-        if (!fan || !try_lines(*m, a, layout == 3, st)) m->lines = Lines{};
+        if (!fan || !try_lines(*m, a, vcos, vsin, layout == 3, st)) m->lines = Lines{};
         m->has_csr = false;
         return m;
     }
